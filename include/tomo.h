@@ -138,13 +138,18 @@ const char *tomo_last_error(void);
  * edge and interior update kernels (1-4); chunk: running-DFT fold interval in
  * steps (a multiple of tsteps, <= 64); grid_mult: persistent workgroups per CU;
  * form: how a physical-mode time block is launched, TOMO_FORM_STREAMS (one
- * kernel per tile class on four streams, joined per block) or
- * TOMO_FORM_FUSED (one launch of a kernel that runs every class);
+ * simulation by itself: one kernel per tile class on four streams, joined per
+ * block; simulations that advance together: as TOMO_FORM_FUSED) or
+ * TOMO_FORM_FUSED (one launch that runs every tile: register tiles on grids of
+ * at least 64 x 32 nodes, whose block depth and tile shape the library picks
+ * for the chunk, else row sweeps under the schedule's own fields).  A context
+ * whose caller has chosen no form, and reference-compatible simulations under
+ * any, take the register tiles too;
  * edge_rows: output rows per corner and row-edge tile (the latency-critical
  * boundary tiles; at most seg_rows). */
 #define TOMO_FORM_STREAMS 1
 #define TOMO_FORM_FUSED 2
-/* TOMO_FORM_RESIDENT: one cooperative launch per DFT chunk in which each
+/* TOMO_FORM_RESIDENT (physical mode): one cooperative launch per DFT chunk in which each
  * workgroup keeps one tile of a simulation (a 64-lane band, seg_rows rows per
  * wave, 8 waves) in registers through every time block, exchanging only a
  * T-deep frame with its neighbours; seg_rows 8 or 12, tsteps 2, 4 or 8.  Runs
@@ -166,10 +171,9 @@ typedef struct tomo_schedule {
 } tomo_schedule;
 int tomo_set_schedule(tomo_ctx *ctx, const tomo_schedule *s);
 int tomo_get_schedule(tomo_ctx *ctx, tomo_schedule *s);
-/* The schedule the FDTD_GPU / FDTD_CPU shims install on their context: the
- * fastest measured at the drop-in size (401^2, 4 excitations advancing
- * together): resident tiles of 12 rows, 8 steps per frame exchange, 64-step
- * DFT chunks.  The DFT chunk sets the FP32 partial sums of the running DFT,
+/* The schedule the FDTD_GPU / FDTD_CPU shims install on their context.  Of its
+ * fields the reference-compatible simulations (register tiles under every form)
+ * take the 64-step DFT chunk.  The DFT chunk sets the FP32 partial sums of the running DFT,
  * so contexts compare bit for bit only under equal chunks. */
 #define TOMO_DROPIN_SCHEDULE {8, 12, 1, 1, 64, 16, TOMO_FORM_RESIDENT, 1, 0}
 
@@ -188,7 +192,7 @@ int tomo_autotune(tomo_ctx *ctx, const tomo_sim_config *cfg, int n_sims, tomo_sc
  * (the psi pair).  `update` is the wall time of the whole update phase (all
  * streams, from the first launch of an epoch to the join of its last block). */
 enum {
-    TOMO_KERNEL_GENERAL = 0, /* k_tblock: every tile of a reference-compatible simulation */
+    TOMO_KERNEL_GENERAL = 0, /* reference-compatible simulations: register tiles, or k_tblock on small grids */
     TOMO_KERNEL_CORNER = 1,  /* k_tedge: corner tiles (and all tiles of small physical grids) */
     TOMO_KERNEL_ROW = 2,     /* k_trow: top / bottom frame between the corners */
     TOMO_KERNEL_COL = 3,     /* k_tcol: left / right frame between the corners */
@@ -196,7 +200,7 @@ enum {
     TOMO_KERNEL_FOLD = 5,    /* k_fold: running-DFT fold of a chunk of samples */
     TOMO_KERNEL_PROJECT = 6, /* k_project_mfma: far-field projection on the matrix cores */
     TOMO_KERNEL_FITNESS = 7, /* k_fitness: FP64 fitness reduction */
-    TOMO_KERNEL_FUSED = 8,   /* k_tfused: every tile class in one launch (TOMO_FORM_FUSED) */
+    TOMO_KERNEL_FUSED = 8,   /* physical mode, every tile in one launch: register tiles, or k_tfused on small grids */
     TOMO_KERNEL_RESIDENT = 9, /* k_tres: a whole epoch in one cooperative launch (TOMO_FORM_RESIDENT) */
     TOMO_KERNEL_TILE = 10,    /* k_twave: register tiles, one launch per time block (TOMO_FORM_TILE) */
     TOMO_KERNEL_COUNT = 11

@@ -1,0 +1,105 @@
+"""The register-tile update against the row sweeps and the oracle.
+
+A context under an installed streams schedule advances a simulation by itself
+with the row-sweep kernels; the fused form takes register tiles.  Every cell
+must come out the same bit for bit: on grids of exactly one tile (64 x 32
+nodes and one more), odd and non-square ones, material, source and contour in
+edge tiles, thin and thick CPML, and DFT chunks that end in a shorter block.
+Reference-compatible simulations (register tiles under every form) are held to
+the FP32 oracle's field tolerance."""
+import numpy as np
+import pytest
+
+import tomography_amd as t
+from cases import PHYS_PARAMS, fat_medium, phys_small, ref_cpu_params, ref_cpu_small, ref_params, ref_small, rel_l2
+
+FIELD_TOL_F32 = 1e-5  # relative L2 against the FP32 oracle, as in test_gpu_parity
+
+
+def tiny(nx, ny):
+    c = t.preset(t.PRESET_CFG4, 64)
+    return c.copy(nx=nx, ny=ny, steps=130, n_freq=2, n_angles=24, ncpml=5, ntff_offset=8, breast_radius=0.005,
+                  skin_thickness=0.001, src_radius=0.006)
+
+
+def wide(**over):
+    c = t.preset(t.PRESET_CFG1).copy(steps=170, n_freq=2, n_angles=24, n_exc=4, breast_radius=0.025, src_radius=0.03)
+    return c.copy(**over)
+
+
+CASES = {
+    "one tile exactly": (tiny(63, 31), PHYS_PARAMS, 0),
+    "one node less (row sweeps)": (tiny(62, 31), PHYS_PARAMS, 0),
+    "one node more": (tiny(64, 32), PHYS_PARAMS, 0),
+    "two tiles high": (tiny(63, 64), PHYS_PARAMS, 0),
+    "wide": (wide(nx=301, ny=140), PHYS_PARAMS, 1),
+    "tall": (wide(nx=140, ny=301), PHYS_PARAMS, 3),
+    "thin CPML": (wide(nx=256, ny=256, ncpml=1, ntff_offset=3), PHYS_PARAMS, 2),
+    "thick CPML": (wide(nx=256, ny=256, ncpml=31, ntff_offset=60), PHYS_PARAMS, 2),
+    "contour inside the phantom": (wide(nx=256, ny=256, ntff_offset=100), PHYS_PARAMS, 1),
+    "source in material, material at the edges": (*(lambda c, p: (c.copy(steps=170), p))(*fat_medium()), 0),
+    "FP64 running DFT": (phys_small(steps=170, n=200, flags=t.FLAG_DFT_FP64), PHYS_PARAMS, 1),
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("chunk", [4, 32, 60])
+@pytest.mark.parametrize("name", list(CASES))
+def test_register_tiles_equal_row_sweeps(name, chunk):
+    cfg, p, exc = CASES[name]
+    out = []
+    for form in (t.FORM_STREAMS, t.FORM_FUSED):
+        with t.Context() as c:
+            c.set_schedule(tsteps=4, seg_rows=16, edge_waves=2, chunk=chunk, form=form)
+            g = c.sim(cfg, p, exc=exc)
+            g.step(37)  # an odd split: partial blocks and chunks
+            g.step(cfg.steps - 37)
+            out.append([*g.fields(), *g.dft(), *g.farfield()])
+            g.close()
+    assert np.abs(out[0][0]).max() > 0
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.gpu
+def test_default_context_and_mixed_sets_equal_row_sweeps():
+    """A context with no schedule installed, and sets of several grids (one of
+    them too small for a tile) advancing together, against the row sweeps."""
+    mix = [tiny(63, 40), tiny(40, 63), wide(nx=150, ny=150, n_exc=2)]
+    with t.Context() as c:
+        c.set_schedule(tsteps=4, seg_rows=16, edge_waves=2, chunk=32, form=t.FORM_STREAMS)
+        want = [c.eval(cfg, PHYS_PARAMS) for cfg in mix]
+    with t.Context() as c:
+        assert [c.eval(cfg, PHYS_PARAMS) for cfg in mix] == want
+        for pick in ((0, 1, 2), (0, 2)):
+            tickets = [c.submit(mix[i], PHYS_PARAMS) for i in pick]
+            assert [c.wait(k)[0] for k in tickets] == [want[i] for i in pick]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n, cpu", [(83, False), (132, True), (260, False)])
+def test_reference_register_tiles_vs_oracle(oracle, n, cpu):
+    cfg, p = (ref_cpu_small(steps=240, n=n), ref_cpu_params(4)) if cpu else (ref_small(steps=240, n=n), ref_params(5))
+    with t.Context() as c:
+        g = c.sim(cfg, p, exc=2)
+        g.step(101)
+        g.step(139)
+        got = g.fields()
+        g.close()
+    o = oracle.sim(cfg, p, exc=2)
+    o.step(240)
+    for name, a, b in zip(("ez", "hx", "hy"), got, o.fields()):
+        assert rel_l2(a, b) < FIELD_TOL_F32, (name, rel_l2(a, b))
+
+
+def test_division_by_known_kappa_is_the_division():
+    """The reference stage divides by kappa in [1, 10]; the kernel multiplies by
+    its 64-bit reciprocal and rounds once, which is the 32-bit quotient itself."""
+    rng = np.random.default_rng(3)
+    k = np.concatenate([rng.uniform(1, 10, 4000), [1, 2, 3, 7, 9.999999]]).astype(np.float32)
+    a = np.concatenate([rng.uniform(-1, 1, 4000), np.nextafter(np.float32(1), np.float32(2)) * np.ones(5)])
+    for e in (-120, -60, -1, 0, 40, 120):
+        x = (a * 2.0 ** e).astype(np.float32)
+        with np.errstate(all="ignore"):
+            assert np.array_equal((x[:, None].astype(np.float64) * (1.0 / k.astype(np.float64))).astype(np.float32),
+                                  x[:, None] / k)

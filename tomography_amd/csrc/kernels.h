@@ -45,6 +45,17 @@ bool twave_supported(int T, int rows_per_wave);
 hipError_t launch_twave(int T, int rows_per_wave, const TileItem* tiles, int ntiles, const LaunchItem* items,
                         const DevSim* sims, int ordinal, int grid, hipStream_t st);
 
+// Register-tile update: one workgroup of `waves` (8 or 16) waves per RegTile
+// advances it one time block of `tsteps` steps.  Every held node is a node of
+// the grid, and the owned nodes lie at least `tsteps` inside the held ones
+// wherever those do not end at the grid's edge.  rows: kTileRowsClean for a
+// tile whose held rows and columns, and the row below them, lie clear of the
+// CPML strips and the grid's edge, with vacuum or physical-mode material
+// without the source; else kTileRowsEdge.  Field planes below 4 GiB.
+constexpr int kTileRowsEdge = 4, kTileRowsClean = 8;
+hipError_t launch_rtile(int mode, int waves, const RegTile* tiles, int ntiles, const LaunchItem* items, const DevSim* sims,
+                        int ordinal, int tsteps, hipStream_t st);
+
 // Resident update form: one cooperative launch advances every simulation of
 // `items` by its epoch (all time blocks), one workgroup per ResTile, all
 // co-resident.  `done` (ntiles counters) must start at zero; `err` is set to 1
@@ -52,8 +63,8 @@ hipError_t launch_twave(int T, int rows_per_wave, const TileItem* tiles, int nti
 constexpr int kResidentWaves = 8;  // waves per workgroup of the resident kernel
 bool tres_supported(int T, int rows_per_wave);
 // Tiles one cooperative launch can hold on `cus` compute units (0: none).
-int tres_max_tiles(int T, int rows_per_wave, int mode, int cus);
-hipError_t launch_tres(int T, int rows_per_wave, int mode, const ResTile* tiles, int ntiles,
+int tres_max_tiles(int T, int rows_per_wave, int cus);
+hipError_t launch_tres(int T, int rows_per_wave, const ResTile* tiles, int ntiles,
                        const LaunchItem* items, const DevSim* sims, int* done, int* err, int spin_limit,
                        hipStream_t st);
 

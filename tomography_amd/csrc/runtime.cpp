@@ -109,6 +109,13 @@ namespace {
 // copies and device copies) and the DevSim table the kernels index.  The
 // context's own staging grows on demand (pinned host memory, device memory);
 // a fixed staging lives in caller-provided memory and never grows.
+// Shape of the register tiles of a launch: T steps per block, `waves` waves
+// per tile.  T == 0: the launch takes the row sweeps.
+struct TilePlan {
+    int T = 0, waves = 0;
+    bool operator==(const TilePlan& o) const { return T == o.T && waves == o.waves; }
+};
+
 struct Staging {
     LaunchItem* h_items = nullptr;
     LaunchItem* d_items = nullptr;
@@ -132,6 +139,8 @@ struct Staging {
     int res_cap = 0, nres = 0;
     int* d_flags = nullptr;  // res_cap counters, then the error word (res_err)
     int res_key_form = 0;    // form the tile lists were built for
+    bool key_together = false;
+    TilePlan plan;           // register tiles of the list (T == 0: none)
 };
 }  // namespace
 
@@ -155,6 +164,7 @@ struct tomo_ctx {
     int T = 4, S = 32, W = 4, K = 32;  // schedule (W: waves per edge workgroup)
     int grid_mult = 4;                 // persistent workgroups per CU
     int form = TOMO_FORM_STREAMS;      // launch form of physical-mode blocks
+    bool form_set = false;             // a caller (or the autotuner) has chosen it
     int ER = 8;                        // output rows per corner / row-edge tile
     int Si = 0;                        // output rows per interior tile (0: S)
     bool use_graph = false;            // replay regular epochs from a captured hipGraph
@@ -638,6 +648,139 @@ void build_wave_tiles(Slot* sl, int item, int T, int RW, std::vector<TileItem>& 
         }
 }
 
+// Split n nodes of an axis into pieces of `held` nodes (n >= held), evenly
+// spaced, of which each owns the nodes at least T inside it, or up to the end
+// of the axis: {first held, first owned, end of owned} per piece.
+struct Piece { int l, a, b; };
+std::vector<Piece> split_axis(int n, int held, int T) {
+    const int k = n <= held ? 1 : (n - 2 * T + held - 2 * T - 1) / (held - 2 * T);
+    std::vector<Piece> v(k);
+    for (int i = 0; i < k; ++i) {
+        v[i].l = k > 1 ? (int)((int64_t)i * (n - held) / (k - 1)) : 0;
+        v[i].a = i ? v[i].l + T : 0;
+        v[i].b = n;
+        if (i) v[i - 1].b = v[i].a;
+    }
+    return v;
+}
+
+// Whether the register tiles of `waves` waves hold a simulation's grid.
+bool reg_tiles_fit(const DevSim& d, int waves) {
+    return d.nx + 1 >= 64 && d.ny + 1 >= waves * kTileRowsEdge && (uint64_t)d.ps * 4 < (1ull << 32);
+}
+
+// Rows of one band of columns cut into register tiles, bottom to top:
+// waves * kTileRowsClean held rows where those are clean and `light(l, l + held)`
+// says so, else waves * kTileRowsEdge.  add(l, a, b, rows): held from l, owned [a, b).
+template <class Light, class Add>
+void cut_rows(const DevSim& d, int T, int waves, bool xs, Light light, Add add) {
+    const int ny = d.ny, nc = d.nc;
+    for (int a = 0, b; a <= ny; a = b) {
+        int rows = kTileRowsClean, held = waves * rows, l = a ? a - T : 0;
+        if (xs || l <= nc + 1 || l + held > ny - nc || !light(l, l + held)) {
+            rows = kTileRowsEdge;
+            held = waves * rows;
+            l = std::min(l, ny + 1 - held);
+        }
+        b = l + held > ny ? ny + 1 : l + held - T;
+        add(l, a, b, rows);
+    }
+}
+
+// Register tiles of one simulation: bands of 64 columns, cut into rows.
+void build_reg_tiles(Slot* sl, int item, const TilePlan& p, std::vector<RegTile>& out) {
+    const DevSim& d = sl->d;
+    for (int k = 0; k < 4; ++k) sl->cls_cells[k] = sl->cls_bytes[k] = 0;
+    const bool phys = d.mode == TOMO_MODE_PHYSICAL;
+    // the kernel's vacuum stage takes these coefficients as they are
+    const float* v = d.coef;
+    const bool vac = v[0] == 1.f && v[2] == 0.f && v[3] == 0.f && v[6] == 0.f;
+    const int* ms = sl->su.mspan.data();
+    for (const Piece& x : split_axis(d.nx + 1, 64, p.T)) {
+        auto has_mat = [&](int r0, int r1) {
+            for (int r = r0; r < r1; ++r)
+                if (!vac || (ms[2 * r] < ms[2 * r + 1] && ms[2 * r] < x.l + 64 && ms[2 * r + 1] > x.l)) return true;
+            return false;
+        };
+        // material keeps to the short tiles in reference mode (its incident field
+        // makes those rows the costliest) and where the source may lie in it
+        auto light = [&](int r0, int r1) {
+            return !has_mat(r0, r1) || (phys && !(d.sx >= x.l && d.sx < x.l + 64 && d.sy >= r0 && d.sy < r1));
+        };
+        cut_rows(d, p.T, p.waves, x.l <= d.nc || x.l + 64 > d.nx - d.nc, light, [&](int l, int a, int b, int rows) {
+            RegTile t{item, sl->idx, x.l, x.a, x.b, l, a, b, rows, 0};
+            for (int w = 0; w < p.waves; ++w)
+                if (has_mat(l + w * rows, l + (w + 1) * rows)) t.matmask |= 1 << w;
+            TileItem own{};
+            own.x0 = x.a; own.xe = x.b; own.y0 = a; own.y1 = b;
+            account_tile(sl, phys ? TILE_INNER : TILE_CORNER, own);
+            out.push_back(t);
+        });
+    }
+}
+
+// Shape of the register tiles for a set of simulations under DFT chunks of K
+// steps (T == 0: some grid does not fit one).  The shape does not change
+// results, only time: per launch a fixed part (dispatch, tables, the tile's loads
+// and stores) and per step the larger of the whole launch's work spread over
+// the SIMDs and one tile's own (waves / 4 waves of a SIMD, each a step's
+// instructions and an exchange).  Deep blocks pay the fixed part less often and
+// recompute more ghost cells.  The constants are a fit to 25 launches measured
+// on MI355X (one grid of 257 to 1025 nodes, 64 of 129 and of 513; 8 and 16
+// waves, blocks of 6 to 20 steps): 9% rms, e.g. 725^2 in blocks of 12, 20.6 us
+// with 8 waves and 15.7 with 16 (model 20.8 and 17.5); 64 of 513^2 in blocks of
+// 8, 217 and 219 us (240 and 220).
+TilePlan plan_reg_tiles(const std::vector<Slot*>& ms, int K, int cus) {
+    constexpr double kFixed = 8.0;                 // us per launch
+    constexpr double kEdge = 106, kClean = 61;     // instructions of a wave's step
+    constexpr double kStepLatency = 25, kGHz = 2.3;
+    TilePlan best;
+    double best_t = 1e300;
+    for (int waves : {8, 16}) {
+        bool fit = true;
+        for (const Slot* s : ms) fit = fit && reg_tiles_fit(s->d, waves);
+        if (!fit) continue;
+        const int tmax = std::min(24, (waves * kTileRowsEdge - 8) / 2);
+        for (int m = (K + tmax - 1) / tmax; m <= K; ++m) {
+            const int T = (K + m - 1) / m;
+            if (T < 4 && best.T) break;
+            int64_t edge = 0, clean = 0;
+            const DevSim* last = nullptr;
+            int64_t e1 = 0, c1 = 0;
+            for (const Slot* s : ms) {
+                const DevSim& d = s->d;
+                if (!last || last->nx != d.nx || last->ny != d.ny || last->nc != d.nc) {
+                    e1 = c1 = 0;
+                    const std::vector<Piece> px = split_axis(d.nx + 1, 64, T);
+                    int64_t e[2] = {0, 0}, c[2] = {0, 0};
+                    for (int xs = 0; xs < 2; ++xs)
+                        cut_rows(d, T, waves, xs, [](int, int) { return true; },
+                                 [&](int, int, int, int rows) { rows == kTileRowsClean ? ++c[xs] : ++e[xs]; });
+                    for (const Piece& x : px) {
+                        const bool xs = x.l <= d.nc || x.l + 64 > d.nx - d.nc;
+                        e1 += e[xs];
+                        c1 += c[xs];
+                    }
+                    last = &d;
+                }
+                edge += e1;
+                clean += c1;
+            }
+            const double per_simd = waves * (edge * kEdge + clean * kClean) * 4 / (4.0 * cus);
+            const int64_t slots = (int64_t)(16 / waves) * cus;  // tiles the device holds at once (four waves a SIMD)
+            const double mates = waves == 8 && edge + clean > cus ? kClean : 0;
+            const double lone = edge + clean <= slots ? waves / 4 * (kEdge + mates) * 4 + kStepLatency : 0;
+            const double t = m * (kFixed + T * std::max(per_simd, lone) / (kGHz * 1e3));
+            if (t < best_t) {
+                best_t = t;
+                best.T = T;
+                best.waves = waves;
+            }
+        }
+    }
+    return best;
+}
+
 // The resident launches' error word: 16-byte aligned past the counters.
 int* res_err(const Staging& st) { return st.d_flags + ((st.res_cap + 3) & ~3) + 32; }
 
@@ -711,8 +854,9 @@ Staging& stage(tomo_ctx* c) {
 }
 
 // Run epochs until every slot in `sl` reaches its target step, staging the
-// launches in `st` (whose d_sims holds the slots' DevSim entries).
-int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st) {
+// launches in `st` (whose d_sims holds the slots' DevSim entries).  `together`:
+// the slots are a batch or the request loop's, not one simulation by itself.
+int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st, bool together) {
     const int T = c->T, S = c->S, W = c->W, K = c->K;
     if (!tblock_supported(T) || K % T || K > 64 || W < 1 || W > 4 || S < 1)
         return fail(TOMO_E_INVALID, "unsupported schedule");
@@ -729,18 +873,40 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st) {
             // tile list (rebuilt only when the set of simulations changes)
             std::vector<uint64_t> key;
             for (Slot* s : ms) key.push_back(s->serial);
-            std::vector<TileItem> te, tr, tc, tn;
             const bool rebuild = key != st.tile_key || st.key_T != T || st.key_S != S || st.key_W != W ||
                                  st.key_Wi != c->Wi || st.key_ER != c->ER || st.key_Si != c->Si ||
-                                 st.res_key_form != c->form;
-            // resident form: every tile of the set in one cooperative launch,
-            // when they fit on the device at once (else the fused form runs)
-            const bool want_res = c->form == TOMO_FORM_RESIDENT && tres_supported(T, S) && !st.fixed;
+                                 st.res_key_form != c->form || st.key_together != together;
             // tile form: whole register tiles, one workgroup each, in place of the four classes
             const bool wave = c->form == TOMO_FORM_TILE && mode == TOMO_MODE_PHYSICAL && twave_supported(T, S);
+            std::vector<TileItem> te, tr, tc, tn;
             std::vector<ResTile> trs;
+            std::vector<RegTile> trg;
             if (rebuild) {
-                for (size_t i = 0; i < ms.size(); ++i) {
+                // resident form: every tile of the set in one cooperative launch,
+                // when they fit on the device at once (else the fused form runs)
+                if (c->form == TOMO_FORM_RESIDENT && mode == TOMO_MODE_PHYSICAL && tres_supported(T, S) && !st.fixed &&
+                    !c->res_refused) {
+                    for (size_t i = 0; i < ms.size(); ++i) build_res_tiles(ms[i], (int)i, T, S, trs);
+                    if ((int)trs.size() > tres_max_tiles(T, S, c->cus)) trs.clear();
+                }
+                // Register tiles wherever the grids allow them (64 columns and 32
+                // rows at least): reference-compatible simulations, the fused form,
+                // and the streams form for simulations that advance together (64 of
+                // 512^2: 131 ms against 174 on four streams; 64 of 128^2: 5.3
+                // against 21).  One simulation by itself under an installed streams
+                // schedule keeps that form's four kernels, as its name says.
+                const bool streams_alone = c->form == TOMO_FORM_STREAMS && c->form_set && !together;
+                st.plan = TilePlan{};
+                if (mode != TOMO_MODE_PHYSICAL || (!wave && trs.empty() && !streams_alone))
+                    st.plan = plan_reg_tiles(ms, K, c->cus);
+                if (st.plan.T) {
+                    for (size_t i = 0; i < ms.size(); ++i) build_reg_tiles(ms[i], (int)i, st.plan, trg);
+                    if (st.fixed && trg.size() * sizeof(RegTile) > st.tiles_cap * sizeof(TileItem)) {
+                        st.plan = TilePlan{};  // the row sweeps' list is the smaller one
+                        trg.clear();
+                    }
+                }
+                for (size_t i = 0; i < ms.size() && !st.plan.T; ++i) {
                     if (wave) build_wave_tiles(ms[i], (int)i, T, S, tn);
                     else build_tiles(ms[i], (int)i, T, S, c->Si ? c->Si : S, W, c->Wi, c->ER, te, tr, tc, tn);
                 }
@@ -750,12 +916,14 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st) {
                     xcd_order(tc);
                     xcd_order(tn);
                 }
-                if (want_res) {
-                    for (size_t i = 0; i < ms.size(); ++i) build_res_tiles(ms[i], (int)i, T, S, trs);
-                    if ((int)trs.size() > tres_max_tiles(T, S, mode, c->cus)) trs.clear();
-                }
             }
-            const int ntiles = rebuild ? (int)(te.size() + tr.size() + tc.size() + tn.size()) : st.ntiles;
+            const TilePlan plan = st.plan;
+            const bool rtile = plan.T > 0;
+            const int Tb = rtile ? plan.T : T;  // steps per launch
+            const int ntiles =
+                rebuild ? (int)(te.size() + tr.size() + tc.size() + tn.size() + trg.size()) : st.ntiles;
+            // (register tiles share the tile list's memory)
+            const int tile_room = rtile ? (int)((ntiles * sizeof(RegTile) + sizeof(TileItem) - 1) / sizeof(TileItem)) : ntiles;
             // Items of E consecutive epochs in one upload: every simulation of
             // the set is active in each of them (only the last may be partial),
             // so the set, and with it the tile list, stays fixed.  A captured
@@ -763,7 +931,7 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st) {
             const int nsim = (int)ms.size();
             int E = (c->use_graph && !st.fixed) ? 1 : std::max(1, std::min(kMaxStagedEpochs, kMaxStagedItems / nsim));
             for (Slot* s : ms) E = std::min(E, (s->target - s->done + K - 1) / K);
-            int rc = ensure_staging(c, st, E * nsim, ntiles);
+            int rc = ensure_staging(c, st, E * nsim, tile_room);
             if (rc) return rc;
             // the host staging is rewritten below: wait for its last upload
             if (st.staged) HIPCHK(hipEventSynchronize(st.staged));
@@ -775,7 +943,7 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st) {
                     LaunchItem& it = st.h_items[e * nsim + i];
                     it.sim = s->idx;
                     it.step0 = s->done + e * K;
-                    it.parity0 = s->parity ^ ((e * (K / T)) & 1);  // epochs before the last are full
+                    it.parity0 = s->parity ^ ((e * ((K + Tb - 1) / Tb)) & 1);  // epochs before the last are full
                     it.nsteps = std::min(K, s->target - s->done - e * K);
                 }
                 maxP = std::max(maxP, s->d.P);
@@ -789,8 +957,9 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st) {
                 h = std::copy(tr.begin(), tr.end(), h);
                 h = std::copy(tc.begin(), tc.end(), h);
                 std::copy(tn.begin(), tn.end(), h);
-                HIPCHK(hipMemcpyAsync(st.d_tiles, st.h_tiles, sizeof(TileItem) * ntiles, hipMemcpyHostToDevice,
-                                      c->stream));
+                if (rtile) std::copy(trg.begin(), trg.end(), (RegTile*)st.h_tiles);
+                HIPCHK(hipMemcpyAsync(st.d_tiles, st.h_tiles, (rtile ? sizeof(RegTile) : sizeof(TileItem)) * ntiles,
+                                      hipMemcpyHostToDevice, c->stream));
                 st.tile_key = key;
                 st.key_T = T; st.key_S = S; st.key_W = W; st.key_Wi = c->Wi;
                 st.key_ER = c->ER;
@@ -800,6 +969,7 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st) {
                 st.n_corner = (int)te.size();
                 st.n_rowedge = (int)tr.size();
                 st.res_key_form = c->form;
+                st.key_together = together;
                 st.nres = 0;
                 if (!trs.empty()) {
                     rc = ensure_res_staging(c, st, (int)trs.size());
@@ -811,7 +981,7 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st) {
                     st.tile_key = key;  // ensure_res_staging may have cleared it
                 }
             }
-            bool resident = want_res && st.nres > 0 && !c->res_refused;
+            bool resident = st.nres > 0 && !c->res_refused;
             if (st.staged) HIPCHK(hipEventRecord(st.staged, c->stream));
             const int n_edge = st.n_edge, n_inner = st.ntiles - st.n_edge;
             const int cap = c->cus * c->grid_mult;
@@ -826,13 +996,13 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st) {
             for (int k = 0; k < 3; ++k) nside += cnt[k] > 0;
             bool fused = mode == TOMO_MODE_PHYSICAL && !resident && !wave &&
                          (c->form == TOMO_FORM_FUSED || c->form == TOMO_FORM_RESIDENT || c->form == TOMO_FORM_TILE);
-            bool multi = mode == TOMO_MODE_PHYSICAL && !fused && !resident && !wave && n_inner > 0 && nside > 0;
+            bool multi = mode == TOMO_MODE_PHYSICAL && !rtile && !fused && !resident && !wave && n_inner > 0 && nside > 0;
             // per-class cell-steps and bytes of block o (kernel timing only)
             auto block_work = [&](int o, int k, double& cells, double& bytes) {
                 cells = bytes = 0;
                 if (!c->prof) return;
                 for (size_t i = 0; i < ms.size(); ++i) {
-                    const int nst = std::min(T, h_it[i].nsteps - o * T);
+                    const int nst = std::min(Tb, h_it[i].nsteps - o * Tb);
                     if (nst <= 0) continue;
                     cells += nst * ms[i]->cls_cells[k];
                     bytes += nst * ms[i]->cls_bytes[k];
@@ -857,7 +1027,7 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st) {
                     HIPCHK(launch_zero(st.d_flags, (sizeof(int) * st.nres + 15) & ~(size_t)15, c->stream));
                     hipEvent_t a = c->prof ? pool_event(c) : nullptr, b = c->prof ? pool_event(c) : nullptr;
                     if (a && b) HIPCHK(hipEventRecord(a, c->stream));
-                    const hipError_t le = launch_tres(T, S, mode, st.d_res, st.nres, d_it, st.d_sims, st.d_flags,
+                    const hipError_t le = launch_tres(T, S, st.d_res, st.nres, d_it, st.d_sims, st.d_flags,
                                                       res_err(st), kResSpinLimit, c->stream);
                     if (le == hipSuccess) {
                         if (a && b) {
@@ -886,6 +1056,15 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st) {
                         block_work(o, k, cells[k], bytes[k]);
                         ucells += cells[k];
                         ubytes += bytes[k];
+                    }
+                    if (rtile) {
+                        LaunchTimer lt(c);
+                        HIPCHK(launch_rtile(mode, plan.waves, (const RegTile*)st.d_tiles, st.ntiles, d_it, st.d_sims, o, Tb,
+                                            c->stream));
+                        const int k = mode == TOMO_MODE_PHYSICAL ? TILE_INNER : TILE_CORNER;
+                        lt.done(mode == TOMO_MODE_PHYSICAL ? TOMO_KERNEL_FUSED : TOMO_KERNEL_GENERAL, cells[k], bytes[k]);
+                        if (!first) first = lt.a;
+                        continue;
                     }
                     if (mode != TOMO_MODE_PHYSICAL) {  // (the resident form skipped this loop)
                         LaunchTimer lt(c);
@@ -968,10 +1147,10 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st) {
                     maxn = std::max(maxn, h_it[i].nsteps);
                     minn = std::min(minn, h_it[i].nsteps);
                 }
-                nl = (maxn + T - 1) / T;
+                nl = (maxn + Tb - 1) / Tb;
                 if (c->use_graph && !st.fixed && !resident && !c->prof && minn == K) {
                     const std::vector<int64_t> gk = {mode, T, S, c->Si, W, c->Wi, c->ER, c->form, K, c->grid_mult, ntiles, maxP,
-                                                     fp32_any, fp64_any, (int64_t)ms.size(), (int64_t)(intptr_t)d_it,
+                                                     fp32_any, fp64_any, (int64_t)ms.size(), plan.T, plan.waves, (int64_t)(intptr_t)d_it,
                                                      (int64_t)(intptr_t)st.d_tiles, (int64_t)(intptr_t)st.d_sims};
                     if (!c->gexec || gk != c->gkey || key != c->gkey_serials) {
                         if (c->gexec) {
@@ -1006,7 +1185,7 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st) {
                     Slot* s = ms[i];
                     const int ns = h_it[i].nsteps;
                     s->done += ns;
-                    s->parity ^= ((ns + T - 1) / T) & 1;
+                    s->parity ^= ((ns + Tb - 1) / Tb) & 1;
                 }
             }  // staged epochs
             std::vector<Slot*> next;
@@ -1110,10 +1289,10 @@ static int project(tomo_ctx* c, const std::vector<Slot*>& sl, const std::vector<
 
 // Run the given simulations (all of one configuration) to completion and
 // project them; D_dev receives [slot][freq][angle].
-static int run_and_project(tomo_ctx* c, const std::vector<Slot*>& sl, float* dD, float* dP) {
+static int run_and_project(tomo_ctx* c, const std::vector<Slot*>& sl, float* dD, float* dP, bool together) {
     int rc = check_uniform_precision(sl);
     if (rc) return rc;
-    rc = run_epochs(c, sl, stage(c));
+    rc = run_epochs(c, sl, stage(c), together);
     if (rc) return rc;
     std::vector<int> off;
     for (size_t i = 0; i < sl.size(); ++i) off.push_back((int)(i * sl[i]->su.cfg.n_freq * sl[i]->su.cfg.n_angles));
@@ -1160,7 +1339,7 @@ static int eval_many(tomo_ctx* c, const tomo_sim_config& cfg, const double* para
                 rc = slot_create(c, cfg, params + v * dim, dim, e, &s);
                 if (rc) break;
                 std::vector<Slot*> one{s};
-                rc = run_and_project(c, one, dD + v * L + (size_t)e * F * A, dP + v * L + (size_t)e * F * A);
+                rc = run_and_project(c, one, dD + v * L + (size_t)e * F * A, dP + v * L + (size_t)e * F * A, false);
                 slot_destroy(c, s);
             }
         }
@@ -1187,7 +1366,7 @@ static int eval_many(tomo_ctx* c, const tomo_sim_config& cfg, const double* para
                 sl.insert(sl.end(), mine.begin(), mine.end());
             }
         run_pass:
-            if (!rc) rc = run_and_project(c, sl, dD + v0 * L, dP + v0 * L);
+            if (!rc) rc = run_and_project(c, sl, dD + v0 * L, dP + v0 * L, true);
             for (Slot* s : sl) slot_destroy(c, s);
             v0 = v;
         }
@@ -1237,7 +1416,7 @@ static int get_target(tomo_ctx* c, const tomo_sim_config& cfg, std::vector<float
     float *dD = nullptr, *dP = nullptr;
     if (!rc && hipMalloc(&dD, L * 4) != hipSuccess) rc = fail(TOMO_E_HIP, "hipMalloc");
     if (!rc && hipMalloc(&dP, L * 4) != hipSuccess) rc = fail(TOMO_E_HIP, "hipMalloc");
-    if (!rc) rc = run_and_project(c, sl, dD, dP);
+    if (!rc) rc = run_and_project(c, sl, dD, dP, true);
     if (!rc) {
         out.resize(L);
         if (hipMemcpy(out.data(), dD, L * 4, hipMemcpyDeviceToHost) != hipSuccess) rc = fail(TOMO_E_HIP, "copy");
@@ -1344,7 +1523,7 @@ static int progress_once(tomo_ctx* c, int* n_active) {
             s->target = std::min(s->su.cfg.steps, s->done + c->K);
             run.push_back(s);
         }
-        int rc = run_epochs(c, run, stage(c));
+        int rc = run_epochs(c, run, stage(c), true);
         if (rc) return rc;
         // retire
         std::vector<Slot*> still;
@@ -1476,7 +1655,7 @@ int eval_noalloc(tomo_ctx* c, char* base, const tomo_sim_config& cfg, const doub
         s->exc = e;
         s->target = cfg.steps;
         const std::vector<Slot*> one{s};
-        rc = run_epochs(c, one, st);
+        rc = run_epochs(c, one, st, false);
         if (rc) return rc;
         rc = project(c, one, {0}, dD + (size_t)e * F * A, dP + (size_t)e * F * A, tbl, pstage, kNoallocProjBytes);
         if (rc) return rc;
@@ -1609,6 +1788,7 @@ static int set_schedule_locked(tomo_ctx* c, const tomo_schedule& s) {
         (s.inner_rows != 0 && (s.inner_rows < 4 || s.inner_rows > 4096)))
         return fail(TOMO_E_INVALID, "bad schedule");
     c->T = T; c->S = S; c->W = W; c->Wi = Wi; c->K = K; c->grid_mult = G; c->form = F; c->ER = ER;
+    if (s.form) c->form_set = true;
     c->Si = s.inner_rows;
     return TOMO_OK;
 }
@@ -1635,12 +1815,12 @@ static int time_epochs(tomo_ctx* c, std::vector<Slot*>& sl, int epochs, double* 
     hipEvent_t a = pool_event(c), b = pool_event(c);
     if (!a || !b) return fail(TOMO_E_HIP, "event");
     for (Slot* s : sl) s->target = std::min(s->su.cfg.steps, s->done + c->K);
-    int rc = run_epochs(c, sl, stage(c));  // untimed: rebuilds and uploads the tile list
+    int rc = run_epochs(c, sl, stage(c), sl.size() > 1);  // untimed: rebuilds and uploads the tile list
     if (rc) return rc;
     HIPCHK(hipEventRecord(a, c->stream));
     for (int e = 0; e < epochs; ++e) {
         for (Slot* s : sl) s->target = std::min(s->su.cfg.steps, s->done + c->K);
-        rc = run_epochs(c, sl, stage(c));
+        rc = run_epochs(c, sl, stage(c), sl.size() > 1);
         if (rc) return rc;
     }
     HIPCHK(hipEventRecord(b, c->stream));
@@ -1918,7 +2098,7 @@ int tomo_sim_step(tomo_sim* sim, int nsteps) {
     std::lock_guard<std::mutex> g(c->mu);
     s->target = std::min(s->su.cfg.steps, s->done + nsteps);
     std::vector<Slot*> one{s};
-    rc = run_epochs(c, one, stage(c));
+    rc = run_epochs(c, one, stage(c), false);
     if (rc) return rc;
     HIPCHK(hipStreamSynchronize(c->stream));
     return TOMO_OK;

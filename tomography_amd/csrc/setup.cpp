@@ -250,23 +250,33 @@ static inline bool in_disc_f32(int x, int y, const tomo_sim_config& c, float r2)
     return s <= r2;
 }
 
-static void physical_spans(const tomo_sim_config& c, SimSetup& s) {
-    // Dispersive tissue is painted only inside the inner (fat) disc.
-    s.span.assign(3 * (c.ny + 1), 0);
-    int off = 0;
+// Columns [lo, hi) of a row inside the disc of squared radius r2 around the
+// grid's centre (lo == hi: none).
+static void disc_row(const tomo_sim_config& c, int y, float r2, int* lo, int* hi) {
     const int cx = c.nx / 2;
+    *lo = *hi = 0;
+    if (!in_disc_f32(cx, y, c, r2)) return;
+    int l = cx, h = cx;
+    while (l - 1 >= 0 && in_disc_f32(l - 1, y, c, r2)) --l;
+    while (h + 1 <= c.nx && in_disc_f32(h + 1, y, c, r2)) ++h;
+    *lo = l;
+    *hi = h + 1;
+}
+
+static void physical_spans(const tomo_sim_config& c, SimSetup& s) {
+    // Dispersive tissue is painted only inside the inner (fat) disc, tissue of
+    // any kind only inside the outer one.
+    s.span.assign(3 * (c.ny + 1), 0);
+    s.mspan.assign(2 * (c.ny + 1), 0);
+    int off = 0;
     for (int y = 0; y <= c.ny; ++y) {
-        int lo = 0, hi = 0;
-        if (in_disc_f32(cx, y, c, s.geom.ri2)) {
-            int l = cx, h = cx;
-            while (l - 1 >= 0 && in_disc_f32(l - 1, y, c, s.geom.ri2)) --l;
-            while (h + 1 <= c.nx && in_disc_f32(h + 1, y, c, s.geom.ri2)) ++h;
-            lo = l; hi = h + 1;
-        }
+        int lo, hi;
+        disc_row(c, y, s.geom.ri2, &lo, &hi);
         s.span[3 * y] = lo;
         s.span[3 * y + 1] = hi;
         s.span[3 * y + 2] = off;
         off += hi - lo;
+        disc_row(c, y, s.geom.ro2, &s.mspan[2 * y], &s.mspan[2 * y + 1]);
     }
     s.jp_len = off;
 }
@@ -284,6 +294,7 @@ static int ref_raster(const tomo_sim_config& c, SimSetup& s) {
     for (int i = 0; i <= nx; ++i) rr.xc[i] = (int)((i - (nx / 2 - (int)(R / dx))) / (2 * R / (np * dx)));
     for (int j = 0; j <= ny; ++j) rr.yc[j] = (int)((j - (ny / 2 - R / dy)) / (2 * R / (np * dy)));
     s.span.assign(3 * (ny + 1), 0);
+    s.mspan.assign(2 * (ny + 1), 0);
     int off = 0;
     for (int j = 0; j <= ny; ++j) {
         int lo = -1, hi = -2;
@@ -302,6 +313,8 @@ static int ref_raster(const tomo_sim_config& c, SimSetup& s) {
         s.span[3 * j] = slo;
         s.span[3 * j + 1] = shi;
         s.span[3 * j + 2] = off;
+        s.mspan[2 * j] = slo;
+        s.mspan[2 * j + 1] = shi;
         off += shi - slo;
     }
     s.jp_len = off;
@@ -421,7 +434,7 @@ struct ConfigProducts {
     std::vector<float> srcw;
     double inv_norm[TOMO_MAX_FREQ] = {};
     RefRaster ref;
-    std::vector<int> span;
+    std::vector<int> span, mspan;
     int jp_len = 0;
     bool has_ref = false, has_phys = false;
 };
@@ -487,11 +500,13 @@ int build_setup(const tomo_sim_config& c, const double* p, size_t np, int exc, S
                 if ((rc = ref_raster(c, tmp))) return rc;
                 cp->ref = tmp.ref;
                 cp->span = tmp.span;
+                cp->mspan = tmp.mspan;
                 cp->jp_len = tmp.jp_len;
                 cp->has_ref = true;
             }
             s.ref = cp->ref;
             s.span = cp->span;
+            s.mspan = cp->mspan;
             s.jp_len = cp->jp_len;
         }
         ref_cpml(c, s);

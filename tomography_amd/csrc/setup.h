@@ -60,6 +60,7 @@ struct SimSetup {
     RefRaster ref;
     std::vector<int> span;            // lo, hi, off per row
     int jp_len = 0;
+    std::vector<int> mspan;           // per row: first and end column of the cells that are not vacuum
     int sx = -1, sy = -1;
     std::vector<float> srcw;
     float inc_dt = 0, inc_c = 0, inc_ax = 0, inc_ay = 0, inc_itau = 0;

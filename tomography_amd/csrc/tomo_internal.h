@@ -99,6 +99,17 @@ struct TileItem {
     int pad;
 };
 
+// Tile of the register-tile update: 64 columns from xl times waves * rows rows
+// from yl, held in registers for one time block, of which the columns [x0, xe)
+// and rows [y0, y1) are owned (written back, sampled).
+struct RegTile {
+    int item;      // index into the LaunchItem array
+    int sim;       // index into the DevSim table (-1: no tile)
+    int xl, x0, xe;
+    int yl, y0, y1;
+    int rows;      // rows per wave
+    int matmask;   // bit w: wave w holds a cell that is not vacuum
+};
 
 // Tile of the resident update form: one workgroup keeps a band of 64 lanes
 // (owned columns [x0, x0 + 64 - 2T), T ghost columns on each side) times the

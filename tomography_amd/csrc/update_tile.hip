@@ -1,0 +1,587 @@
+// update_tile.hip — the register-tile update kernel: one launch advances every
+// tile of every simulation by one time block (replaces H_field_update +
+// E_field_update + calculate_JandM's sampling, FDTD_GPU.cu:231-434).
+//
+// A workgroup of NW waves holds 64 columns times NW * R rows, R rows per wave,
+// one column per lane, in registers; it requests them all at once, advances
+// them up to 24 steps and stores the cells it owns.  A step invalidates one
+// lane and one row at each edge of the tile that is not the grid's edge, so
+// tiles overlap by twice the block's steps.  Waves couple through LDS: each
+// publishes its bottom and top Ez rows, advances what needs no neighbour (H of
+// all rows but the top one, E of the rows between), meets the others at the
+// step's only barrier and finishes its two edge rows.  The Hx of the row below
+// a wave is advanced by both waves, so H needs no exchange.
+//
+// Against the row sweeps (kernels.hip) no row waits for a memory round trip or
+// for the stage before it, no register moves from stage to stage, and a wave
+// takes the stage its cells need: the bare vacuum one (9 VALU instructions a
+// row; 92% of a 256 mm domain is vacuum), with material coefficients in
+// registers, or with the CPML recursions of its columns and rows.  All of them
+// round as the row sweeps do, so every form gives the same bits.
+//
+// What bounds it: a single grid's launch is 5 us of dispatch, first loads and
+// last stores, and per step one tile's own instruction issue (R rows of the
+// costliest stage on NW / 4 waves of a SIMD) and the LDS exchange; a batch is
+// bound by VALU issue, a fifth to a half of it on ghost cells.  Edge tiles take
+// 4 rows per wave (a corner row in material costs 3 times a vacuum one) and
+// clean ones 8, which also keeps both under the 128 VGPRs of four waves per SIMD.
+// Measured (evaluations, row sweeps -> register tiles): 256^2 9.5 -> 3.3 ms,
+// 725^2 27.2 -> 12.8, 1024^2 39.6 -> 21.5, 64 simulations of 512^2 174 -> 131;
+// the reference's 4 x 401^2 24.5 (resident form) -> 7.0, 16 of them 106 -> 15.4.
+#include "device.h"
+#include "kernels.h"
+
+namespace tomo {
+namespace {
+
+constexpr int kLane = 64;
+
+// Lane shifts on the VALU (DPP wave_shl:1 / wave_shr:1), folded by the compiler
+// into the subtraction that uses them: next(v)[i] = v[i+1], prev(v)[i] = v[i-1],
+// 0 past the edge lane (a ghost lane, or a lane whose result is masked).
+__device__ __forceinline__ float next_lane(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x130, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float prev_lane(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x138, 0xF, 0xF, true));
+}
+
+__device__ __forceinline__ float read_lane(float v, int i) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), i));
+}
+
+// a / k for a divisor whose reciprocal r = 1 / (double)k is known: the product in
+// 64 bits is within 2^-52 of the quotient, which (a ratio of two 24-bit
+// numbers) lies at least 2^-49 from any point where rounding to 32 bits turns,
+// so this is the division's own result (but for ties among denormal results) in
+// three instructions instead of eleven.
+__device__ __forceinline__ float div_known(float a, double r) { return (float)((double)a * r); }
+
+// Barrier over the LDS traffic alone: the sample and field stores in flight are
+// not waited for.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// CPML coefficients of a row or a lane.  Off the strips 1/kappa = 1 and
+// a = b = 0, so that strip cells and others take the same instructions; r = 0
+// marks them for the reference's stage.
+struct alignas(16) Profile {
+    float a, b;
+    union {
+        float ik;  // 1/kappa, physical mode
+        double r;  // 1/kappa, reference-compatible mode (which divides by kappa)
+    };
+};
+
+template <int NW>
+struct TileLds {
+    float4 coef[TOMO_MAX_MAT * 2];        // filled when a wave of the tile holds material
+    Profile row_e[NW * kTileRowsEdge], row_h[NW * kTileRowsEdge + 1];  // of E row yl + i and of H row yl - 1 + i
+    float ez[2][NW][2][kLane];            // per step parity: each wave's bottom and top Ez row
+};
+
+// CPML profile entry of E node v (1..n-1) and of H node v (0..n-1) of a line of
+// n cells, -1 off the strips.
+__device__ __forceinline__ int strip_e(int v, int n, int nc) {
+    return (v >= 1 && v <= nc) ? nc - v : ((v >= n - nc && v <= n - 1) ? v - n + nc : -1);
+}
+__device__ __forceinline__ int strip_h(int v, int n, int nc) {
+    return (v >= 0 && v < nc) ? nc - 1 - v : ((v >= n - nc && v < n) ? v - n + nc : -1);
+}
+template <bool REF>
+__device__ __forceinline__ Profile profile(float k, float ik, float a, float b, int i) {
+    Profile p;
+    p.a = i < 0 ? 0.f : a;
+    p.b = i < 0 ? 0.f : b;
+    if constexpr (REF) p.r = i < 0 ? 0.0 : 1.0 / (double)k;
+    else p.ik = i < 0 ? 1.f : ik;
+    return p;
+}
+template <bool REF>
+__device__ __forceinline__ Profile profile_e(const DevSim* __restrict__ S, int i) {
+    const int j = max(i, 0);
+    return profile<REF>(S->ke[j], S->ike[j], S->ae[j], S->be[j], i);
+}
+template <bool REF>
+__device__ __forceinline__ Profile profile_h(const DevSim* __restrict__ S, int i) {
+    const int j = max(i, 0);
+    return profile<REF>(S->km[j], S->ikm[j], S->am[j], S->bm[j], i);
+}
+
+// Wave-uniform value that the compiler may not fold into values computed
+// outside a loop: row conditions then cost a scalar compare where they are
+// used and hold no scalar register across the step loop.
+__device__ __forceinline__ int opaque(int v) {
+    v = __builtin_amdgcn_readfirstlane(v);
+    asm volatile("" : "+s"(v));
+    return v;
+}
+
+// One wave's share of a tile: R rows [yb, yb + R) of 64 columns [xl, xl + 64),
+// advanced nst steps.  XS / YS: the lanes / rows reach a CPML strip or the PEC
+// edge; MAT: some cell is not vacuum; SRC: the source cell is one of the wave's
+// and may lie in material.
+template <int MODE, int R, int NW, bool XS, bool YS, bool MAT, bool SRC>
+__device__ __forceinline__ void tile_wave(const RegTile& tile, const DevSim* __restrict__ Sp, TileLds<NW>& lds,
+                                          int par, int step0, int k0, int nst, int wv, int lane, bool tables, bool frows) {
+    constexpr bool REF = MODE == TOMO_MODE_REF_COMPAT;
+    const int nx = Sp->nx, ny = Sp->ny, nc = Sp->nc, pitch = Sp->pitch, ps = Sp->ps;
+    const int x = tile.xl + lane, yb = tile.yl + wv * R;
+    const int w2 = 2 * nc;
+    // x-strip columns of the lane in the psi arrays
+    const int je = (x >= 1 && x <= nc) ? x - 1 : ((x >= nx - nc && x <= nx - 1) ? nc + x - (nx - nc) : -1);
+    const int jh = x < nc ? x : ((x >= nx - nc && x < nx) ? nc + x - (nx - nc) : -1);
+    // psi rows of the y strips: E node rows 1..nc and ny-nc..ny-1, H rows 0..nc-1
+    // and ny-nc..ny-1 (a wave's rows never reach both strips: ny >= 2 nc + 4)
+    const bool hi = yb + R > ny - nc;
+    auto row_e = [&](int y) { return (unsigned)(hi ? y - (ny - nc) : y - 1) < (unsigned)nc; };
+    auto row_h = [&](int y) { return (unsigned)(hi ? y - (ny - nc) : y) < (unsigned)nc; };
+    const int re0 = hi ? 2 * nc - ny : -1, rh0 = hi ? 2 * nc - ny : 0;
+    // Scalar plane bases and one 32-bit byte offset per lane and row (the planes
+    // are smaller than 4 GiB).
+    auto at = [](gcfloat* base, unsigned off) { return *(gcfloat*)((GAS const char*)base + off); };
+    auto to = [](gfloat* base, unsigned off, float v) { *(gfloat*)((GAS char*)base + off) = v; };
+    const unsigned o0 = ((unsigned)yb * (unsigned)pitch + (unsigned)x) * 4u, op = (unsigned)pitch * 4u;
+
+    // ---- the whole tile is requested at once: no row waits for another
+    float ez[R], hx[R], hy[R], jp[MAT ? R : 1], phx[XS ? R : 1], pex[XS ? R : 1], phy[YS ? R : 1], pey[YS ? R : 1];
+    int mat[MAT ? R : 1];
+    float hxb, phyb = 0.f;  // Hx (and its psi) of the row below the wave, which it advances beside its own
+    {
+        gcfloat* fe = (gcfloat*)Sp->fbase + (size_t)par * ps;
+        gcfloat* fx = fe + 2 * (size_t)ps;
+        gcfloat* fy = fe + 4 * (size_t)ps;
+        if constexpr (MAT) {
+#pragma unroll
+            for (int i = 0; i < R; ++i) mat[i] = ((gcu8*)Sp->mat)[(o0 + i * op) >> 2];
+        }
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            ez[i] = at(fe, o0 + i * op);
+            hx[i] = at(fx, o0 + i * op);
+            hy[i] = at(fy, o0 + i * op);
+        }
+        hxb = at(fx, yb > 0 ? o0 - op : o0);
+        if constexpr (MAT) {
+            kcint* span = (kcint*)Sp->span;
+            gcfloat* jin = (gcfloat*)Sp->jbase + (size_t)par * Sp->js;
+#pragma unroll
+            for (int i = 0; i < R; ++i) {
+                const int lo = span[3 * (yb + i)], hi = span[3 * (yb + i) + 1], off = span[3 * (yb + i) + 2];
+                jp[i] = 0.f;
+                if (x >= lo && x < hi) jp[i] = at(jin, (unsigned)(off - lo + x) * 4u);
+            }
+        }
+        if constexpr (XS) {
+            gcfloat* pe = (gcfloat*)Sp->xbase + (size_t)par * Sp->xs;
+            gcfloat* ph = pe + 2 * (size_t)Sp->xs;
+            const unsigned qe = (unsigned)(yb * w2 + max(je, 0)) * 4u, qh = (unsigned)(yb * w2 + max(jh, 0)) * 4u;
+#pragma unroll
+            for (int i = 0; i < R; ++i) {
+                pex[i] = at(pe, qe + (unsigned)(i * w2) * 4u);
+                phx[i] = at(ph, qh + (unsigned)(i * w2) * 4u);
+            }
+        }
+        if constexpr (YS) {
+            gcfloat* pe = (gcfloat*)Sp->ybase + (size_t)par * Sp->ys;
+            gcfloat* ph = pe + 2 * (size_t)Sp->ys;
+#pragma unroll
+            for (int i = 0; i < R; ++i) {
+                pey[i] = at(pe, (unsigned)(min(max(yb + i + re0, 0), w2 - 1) * pitch + x) * 4u);
+                phy[i] = at(ph, (unsigned)(min(max(yb + i + rh0, 0), w2 - 1) * pitch + x) * 4u);
+            }
+            phyb = at(ph, (unsigned)(min(max(yb - 1 + rh0, 0), w2 - 1) * pitch + x) * 4u);
+        }
+    }
+    // the tile's tables, while those loads are on their way
+    if (tables) {
+        if (tile.matmask) {
+            float* lcf = (float*)lds.coef;
+            for (int i = threadIdx.x; i < Sp->nmat * TOMO_NCOEF; i += NW * kLane) lcf[i] = Sp->coef[i];
+        }
+        if (frows) {
+            for (int i = threadIdx.x; i <= NW * R; i += NW * kLane) {
+                if (i < NW * R) lds.row_e[i] = profile_e<REF>(Sp, strip_e(tile.yl + i, ny, nc));
+                lds.row_h[i] = profile_h<REF>(Sp, strip_h(tile.yl - 1 + i, ny, nc));
+            }
+        }
+        lds_barrier();
+    }
+    const float chx = Sp->chx, chy = Sp->chy, dxf = Sp->dxf, dyf = Sp->dyf, chx_d = Sp->chx_d, chy_d = Sp->chy_d;
+    const float cb0 = Sp->coef[1];  // vacuum curl coefficient (the vacuum Ez coefficient is exactly 1)
+    const bool clamp = REF && !(Sp->flags & TOMO_FLAG_NO_NAN_CLAMP);
+    const bool ex_ok = !XS || (x >= 1 && x < nx);
+    const bool bot = YS && yb == 0, top = YS && yb + R - 1 == ny;  // PEC rows: the wave's first, its last
+    Profile Le, Lh;
+    if constexpr (XS) {
+        Le = profile_e<REF>(Sp, strip_e(x, nx, nc));
+        Lh = profile_h<REF>(Sp, strip_h(x, nx, nc));
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            pex[i] = je >= 0 ? pex[i] : 0.f;
+            phx[i] = jh >= 0 ? phx[i] : 0.f;
+        }
+    }
+    if constexpr (YS) {
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            pey[i] = row_e(yb + i) ? pey[i] : 0.f;
+            phy[i] = row_h(yb + i) ? phy[i] : 0.f;
+        }
+        phyb = row_h(yb - 1) ? phyb : 0.f;
+        hxb = bot ? 0.f : hxb;
+    }
+    float4 qa[MAT ? R : 1], qb[MAT ? R : 1];
+    float f0[MAT && REF ? R : 1];  // the incident field half a step back: each step's new one is the next step's old
+    auto delay = [&](int i) {
+        const float X = Sp->inc_abs_origin ? (float)x : (float)(x - nx / 2);
+        const float Y = Sp->inc_abs_origin ? (float)(yb + i) : (float)(yb + i - ny / 2);
+        return Sp->inc_c - Sp->inc_ay * Y - Sp->inc_ax * X;
+    };
+    if constexpr (MAT) {
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            qa[i] = lds.coef[2 * mat[i]];
+            qb[i] = lds.coef[2 * mat[i] + 1];
+            if constexpr (REF) {
+                const float a0 = (((float)step0 - 0.5f) * Sp->inc_dt + delay(i)) * Sp->inc_itau;
+                f0[i] = expf(-a0 * a0);
+            }
+        }
+    }
+
+    // ---- contour samples: face rows / columns hold H and Ez, their outer neighbours Ez
+    const int D = Sp->D, P = Sp->P, K = Sp->chunk, cx_hi = Sp->cx_hi, cy_lo = Sp->cy_lo;
+    const bool own = x >= tile.x0 && x < tile.xe;
+    gfloat* samp = (gfloat*)Sp->samp;
+    // rows of the wave that the tile owns: [ra, rb)
+    const int ra = max(tile.y0 - yb, 0), rb = min(tile.y1 - yb, R);
+    // bits of the owned rows that are face rows and their outer neighbours (lo:
+    // the bottom leg's), and of the rows in the x legs' range
+    const unsigned mine = rb > ra ? ((1u << rb) - 1u) & ~((1u << ra) - 1u) : 0u;
+    auto bit = [&](int y) { return (unsigned)(y - yb) < (unsigned)R ? 1u << (y - yb) : 0u; };
+    const int m_face = mine & (bit(D) | bit(ny - D - 1)), m_out = mine & (bit(D + 1) | bit(ny - D));
+    int m_x = 0;
+    auto has_col = [&](int c) { return c >= tile.x0 && c < tile.xe; };
+    if (has_col(D) || has_col(D + 1) || has_col(nx - D - 1) || has_col(nx - D)) {
+        const int a = min(max(cy_lo - yb, 0), R), z = min(max(ny - D - yb, 0), R);
+        m_x = z > a ? mine & ((1u << z) - 1u) & ~((1u << a) - 1u) : 0;
+    }
+    const bool y_lane = own && x >= D + 1 && x <= cx_hi;
+    const bool x_face = x == D || x == nx - D - 1;
+    const bool x_lane = own && (x_face || x == D + 1 || x == nx - D);
+    const int x_dir = x >= nx - D - 1 ? 1 : -1;
+    const unsigned x_off = (unsigned)((x >= nx - D - 1 ? Sp->L1 - cy_lo : Sp->L3 + ny - D - 1) + x_dir * yb) + (x_face ? 0u : 2u * K * P);
+    const int L2 = Sp->L2;
+    auto sample = [&](int k) {
+        gfloat* sk = samp + (size_t)k * P;
+        const int f = opaque(m_face), o = opaque(m_out), xr = opaque(m_x);
+        if (f | o) {
+            // a wave holds rows of both y legs only on grids of a few rows
+            if (y_lane) {
+#pragma unroll
+                for (int i = 0; i < R; ++i) {
+                    if (!((f | o) >> i & 1)) continue;  // wave-uniform
+                    const unsigned p = 2 * (yb + i) < ny ? x - D - 1 : L2 + (cx_hi - x);
+                    if (f >> i & 1) {
+                        sk[p] = hx[i];
+                        (sk + (size_t)K * P)[p] = ez[i];
+                    } else {
+                        (sk + 2 * (size_t)K * P)[p] = ez[i];
+                    }
+                }
+            }
+        }
+        if (xr && x_lane) {
+            unsigned p = x_off;
+#pragma unroll
+            for (int i = 0; i < R; ++i) {
+                if (xr >> i & 1) {  // wave-uniform
+                    sk[p] = x_face ? hy[i] : ez[i];
+                    if (x_face) (sk + (size_t)K * P)[p] = ez[i];
+                }
+                p += x_dir;
+            }
+        }
+    };
+
+    // ---- source
+    const int isrc = Sp->sy - yb;  // row of the source, if it is one of the wave's
+    const bool wsrc = !REF && isrc >= 0 && isrc < R && Sp->sx >= tile.xl && Sp->sx < tile.xl + kLane;
+    const bool lsrc = x == Sp->sx;
+    const bool extra = wsrc || (m_face | m_out | m_x) != 0;  // a step has more to do than the update
+    float sw = 0.f;  // lane t: the waveform of the block's step t
+    if (wsrc && lane < nst) sw = ((gcfloat*)Sp->srcw)[step0 + lane];
+
+    // H half-step of one row, in place; the psi of the strips advance with it.
+    // Columns x = nx and the row y = ny have no H nodes: their Ez and the Ez
+    // beyond them are 0 (next_lane past lane 63, ez_up above the top row), so
+    // their H and psi, loaded as 0, stay 0 without a mask.
+    auto h_step = [&](float ez_c, float ez_up, float& hx_, float* hy_, float* phx_, float* phy_, const Profile W) {
+        const float dEy = ez_up - ez_c;
+        float hxn, tx = dEy;
+        if constexpr (REF) {
+            hxn = hx_ - chx * dEy;
+            if constexpr (YS) {
+                const float u = chx * dEy;
+                const float q = hx_ - div_known(u, W.r);
+                *phy_ = W.b * *phy_ + W.a * dEy;
+                hxn = W.r != 0.0 ? q - chx_d * *phy_ : hxn;
+            }
+            if (clamp) hxn = __builtin_isnan(hxn) ? 0.f : hxn;
+        } else {
+            if constexpr (YS) {
+                *phy_ = W.b * *phy_ + W.a * dEy;
+                tx = dEy * W.ik + dyf * *phy_;
+            }
+            hxn = hx_ - chx * tx;
+        }
+        hx_ = hxn;
+        if (!hy_) return;
+        const float dEx = next_lane(ez_c) - ez_c;
+        float hyn, ty = dEx;
+        if constexpr (REF) {
+            hyn = *hy_ + chy * dEx;
+            if constexpr (XS) {
+                const float u = chy * dEx;
+                const float q = *hy_ + div_known(u, Lh.r);
+                *phx_ = Lh.b * *phx_ + Lh.a * dEx;
+                hyn = jh >= 0 ? q + chy_d * *phx_ : hyn;
+            }
+            if (clamp) hyn = __builtin_isnan(hyn) ? 0.f : hyn;
+        } else {
+            if constexpr (XS) {
+                *phx_ = Lh.b * *phx_ + Lh.a * dEx;
+                ty = dEx * Lh.ik + dxf * *phx_;
+            }
+            hyn = *hy_ + chy * ty;
+        }
+        *hy_ = hyn;
+    };
+    // E half-step of row i given its new H and the new Hx of the row below;
+    // `edge`: a PEC row.
+    auto e_step = [&](int i, float hx_dn, int n, float s, const Profile W, bool edge) {
+        const float dHy = hy[i] - prev_lane(hy[i]);
+        const float dHx = hx[i] - hx_dn;
+        const bool eok = ex_ok && !(YS && edge);
+        const float e0 = ez[i];
+        float4 A = make_float4(1.f, cb0, 0.f, 0.f), B = make_float4(0.f, 0.f, 0.f, 0.f);
+        if constexpr (MAT) {
+            A = qa[i];
+            B = qb[i];
+        }
+        float en;
+        if constexpr (REF) {
+            if constexpr (MAT) {
+                const float a1 = (((float)n + 0.5f) * Sp->inc_dt + delay(i)) * Sp->inc_itau;
+                const float f1 = expf(-a1 * a1), fo = f0[i];
+                f0[i] = f1;
+                en = A.x * e0 + A.y * dHy - A.y * dHx + A.z * f1 + A.w * fo - B.x * jp[i];
+                const float jn = B.y * jp[i] + B.z * (en - e0 + f1 - fo);
+                jp[i] = (XS || YS) ? (eok ? jn : 0.f) : jn;
+            } else {
+                const float u = A.y * dHy;
+                const float v = e0 + u;
+                en = v - A.y * dHx;
+            }
+            if constexpr (XS || YS) {
+                const float uy = A.y * dHy, ux = A.y * dHx;
+                if constexpr (XS) {
+                    pex[i] = edge ? pex[i] : Le.b * pex[i] + Le.a * dHy;
+                    float b = A.x * e0 + div_known(uy, Le.r);
+                    b = b - div_known(ux, Le.r);
+                    b = b + A.y * dxf * pex[i];
+                    en = je >= 0 ? b : en;
+                }
+                if constexpr (YS) {
+                    pey[i] = ex_ok ? W.b * pey[i] + W.a * dHx : pey[i];
+                    float b = A.x * e0 + div_known(uy, W.r);
+                    b = b - div_known(ux, W.r);
+                    b = b - A.y * dyf * pey[i];
+                    en = W.r != 0.0 ? b : en;
+                }
+            }
+            if (clamp) en = __builtin_isnan(en) ? 0.f : en;
+        } else {
+            float cy = dHy, cx = dHx;
+            if constexpr (XS) {
+                pex[i] = Le.b * pex[i] + Le.a * dHy;
+                cy = dHy * Le.ik + dxf * pex[i];
+            }
+            if constexpr (YS) {
+                pey[i] = W.b * pey[i] + W.a * dHx;
+                cx = dHx * W.ik + dyf * pey[i];
+            }
+            if constexpr (MAT) {
+                en = A.x * e0 + A.y * cy - A.y * cx - B.x * jp[i];
+                if constexpr (SRC) {
+                    if (i == opaque(isrc)) en = lsrc ? en + s : en;
+                }
+                // (a PEC node: Ez stays 0, and so does Jp)
+                if constexpr (XS || YS) en = eok ? en : 0.f;
+                jp[i] = B.y * jp[i] + B.z * (en - e0);
+            } else {
+                // the material expression with Ez coefficient 1 and no Jp: the same roundings
+                const float u = cb0 * cy;
+                const float v = e0 + u;
+                en = v - cb0 * cx;
+                if constexpr (XS || YS) en = eok ? en : 0.f;
+            }
+        }
+        if constexpr (REF && (XS || YS)) en = eok ? en : 0.f;
+        ez[i] = en;
+    };
+    const Profile* we = lds.row_e + wv * R;      // E row i
+    const Profile* wh = lds.row_h + wv * R + 1;  // H row i
+    auto E = [&](int i) { return YS ? we[i] : Profile{}; };
+    auto H = [&](int i) { return YS ? wh[i] : Profile{}; };
+    auto hs = [&](int i, float up) {
+        h_step(ez[i], up, hx[i], &hy[i], XS ? &phx[XS ? i : 0] : nullptr, YS ? &phy[YS ? i : 0] : nullptr, H(i));
+    };
+
+    const int wu = min(wv + 1, NW - 1), wd = max(wv - 1, 0);
+    for (int t = 0; t < nst; ++t) {
+        const int n = step0 + t, b = t & 1;
+        const float s = SRC ? read_lane(sw, t) : 0.f;
+        lds.ez[b][wv][0][lane] = ez[0];
+        lds.ez[b][wv][1][lane] = ez[R - 1];
+        // what needs no neighbour: H of all rows but the top one, E of the rows in between
+#pragma unroll
+        for (int i = 0; i + 1 < R; ++i) hs(i, ez[i + 1]);
+        const float ez0 = ez[0];
+#pragma unroll
+        for (int i = 1; i + 1 < R; ++i) e_step(i, hx[i - 1], n, s, E(i), false);
+        lds_barrier();
+        float ez_up = lds.ez[b][wu][0][lane], ez_dn = lds.ez[b][wd][1][lane];
+        if constexpr (YS) {
+            ez_up = top ? 0.f : ez_up;
+            ez_dn = bot ? 0.f : ez_dn;
+        }
+        h_step(ez_dn, ez0, hxb, nullptr, nullptr, &phyb, H(-1));
+        hs(R - 1, ez_up);
+        e_step(0, hxb, n, s, E(0), bot);
+        e_step(R - 1, hx[R - 2], n, s, E(R - 1), top);
+        if (extra) {
+            if constexpr (!MAT && !REF) {
+                // a source in vacuum: Jp does not see it, so it can be added to the finished row
+                if (wsrc) {
+                    const int is = opaque(isrc);
+                    const float sv = read_lane(sw, t);
+#pragma unroll
+                    for (int i = 0; i < R; ++i)
+                        if (i == is) ez[i] = lsrc ? ez[i] + sv : ez[i];
+                }
+            }
+            sample(k0 + t);
+        }
+    }
+
+    // ---- owned cells to the other buffer
+    const int keep = opaque(mine);
+    if (!own) return;
+    gfloat* fe = (gfloat*)Sp->fbase + (size_t)(par ^ 1) * ps;
+    gfloat* fx = fe + 2 * (size_t)ps;
+    gfloat* fy = fe + 4 * (size_t)ps;
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        if (!(keep >> i & 1)) continue;  // wave-uniform
+        to(fe, o0 + i * op, ez[i]);
+        to(fx, o0 + i * op, hx[i]);
+        to(fy, o0 + i * op, hy[i]);
+        const int y = yb + i;
+        if constexpr (MAT) {
+            kcint* span = (kcint*)Sp->span;
+            gfloat* jout = (gfloat*)Sp->jbase + (size_t)(par ^ 1) * Sp->js;
+            const int lo = span[3 * y], hi = span[3 * y + 1], off = span[3 * y + 2];
+            if (x >= lo && x < hi) to(jout, (unsigned)(off - lo + x) * 4u, jp[i]);
+        }
+        if constexpr (XS) {
+            gfloat* pe = (gfloat*)Sp->xbase + (size_t)(par ^ 1) * Sp->xs;
+            gfloat* ph = pe + 2 * (size_t)Sp->xs;
+            if (je >= 0) pe[y * w2 + je] = pex[i];
+            if (jh >= 0) ph[y * w2 + jh] = phx[i];
+        }
+        if constexpr (YS) {
+            gfloat* pe = (gfloat*)Sp->ybase + (size_t)(par ^ 1) * Sp->ys;
+            gfloat* ph = pe + 2 * (size_t)Sp->ys;
+            if (row_e(y)) pe[(y + re0) * pitch + x] = pey[i];
+            if (row_h(y)) ph[(y + rh0) * pitch + x] = phy[i];
+        }
+    }
+}
+
+template <int MODE, int NW>
+__global__ __launch_bounds__(NW* kLane) __attribute__((amdgpu_waves_per_eu(4))) void k_rtile(
+    const RegTile* __restrict__ tiles, const LaunchItem* __restrict__ items, const DevSim* __restrict__ sims, int ordinal,
+    int tsteps) {
+    __shared__ TileLds<NW> lds;
+    const RegTile tile = tiles[blockIdx.x];
+    if (tile.sim < 0) return;
+    const LaunchItem it = items[tile.item];
+    const DevSim* Sp = sims + tile.sim;
+    const int nst = min(tsteps, it.nsteps - ordinal * tsteps);
+    if (nst <= 0) return;  // uniform over the workgroup
+    const int lane = threadIdx.x & (kLane - 1);
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kLane);
+    const int par = it.parity0 ^ (ordinal & 1), step0 = it.step0 + ordinal * tsteps, k0 = ordinal * tsteps;
+    const bool mat = (tile.matmask >> wv) & 1;
+#define TW(R, XS, YS, MAT, SRC) \
+    tile_wave<MODE, R, NW, XS, YS, MAT, SRC>(tile, Sp, lds, par, step0, k0, nst, wv, lane, tables, frows)
+    if (tile.rows == kTileRowsClean) {
+        const bool tables = tile.matmask != 0, frows = false;
+        if constexpr (MODE == TOMO_MODE_PHYSICAL) {  // (reference-mode material takes 4-row tiles)
+            if (mat) {
+                TW(kTileRowsClean, false, false, true, false);
+                return;
+            }
+        }
+        TW(kTileRowsClean, false, false, false, false);
+        return;
+    }
+    constexpr int R = kTileRowsEdge;
+    const int nx = Sp->nx, ny = Sp->ny, nc = Sp->nc, yb = tile.yl + wv * R;
+    const bool xs = tile.xl <= nc || tile.xl + kLane > nx - nc;  // lanes reach a strip or an edge
+    const bool tys = tile.yl <= nc + 1 || tile.yl + NW * R > ny - nc;
+    // rows reach a strip or an edge (the row below the wave is advanced too)
+    const bool ys = yb <= nc + 1 || yb + R > ny - nc;
+    const bool tsrc = MODE == TOMO_MODE_PHYSICAL && Sp->sy >= tile.yl && Sp->sy < tile.yl + NW * R &&
+                      Sp->sx >= tile.xl && Sp->sx < tile.xl + kLane;
+    const bool src = tsrc && mat && Sp->sy >= yb && Sp->sy < yb + R;
+    // row profiles: also where the source lies in material, whose wave takes the general stage
+    const bool frows = tys || (tsrc && tile.matmask);
+    const bool tables = tile.matmask || frows;
+    if (src) TW(R, true, true, true, true);
+    else if (mat) {
+        if (xs) {
+            if (ys) TW(R, true, true, true, false);
+            else TW(R, true, false, true, false);
+        } else if (ys) TW(R, false, true, true, false);
+        else TW(R, false, false, true, false);
+    } else if (xs) {
+        if (ys) TW(R, true, true, false, false);
+        else TW(R, true, false, false, false);
+    } else if (ys) TW(R, false, true, false, false);
+    else TW(R, false, false, false, false);
+#undef TW
+}
+
+}  // namespace
+
+hipError_t launch_rtile(int mode, int waves, const RegTile* tiles, int ntiles, const LaunchItem* items, const DevSim* sims,
+                        int ordinal, int tsteps, hipStream_t st) {
+    if (ntiles <= 0) return hipErrorInvalidValue;
+    dim3 g(ntiles), b(waves * kLane);
+#define TT(MM, WW)                                                                                \
+    if (mode == MM && waves == WW) {                                                              \
+        TIMED_LAUNCH((k_rtile<MM, WW>), g, b, 0, st, tiles, items, sims, ordinal, tsteps);        \
+        return hipGetLastError();                                                                 \
+    }
+    TT(TOMO_MODE_PHYSICAL, 8) TT(TOMO_MODE_PHYSICAL, 16) TT(TOMO_MODE_REF_COMPAT, 8) TT(TOMO_MODE_REF_COMPAT, 16)
+#undef TT
+    return hipErrorInvalidValue;
+}
+
+}  // namespace tomo
