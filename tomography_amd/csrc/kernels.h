@@ -48,11 +48,12 @@ hipError_t launch_twave(int T, int rows_per_wave, const TileItem* tiles, int nti
 // Register-tile update: one workgroup of `waves` (8 or 16) waves per RegTile
 // advances it one time block of `tsteps` steps.  Every held node is a node of
 // the grid, and the owned nodes lie at least `tsteps` inside the held ones
-// wherever those do not end at the grid's edge.  rows: kTileRowsClean for a
-// tile whose held rows and columns, and the row below them, lie clear of the
-// CPML strips and the grid's edge, with vacuum or physical-mode material
-// without the source; else kTileRowsEdge.  Field planes below 4 GiB.
-constexpr int kTileRowsEdge = 4, kTileRowsClean = 8;
+// wherever those do not end at the grid's edge.  rows: kTileRowsTall for a tile
+// of vacuum clear of the CPML strips and the grid's edge (held rows and columns
+// and the row below); kTileRowsClean for vacuum at the strips of one axis, and
+// for physical-mode material clear of them and of the source; else
+// kTileRowsEdge.  The six field planes take less than 2 GiB together.
+constexpr int kTileRowsEdge = 4, kTileRowsClean = 8, kTileRowsTall = 16;
 hipError_t launch_rtile(int mode, int waves, const RegTile* tiles, int ntiles, const LaunchItem* items, const DevSim* sims,
                         int ordinal, int tsteps, hipStream_t st);
 

@@ -113,7 +113,8 @@ namespace {
 // per tile.  T == 0: the launch takes the row sweeps.
 struct TilePlan {
     int T = 0, waves = 0;
-    bool operator==(const TilePlan& o) const { return T == o.T && waves == o.waves; }
+    bool tall = false;  // vacuum tiles of kTileRowsTall rows per wave
+    bool operator==(const TilePlan& o) const { return T == o.T && waves == o.waves && tall == o.tall; }
 };
 
 struct Staging {
@@ -666,23 +667,31 @@ std::vector<Piece> split_axis(int n, int held, int T) {
 
 // Whether the register tiles of `waves` waves hold a simulation's grid.
 bool reg_tiles_fit(const DevSim& d, int waves) {
-    return d.nx + 1 >= 64 && d.ny + 1 >= waves * kTileRowsEdge && (uint64_t)d.ps * 4 < (1ull << 32);
+    return d.nx + 1 >= 64 && d.ny + 1 >= waves * kTileRowsEdge && (uint64_t)d.ps * 24 < (1ull << 31);
 }
 
-// Rows of one band of columns cut into register tiles, bottom to top:
-// waves * kTileRowsClean held rows where those are clean and `light(l, l + held)`
-// says so, else waves * kTileRowsEdge.  add(l, a, b, rows): held from l, owned [a, b).
-template <class Light, class Add>
-void cut_rows(const DevSim& d, int T, int waves, bool xs, Light light, Add add) {
+// Rows of one band of columns cut into register tiles, bottom to top, each the
+// tallest whose held rows the kernel takes at that height (kernels.h).  empty(l,
+// e): rows [l, e) of the band are vacuum; plain(l, e): and without the source in
+// material.  add(l, a, b, rows): held from l, owned [a, b).
+template <class Empty, class Plain, class Add>
+void cut_rows(const DevSim& d, const TilePlan& p, bool xs, Empty empty, Plain plain, Add add) {
     const int ny = d.ny, nc = d.nc;
     for (int a = 0, b; a <= ny; a = b) {
-        int rows = kTileRowsClean, held = waves * rows, l = a ? a - T : 0;
-        if (xs || l <= nc + 1 || l + held > ny - nc || !light(l, l + held)) {
-            rows = kTileRowsEdge;
-            held = waves * rows;
-            l = std::min(l, ny + 1 - held);
+        int rows = 0, held = 0, l = 0;
+        auto try_rows = [&](int r) {
+            rows = r;
+            held = p.waves * r;
+            l = std::min(a ? a - p.T : 0, ny + 1 - held);
+            return l > nc + 1 && l + held <= ny - nc;  // clear of the strips and edge rows
+        };
+        bool inside = p.tall && try_rows(kTileRowsTall);
+        if (!inside || xs || !empty(l, l + held)) {
+            inside = try_rows(kTileRowsClean);
+            const bool clear = inside && !xs, one_axis = l >= 0 && (inside || !xs);
+            if (!(clear && plain(l, l + held)) && !(p.tall && one_axis && empty(l, l + held))) try_rows(kTileRowsEdge);
         }
-        b = l + held > ny ? ny + 1 : l + held - T;
+        b = l + held > ny ? ny + 1 : l + held - p.T;
         add(l, a, b, rows);
     }
 }
@@ -704,10 +713,10 @@ void build_reg_tiles(Slot* sl, int item, const TilePlan& p, std::vector<RegTile>
         };
         // material keeps to the short tiles in reference mode (its incident field
         // makes those rows the costliest) and where the source may lie in it
-        auto light = [&](int r0, int r1) {
+        auto plain = [&](int r0, int r1) {
             return !has_mat(r0, r1) || (phys && !(d.sx >= x.l && d.sx < x.l + 64 && d.sy >= r0 && d.sy < r1));
         };
-        cut_rows(d, p.T, p.waves, x.l <= d.nc || x.l + 64 > d.nx - d.nc, light, [&](int l, int a, int b, int rows) {
+        cut_rows(d, p, x.l <= d.nc || x.l + 64 > d.nx - d.nc, [&](int l, int e) { return !has_mat(l, e); }, plain, [&](int l, int a, int b, int rows) {
             RegTile t{item, sl->idx, x.l, x.a, x.b, l, a, b, rows, 0};
             for (int w = 0; w < p.waves; ++w)
                 if (has_mat(l + w * rows, l + (w + 1) * rows)) t.matmask |= 1 << w;
@@ -720,65 +729,45 @@ void build_reg_tiles(Slot* sl, int item, const TilePlan& p, std::vector<RegTile>
 }
 
 // Shape of the register tiles for a set of simulations under DFT chunks of K
-// steps (T == 0: some grid does not fit one).  The shape does not change
-// results, only time: per launch a fixed part (dispatch, tables, the tile's loads
-// and stores) and per step the larger of the whole launch's work spread over
-// the SIMDs and one tile's own (waves / 4 waves of a SIMD, each a step's
-// instructions and an exchange).  Deep blocks pay the fixed part less often and
-// recompute more ghost cells.  The constants are a fit to 25 launches measured
-// on MI355X (one grid of 257 to 1025 nodes, 64 of 129 and of 513; 8 and 16
-// waves, blocks of 6 to 20 steps): 9% rms, e.g. 725^2 in blocks of 12, 20.6 us
-// with 8 waves and 15.7 with 16 (model 20.8 and 17.5); 64 of 513^2 in blocks of
-// 8, 217 and 219 us (240 and 220).
-TilePlan plan_reg_tiles(const std::vector<Slot*>& ms, int K, int cus) {
-    constexpr double kFixed = 8.0;                 // us per launch
-    constexpr double kEdge = 106, kClean = 61;     // instructions of a wave's step
-    constexpr double kStepLatency = 25, kGHz = 2.3;
-    TilePlan best;
-    double best_t = 1e300;
-    for (int waves : {8, 16}) {
-        bool fit = true;
-        for (const Slot* s : ms) fit = fit && reg_tiles_fit(s->d, waves);
-        if (!fit) continue;
-        const int tmax = std::min(24, (waves * kTileRowsEdge - 8) / 2);
-        for (int m = (K + tmax - 1) / tmax; m <= K; ++m) {
-            const int T = (K + m - 1) / m;
-            if (T < 4 && best.T) break;
-            int64_t edge = 0, clean = 0;
-            const DevSim* last = nullptr;
-            int64_t e1 = 0, c1 = 0;
-            for (const Slot* s : ms) {
-                const DevSim& d = s->d;
-                if (!last || last->nx != d.nx || last->ny != d.ny || last->nc != d.nc) {
-                    e1 = c1 = 0;
-                    const std::vector<Piece> px = split_axis(d.nx + 1, 64, T);
-                    int64_t e[2] = {0, 0}, c[2] = {0, 0};
-                    for (int xs = 0; xs < 2; ++xs)
-                        cut_rows(d, T, waves, xs, [](int, int) { return true; },
-                                 [&](int, int, int, int rows) { rows == kTileRowsClean ? ++c[xs] : ++e[xs]; });
-                    for (const Piece& x : px) {
-                        const bool xs = x.l <= d.nc || x.l + 64 > d.nx - d.nc;
-                        e1 += e[xs];
-                        c1 += c[xs];
-                    }
-                    last = &d;
-                }
-                edge += e1;
-                clean += c1;
-            }
-            const double per_simd = waves * (edge * kEdge + clean * kClean) * 4 / (4.0 * cus);
-            const int64_t slots = (int64_t)(16 / waves) * cus;  // tiles the device holds at once (four waves a SIMD)
-            const double mates = waves == 8 && edge + clean > cus ? kClean : 0;
-            const double lone = edge + clean <= slots ? waves / 4 * (kEdge + mates) * 4 + kStepLatency : 0;
-            const double t = m * (kFixed + T * std::max(per_simd, lone) / (kGHz * 1e3));
-            if (t < best_t) {
-                best_t = t;
-                best.T = T;
-                best.waves = waves;
-            }
-        }
+// steps (T == 0: some grid does not fit one).  It changes no result, only time.
+// A launch pays dispatch, the tiles' loads and stores once, so deep blocks win
+// until their ghost cells outweigh that; tall tiles do fewer loads per owned
+// cell and need enough nodes to fill the device; 16 waves give short grids a
+// whole column of tiles each.  Measured us per step on MI355X (steps x waves,
+// t: tall; chunks of 60 steps):
+//   one 256^2  12x8 1.15, 8x8 1.28, 12x8t 1.32    one 512^2  10x8 1.10, 12x8 1.18, 12x8t 1.32
+//   one 1024^2 12x8t 1.88, 10x8 2.07, 12x16 2.3   one 2048^2 12x8t 3.95, 8x8t 4.39, 8x8 4.88
+//   64 x 128^2 15x16 3.08, 12x16 3.40, 6x8 3.99   8 x 256^2  12x16 1.59, 8x8 1.69, 15x16 1.95
+//   8 x 725^2  12x8t 4.61, 8x8t 5.11, 8x8 5.34    reference 4 x 401^2 6x8 2.08, 10x8t 2.56;
+//   reference 16 x 401^2 10x8t 5.65, 6x8 6.10
+TilePlan plan_reg_tiles(const std::vector<Slot*>& ms, int K) {
+    int64_t nodes = 0;
+    int longest = 0;
+    bool fit8 = true, fit16 = true;
+    for (const Slot* s : ms) {
+        nodes += (int64_t)(s->d.nx + 1) * (s->d.ny + 1);
+        longest = std::max(longest, s->d.ny + 1);
+        fit8 = fit8 && reg_tiles_fit(s->d, 8);
+        fit16 = fit16 && reg_tiles_fit(s->d, 16);
     }
-    return best;
+    TilePlan p;
+    if (!fit8) return p;
+    int deep;
+    if (ms[0]->d.mode != TOMO_MODE_PHYSICAL) {
+        p.waves = 8;
+        p.tall = nodes > 1000000;
+        deep = p.tall ? 10 : 6;
+    } else if (fit16 && ms.size() > 1 && longest <= 300) {
+        p.waves = 16;
+        deep = longest <= 160 ? 15 : 12;
+    } else {
+        p.waves = 8;
+        p.tall = nodes > 500000;
+        deep = p.tall || nodes < 200000 ? 12 : 10;
+    }
+    const int launches = (K + deep - 1) / deep;
+    p.T = (K + launches - 1) / launches;
+    return p;
 }
 
 // The resident launches' error word: 16-byte aligned past the counters.
@@ -898,7 +887,7 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st, bool toge
                 const bool streams_alone = c->form == TOMO_FORM_STREAMS && c->form_set && !together;
                 st.plan = TilePlan{};
                 if (mode != TOMO_MODE_PHYSICAL || (!wave && trs.empty() && !streams_alone))
-                    st.plan = plan_reg_tiles(ms, K, c->cus);
+                    st.plan = plan_reg_tiles(ms, K);
                 if (st.plan.T) {
                     for (size_t i = 0; i < ms.size(); ++i) build_reg_tiles(ms[i], (int)i, st.plan, trg);
                     if (st.fixed && trg.size() * sizeof(RegTile) > st.tiles_cap * sizeof(TileItem)) {
@@ -1150,7 +1139,7 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st, bool toge
                 nl = (maxn + Tb - 1) / Tb;
                 if (c->use_graph && !st.fixed && !resident && !c->prof && minn == K) {
                     const std::vector<int64_t> gk = {mode, T, S, c->Si, W, c->Wi, c->ER, c->form, K, c->grid_mult, ntiles, maxP,
-                                                     fp32_any, fp64_any, (int64_t)ms.size(), plan.T, plan.waves, (int64_t)(intptr_t)d_it,
+                                                     fp32_any, fp64_any, (int64_t)ms.size(), plan.T, plan.waves, plan.tall, (int64_t)(intptr_t)d_it,
                                                      (int64_t)(intptr_t)st.d_tiles, (int64_t)(intptr_t)st.d_sims};
                     if (!c->gexec || gk != c->gkey || key != c->gkey_serials) {
                         if (c->gexec) {

@@ -104,7 +104,7 @@ struct TileItem {
 // and rows [y0, y1) are owned (written back, sampled).
 struct RegTile {
     int item;      // index into the LaunchItem array
-    int sim;       // index into the DevSim table (-1: no tile)
+    int sim;       // index into the DevSim table
     int xl, x0, xe;
     int yl, y0, y1;
     int rows;      // rows per wave

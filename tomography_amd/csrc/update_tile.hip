@@ -19,15 +19,14 @@
 // registers, or with the CPML recursions of its columns and rows.  All of them
 // round as the row sweeps do, so every form gives the same bits.
 //
-// What bounds it: a single grid's launch is 5 us of dispatch, first loads and
-// last stores, and per step one tile's own instruction issue (R rows of the
-// costliest stage on NW / 4 waves of a SIMD) and the LDS exchange; a batch is
-// bound by VALU issue, a fifth to a half of it on ghost cells.  Edge tiles take
-// 4 rows per wave (a corner row in material costs 3 times a vacuum one) and
-// clean ones 8, which also keeps both under the 128 VGPRs of four waves per SIMD.
-// Measured (evaluations, row sweeps -> register tiles): 256^2 9.5 -> 3.3 ms,
-// 725^2 27.2 -> 12.8, 1024^2 39.6 -> 21.5, 64 simulations of 512^2 174 -> 131;
-// the reference's 4 x 401^2 24.5 (resident form) -> 7.0, 16 of them 106 -> 15.4.
+// What bounds it: per launch dispatch (5 us) and the tiles' loads and stores
+// (one step of 64 simulations of 512^2 costs 143 us, each further one 7: 3.5 TB/s
+// of field traffic that little compute overlaps), per step one tile's own
+// instruction issue and the LDS exchange.  So the tallest tiles whose state fits
+// the 128 VGPRs of four waves per SIMD without spilling: 16 rows of vacuum, 8
+// with one axis' CPML psi or with material coefficients, 4 with both (a corner
+// row in material costs 3 times a vacuum one).  Spilled prologues cost more than
+// shorter tiles (16 rows at the strips: 169 -> 270 us).
 #include "device.h"
 #include "kernels.h"
 
@@ -57,6 +56,23 @@ __device__ __forceinline__ float read_lane(float v, int i) {
 // three instructions instead of eleven.
 __device__ __forceinline__ float div_known(float a, double r) { return (float)((double)a * r); }
 
+// Buffer views of one array: the address of an access is base + a per-lane byte
+// offset + a wave-uniform one, so a tile's rows share one lane offset and step
+// in scalar registers, and the hardware drops the lanes whose offset lies past
+// the array (kOff): loads return 0 and stores do nothing, with no branch or
+// execution mask.  Arrays are smaller than 2 GiB.
+typedef __amdgpu_buffer_rsrc_t Buffer;
+constexpr unsigned kOff = 0x80000000u;
+__device__ __forceinline__ Buffer buffer_of(const void* base, size_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes, 0x00027000);
+}
+__device__ __forceinline__ float ld(Buffer b, unsigned lane_off, int off) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(b, lane_off, off, 0));
+}
+__device__ __forceinline__ void st(Buffer b, unsigned lane_off, int off, float v) {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), b, lane_off, off, 0);
+}
+
 // Barrier over the LDS traffic alone: the sample and field stores in flight are
 // not waited for.
 __device__ __forceinline__ void lds_barrier() {
@@ -65,21 +81,24 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// CPML coefficients of a row or a lane.  Off the strips 1/kappa = 1 and
-// a = b = 0, so that strip cells and others take the same instructions; r = 0
-// marks them for the reference's stage.
-struct alignas(16) Profile {
+// CPML coefficients of a row or a lane: the recursion's a and b and k = 1/kappa
+// (in 64 bits for reference-compatible mode, which divides by kappa).  Off the
+// strips a = b = 0 and k = 1, so that strip cells and others take the same
+// instructions; the reference's stage tells them apart by k = 0.
+template <bool REF>
+struct Profile {
+    float a, b, k;
+};
+template <>
+struct Profile<true> {
     float a, b;
-    union {
-        float ik;  // 1/kappa, physical mode
-        double r;  // 1/kappa, reference-compatible mode (which divides by kappa)
-    };
+    double k;
 };
 
-template <int NW>
+template <bool REF, int NW>
 struct TileLds {
     float4 coef[TOMO_MAX_MAT * 2];        // filled when a wave of the tile holds material
-    Profile row_e[NW * kTileRowsEdge], row_h[NW * kTileRowsEdge + 1];  // of E row yl + i and of H row yl - 1 + i
+    Profile<REF> row_e[NW * kTileRowsTall], row_h[NW * kTileRowsTall + 1];  // of E row yl + i and of H row yl - 1 + i
     float ez[2][NW][2][kLane];            // per step parity: each wave's bottom and top Ez row
 };
 
@@ -92,23 +111,23 @@ __device__ __forceinline__ int strip_h(int v, int n, int nc) {
     return (v >= 0 && v < nc) ? nc - 1 - v : ((v >= n - nc && v < n) ? v - n + nc : -1);
 }
 template <bool REF>
-__device__ __forceinline__ Profile profile(float k, float ik, float a, float b, int i) {
-    Profile p;
-    p.a = i < 0 ? 0.f : a;
-    p.b = i < 0 ? 0.f : b;
-    if constexpr (REF) p.r = i < 0 ? 0.0 : 1.0 / (double)k;
-    else p.ik = i < 0 ? 1.f : ik;
+__device__ __forceinline__ Profile<REF> profile(const float* k, const float* ik, const float* a, const float* b, int i) {
+    Profile<REF> p{0.f, 0.f, REF ? 0.f : 1.f};
+    if (i >= 0) {
+        p.a = a[i];
+        p.b = b[i];
+        if constexpr (REF) p.k = 1.0 / (double)k[i];
+        else p.k = ik[i];
+    }
     return p;
 }
 template <bool REF>
-__device__ __forceinline__ Profile profile_e(const DevSim* __restrict__ S, int i) {
-    const int j = max(i, 0);
-    return profile<REF>(S->ke[j], S->ike[j], S->ae[j], S->be[j], i);
+__device__ __forceinline__ Profile<REF> profile_e(const DevSim* __restrict__ S, int i) {
+    return profile<REF>(S->ke, S->ike, S->ae, S->be, i);
 }
 template <bool REF>
-__device__ __forceinline__ Profile profile_h(const DevSim* __restrict__ S, int i) {
-    const int j = max(i, 0);
-    return profile<REF>(S->km[j], S->ikm[j], S->am[j], S->bm[j], i);
+__device__ __forceinline__ Profile<REF> profile_h(const DevSim* __restrict__ S, int i) {
+    return profile<REF>(S->km, S->ikm, S->am, S->bm, i);
 }
 
 // Wave-uniform value that the compiler may not fold into values computed
@@ -125,7 +144,7 @@ __device__ __forceinline__ int opaque(int v) {
 // edge; MAT: some cell is not vacuum; SRC: the source cell is one of the wave's
 // and may lie in material.
 template <int MODE, int R, int NW, bool XS, bool YS, bool MAT, bool SRC>
-__device__ __forceinline__ void tile_wave(const RegTile& tile, const DevSim* __restrict__ Sp, TileLds<NW>& lds,
+__device__ __forceinline__ void tile_wave(const RegTile& tile, const DevSim* __restrict__ Sp, TileLds<MODE == TOMO_MODE_REF_COMPAT, NW>& lds,
                                           int par, int step0, int k0, int nst, int wv, int lane, bool tables, bool frows) {
     constexpr bool REF = MODE == TOMO_MODE_REF_COMPAT;
     const int nx = Sp->nx, ny = Sp->ny, nc = Sp->nc, pitch = Sp->pitch, ps = Sp->ps;
@@ -140,61 +159,59 @@ __device__ __forceinline__ void tile_wave(const RegTile& tile, const DevSim* __r
     auto row_e = [&](int y) { return (unsigned)(hi ? y - (ny - nc) : y - 1) < (unsigned)nc; };
     auto row_h = [&](int y) { return (unsigned)(hi ? y - (ny - nc) : y) < (unsigned)nc; };
     const int re0 = hi ? 2 * nc - ny : -1, rh0 = hi ? 2 * nc - ny : 0;
-    // Scalar plane bases and one 32-bit byte offset per lane and row (the planes
-    // are smaller than 4 GiB).
-    auto at = [](gcfloat* base, unsigned off) { return *(gcfloat*)((GAS const char*)base + off); };
-    auto to = [](gfloat* base, unsigned off, float v) { *(gfloat*)((GAS char*)base + off) = v; };
-    const unsigned o0 = ((unsigned)yb * (unsigned)pitch + (unsigned)x) * 4u, op = (unsigned)pitch * 4u;
+    const Buffer F = buffer_of(Sp->fbase, (size_t)ps * 24), Q = buffer_of(Sp->xbase, (size_t)Sp->xs * 16),
+                 Y = buffer_of(Sp->ybase, (size_t)Sp->ys * 16), Jb = buffer_of(Sp->jbase, (size_t)Sp->js * 8);
+    const unsigned vx = (unsigned)x * 4u;
+    const unsigned ve = XS && je >= 0 ? (unsigned)je * 4u : kOff, vh = XS && jh >= 0 ? (unsigned)jh * 4u : kOff;
+    const int row4 = pitch * 4, plane = ps * 4;  // bytes
+    kcint* span = (kcint*)Sp->span;
+    // lane offset of row y's Jp (compact: one run per row over the dispersive span)
+    auto jp_off = [&](int y) {
+        const int lo = span[3 * y], hi = span[3 * y + 1], off = span[3 * y + 2];
+        return x >= lo && x < hi ? (unsigned)(off - lo + x) * 4u : kOff;
+    };
 
     // ---- the whole tile is requested at once: no row waits for another
     float ez[R], hx[R], hy[R], jp[MAT ? R : 1], phx[XS ? R : 1], pex[XS ? R : 1], phy[YS ? R : 1], pey[YS ? R : 1];
     int mat[MAT ? R : 1];
     float hxb, phyb = 0.f;  // Hx (and its psi) of the row below the wave, which it advances beside its own
-    {
-        gcfloat* fe = (gcfloat*)Sp->fbase + (size_t)par * ps;
-        gcfloat* fx = fe + 2 * (size_t)ps;
-        gcfloat* fy = fe + 4 * (size_t)ps;
-        if constexpr (MAT) {
+    if constexpr (MAT) {
+        const Buffer M = buffer_of(Sp->mat, (size_t)(ny + 1) * pitch);
 #pragma unroll
-            for (int i = 0; i < R; ++i) mat[i] = ((gcu8*)Sp->mat)[(o0 + i * op) >> 2];
-        }
+        for (int i = 0; i < R; ++i) mat[i] = (uint8_t)__builtin_amdgcn_raw_buffer_load_b8(M, (unsigned)x, (yb + i) * pitch, 0);
+    }
+    {
+        const int o = par * plane + yb * row4;
 #pragma unroll
         for (int i = 0; i < R; ++i) {
-            ez[i] = at(fe, o0 + i * op);
-            hx[i] = at(fx, o0 + i * op);
-            hy[i] = at(fy, o0 + i * op);
+            ez[i] = ld(F, vx, o + i * row4);
+            hx[i] = ld(F, vx, o + i * row4 + 2 * plane);
+            hy[i] = ld(F, vx, o + i * row4 + 4 * plane);
         }
-        hxb = at(fx, yb > 0 ? o0 - op : o0);
-        if constexpr (MAT) {
-            kcint* span = (kcint*)Sp->span;
-            gcfloat* jin = (gcfloat*)Sp->jbase + (size_t)par * Sp->js;
+        hxb = ld(F, yb > 0 ? vx : kOff, o - (yb > 0 ? row4 : 0) + 2 * plane);
+    }
+    if constexpr (MAT) {
 #pragma unroll
-            for (int i = 0; i < R; ++i) {
-                const int lo = span[3 * (yb + i)], hi = span[3 * (yb + i) + 1], off = span[3 * (yb + i) + 2];
-                jp[i] = 0.f;
-                if (x >= lo && x < hi) jp[i] = at(jin, (unsigned)(off - lo + x) * 4u);
-            }
-        }
-        if constexpr (XS) {
-            gcfloat* pe = (gcfloat*)Sp->xbase + (size_t)par * Sp->xs;
-            gcfloat* ph = pe + 2 * (size_t)Sp->xs;
-            const unsigned qe = (unsigned)(yb * w2 + max(je, 0)) * 4u, qh = (unsigned)(yb * w2 + max(jh, 0)) * 4u;
+        for (int i = 0; i < R; ++i) jp[i] = ld(Jb, jp_off(yb + i), par * Sp->js * 4);
+    }
+    if constexpr (XS) {
+        const int o = (par * Sp->xs + yb * w2) * 4;
 #pragma unroll
-            for (int i = 0; i < R; ++i) {
-                pex[i] = at(pe, qe + (unsigned)(i * w2) * 4u);
-                phx[i] = at(ph, qh + (unsigned)(i * w2) * 4u);
-            }
+        for (int i = 0; i < R; ++i) {
+            pex[i] = ld(Q, ve, o + i * w2 * 4);
+            phx[i] = ld(Q, vh, o + i * w2 * 4 + Sp->xs * 8);
         }
-        if constexpr (YS) {
-            gcfloat* pe = (gcfloat*)Sp->ybase + (size_t)par * Sp->ys;
-            gcfloat* ph = pe + 2 * (size_t)Sp->ys;
+    }
+    if constexpr (YS) {
+        const int oe = (par * Sp->ys + re0 * pitch) * 4, oh = ((par + 2) * Sp->ys + rh0 * pitch) * 4;
+        // (rows off the strips: the lane offset drops them, the row offset is the array's start)
+        auto psi = [&](bool in, int o, int y) { return ld(Y, in ? vx : kOff, in ? o + y * row4 : 0); };
 #pragma unroll
-            for (int i = 0; i < R; ++i) {
-                pey[i] = at(pe, (unsigned)(min(max(yb + i + re0, 0), w2 - 1) * pitch + x) * 4u);
-                phy[i] = at(ph, (unsigned)(min(max(yb + i + rh0, 0), w2 - 1) * pitch + x) * 4u);
-            }
-            phyb = at(ph, (unsigned)(min(max(yb - 1 + rh0, 0), w2 - 1) * pitch + x) * 4u);
+        for (int i = 0; i < R; ++i) {
+            pey[i] = psi(row_e(yb + i), oe, yb + i);
+            phy[i] = psi(row_h(yb + i), oh, yb + i);
         }
+        phyb = psi(row_h(yb - 1), oh, yb - 1);
     }
     // the tile's tables, while those loads are on their way
     if (tables) {
@@ -215,24 +232,10 @@ __device__ __forceinline__ void tile_wave(const RegTile& tile, const DevSim* __r
     const bool clamp = REF && !(Sp->flags & TOMO_FLAG_NO_NAN_CLAMP);
     const bool ex_ok = !XS || (x >= 1 && x < nx);
     const bool bot = YS && yb == 0, top = YS && yb + R - 1 == ny;  // PEC rows: the wave's first, its last
-    Profile Le, Lh;
+    Profile<REF> Le, Lh;
     if constexpr (XS) {
         Le = profile_e<REF>(Sp, strip_e(x, nx, nc));
         Lh = profile_h<REF>(Sp, strip_h(x, nx, nc));
-#pragma unroll
-        for (int i = 0; i < R; ++i) {
-            pex[i] = je >= 0 ? pex[i] : 0.f;
-            phx[i] = jh >= 0 ? phx[i] : 0.f;
-        }
-    }
-    if constexpr (YS) {
-#pragma unroll
-        for (int i = 0; i < R; ++i) {
-            pey[i] = row_e(yb + i) ? pey[i] : 0.f;
-            phy[i] = row_h(yb + i) ? phy[i] : 0.f;
-        }
-        phyb = row_h(yb - 1) ? phyb : 0.f;
-        hxb = bot ? 0.f : hxb;
     }
     float4 qa[MAT ? R : 1], qb[MAT ? R : 1];
     float f0[MAT && REF ? R : 1];  // the incident field half a step back: each step's new one is the next step's old
@@ -256,7 +259,7 @@ __device__ __forceinline__ void tile_wave(const RegTile& tile, const DevSim* __r
     // ---- contour samples: face rows / columns hold H and Ez, their outer neighbours Ez
     const int D = Sp->D, P = Sp->P, K = Sp->chunk, cx_hi = Sp->cx_hi, cy_lo = Sp->cy_lo;
     const bool own = x >= tile.x0 && x < tile.xe;
-    gfloat* samp = (gfloat*)Sp->samp;
+    const Buffer Z = buffer_of(Sp->samp, (size_t)3 * K * P * 4);
     // rows of the wave that the tile owns: [ra, rb)
     const int ra = max(tile.y0 - yb, 0), rb = min(tile.y1 - yb, R);
     // bits of the owned rows that are face rows and their outer neighbours (lo:
@@ -270,40 +273,39 @@ __device__ __forceinline__ void tile_wave(const RegTile& tile, const DevSim* __r
         const int a = min(max(cy_lo - yb, 0), R), z = min(max(ny - D - yb, 0), R);
         m_x = z > a ? mine & ((1u << z) - 1u) & ~((1u << a) - 1u) : 0;
     }
+    // lane offsets of the samples: plane 0 (H) or, for the outer neighbours, plane 2 (their Ez)
     const bool y_lane = own && x >= D + 1 && x <= cx_hi;
     const bool x_face = x == D || x == nx - D - 1;
-    const bool x_lane = own && (x_face || x == D + 1 || x == nx - D);
-    const int x_dir = x >= nx - D - 1 ? 1 : -1;
-    const unsigned x_off = (unsigned)((x >= nx - D - 1 ? Sp->L1 - cy_lo : Sp->L3 + ny - D - 1) + x_dir * yb) + (x_face ? 0u : 2u * K * P);
+    const bool x_lane = own && (x_face || x == D + 1 || x == nx - D), x_hi = x >= nx - D - 1;
+    const int kp4 = K * P * 4, x_dir = x_hi ? 4 : -4;
+    const unsigned zx0 = x_lane ? (unsigned)((x_hi ? Sp->L1 - cy_lo + yb : Sp->L3 + ny - D - 1 - yb) * 4 + (x_face ? 0 : 2 * kp4)) : kOff;
+    const unsigned zx1 = x_lane && x_face ? zx0 + (unsigned)kp4 : kOff;
     const int L2 = Sp->L2;
     auto sample = [&](int k) {
-        gfloat* sk = samp + (size_t)k * P;
-        const int f = opaque(m_face), o = opaque(m_out), xr = opaque(m_x);
-        if (f | o) {
-            // a wave holds rows of both y legs only on grids of a few rows
-            if (y_lane) {
+        const int o = k * P * 4, f = opaque(m_face), g = opaque(m_out), xr = opaque(m_x);
+        if (f | g) {
 #pragma unroll
-                for (int i = 0; i < R; ++i) {
-                    if (!((f | o) >> i & 1)) continue;  // wave-uniform
-                    const unsigned p = 2 * (yb + i) < ny ? x - D - 1 : L2 + (cx_hi - x);
-                    if (f >> i & 1) {
-                        sk[p] = hx[i];
-                        (sk + (size_t)K * P)[p] = ez[i];
-                    } else {
-                        (sk + 2 * (size_t)K * P)[p] = ez[i];
-                    }
+            for (int i = 0; i < R; ++i) {
+                if (!((f | g) >> i & 1)) continue;  // wave-uniform
+                const unsigned z = !y_lane ? kOff : (unsigned)(2 * (yb + i) < ny ? x - D - 1 : L2 + cx_hi - x) * 4u;
+                if (f >> i & 1) {
+                    st(Z, z, o, hx[i]);
+                    st(Z, z, o + kp4, ez[i]);
+                } else {
+                    st(Z, z, o + 2 * kp4, ez[i]);
                 }
             }
         }
-        if (xr && x_lane) {
-            unsigned p = x_off;
+        if (xr) {
+            unsigned z0 = zx0, z1 = zx1;
 #pragma unroll
             for (int i = 0; i < R; ++i) {
                 if (xr >> i & 1) {  // wave-uniform
-                    sk[p] = x_face ? hy[i] : ez[i];
-                    if (x_face) (sk + (size_t)K * P)[p] = ez[i];
+                    st(Z, z0, o, x_face ? hy[i] : ez[i]);
+                    st(Z, z1, o, ez[i]);
                 }
-                p += x_dir;
+                z0 += x_dir;
+                z1 += x_dir;
             }
         }
     };
@@ -320,22 +322,21 @@ __device__ __forceinline__ void tile_wave(const RegTile& tile, const DevSim* __r
     // Columns x = nx and the row y = ny have no H nodes: their Ez and the Ez
     // beyond them are 0 (next_lane past lane 63, ez_up above the top row), so
     // their H and psi, loaded as 0, stay 0 without a mask.
-    auto h_step = [&](float ez_c, float ez_up, float& hx_, float* hy_, float* phx_, float* phy_, const Profile W) {
+    auto h_step = [&](float ez_c, float ez_up, float& hx_, float* hy_, float* phx_, float* phy_, const Profile<REF> W) {
         const float dEy = ez_up - ez_c;
         float hxn, tx = dEy;
         if constexpr (REF) {
             hxn = hx_ - chx * dEy;
             if constexpr (YS) {
                 const float u = chx * dEy;
-                const float q = hx_ - div_known(u, W.r);
+                const float q = hx_ - div_known(u, W.k);
                 *phy_ = W.b * *phy_ + W.a * dEy;
-                hxn = W.r != 0.0 ? q - chx_d * *phy_ : hxn;
+                hxn = W.k != 0.0 ? q - chx_d * *phy_ : hxn;
             }
-            if (clamp) hxn = __builtin_isnan(hxn) ? 0.f : hxn;
         } else {
             if constexpr (YS) {
                 *phy_ = W.b * *phy_ + W.a * dEy;
-                tx = dEy * W.ik + dyf * *phy_;
+                tx = dEy * W.k + dyf * *phy_;
             }
             hxn = hx_ - chx * tx;
         }
@@ -347,15 +348,14 @@ __device__ __forceinline__ void tile_wave(const RegTile& tile, const DevSim* __r
             hyn = *hy_ + chy * dEx;
             if constexpr (XS) {
                 const float u = chy * dEx;
-                const float q = *hy_ + div_known(u, Lh.r);
+                const float q = *hy_ + div_known(u, Lh.k);
                 *phx_ = Lh.b * *phx_ + Lh.a * dEx;
                 hyn = jh >= 0 ? q + chy_d * *phx_ : hyn;
             }
-            if (clamp) hyn = __builtin_isnan(hyn) ? 0.f : hyn;
         } else {
             if constexpr (XS) {
                 *phx_ = Lh.b * *phx_ + Lh.a * dEx;
-                ty = dEx * Lh.ik + dxf * *phx_;
+                ty = dEx * Lh.k + dxf * *phx_;
             }
             hyn = *hy_ + chy * ty;
         }
@@ -363,7 +363,7 @@ __device__ __forceinline__ void tile_wave(const RegTile& tile, const DevSim* __r
     };
     // E half-step of row i given its new H and the new Hx of the row below;
     // `edge`: a PEC row.
-    auto e_step = [&](int i, float hx_dn, int n, float s, const Profile W, bool edge) {
+    auto e_step = [&](int i, float hx_dn, int n, float s, const Profile<REF> W, bool edge) {
         const float dHy = hy[i] - prev_lane(hy[i]);
         const float dHx = hx[i] - hx_dn;
         const bool eok = ex_ok && !(YS && edge);
@@ -391,29 +391,28 @@ __device__ __forceinline__ void tile_wave(const RegTile& tile, const DevSim* __r
                 const float uy = A.y * dHy, ux = A.y * dHx;
                 if constexpr (XS) {
                     pex[i] = edge ? pex[i] : Le.b * pex[i] + Le.a * dHy;
-                    float b = A.x * e0 + div_known(uy, Le.r);
-                    b = b - div_known(ux, Le.r);
+                    float b = A.x * e0 + div_known(uy, Le.k);
+                    b = b - div_known(ux, Le.k);
                     b = b + A.y * dxf * pex[i];
                     en = je >= 0 ? b : en;
                 }
                 if constexpr (YS) {
                     pey[i] = ex_ok ? W.b * pey[i] + W.a * dHx : pey[i];
-                    float b = A.x * e0 + div_known(uy, W.r);
-                    b = b - div_known(ux, W.r);
+                    float b = A.x * e0 + div_known(uy, W.k);
+                    b = b - div_known(ux, W.k);
                     b = b - A.y * dyf * pey[i];
-                    en = W.r != 0.0 ? b : en;
+                    en = W.k != 0.0 ? b : en;
                 }
             }
-            if (clamp) en = __builtin_isnan(en) ? 0.f : en;
         } else {
             float cy = dHy, cx = dHx;
             if constexpr (XS) {
                 pex[i] = Le.b * pex[i] + Le.a * dHy;
-                cy = dHy * Le.ik + dxf * pex[i];
+                cy = dHy * Le.k + dxf * pex[i];
             }
             if constexpr (YS) {
                 pey[i] = W.b * pey[i] + W.a * dHx;
-                cx = dHx * W.ik + dyf * pey[i];
+                cx = dHx * W.k + dyf * pey[i];
             }
             if constexpr (MAT) {
                 en = A.x * e0 + A.y * cy - A.y * cx - B.x * jp[i];
@@ -434,13 +433,21 @@ __device__ __forceinline__ void tile_wave(const RegTile& tile, const DevSim* __r
         if constexpr (REF && (XS || YS)) en = eok ? en : 0.f;
         ez[i] = en;
     };
-    const Profile* we = lds.row_e + wv * R;      // E row i
-    const Profile* wh = lds.row_h + wv * R + 1;  // H row i
-    auto E = [&](int i) { return YS ? we[i] : Profile{}; };
-    auto H = [&](int i) { return YS ? wh[i] : Profile{}; };
+    const Profile<REF>* we = lds.row_e + wv * R;      // E row i
+    const Profile<REF>* wh = lds.row_h + wv * R + 1;  // H row i
+    auto E = [&](int i) { return YS ? we[i] : Profile<REF>{}; };
+    auto H = [&](int i) { return YS ? wh[i] : Profile<REF>{}; };
     auto hs = [&](int i, float up) {
         h_step(ez[i], up, hx[i], &hy[i], XS ? &phx[XS ? i : 0] : nullptr, YS ? &phy[YS ? i : 0] : nullptr, H(i));
     };
+
+    // The reference's NaN clamp: NaN rows are looked for in pairs of values, and
+    // the values replaced only where one was found (a compare and a select per
+    // value cost a third of the reference's vacuum stage).
+    auto clamp_nan = [&](bool bad, auto fix) {
+        if (clamp && __builtin_amdgcn_ballot_w64(bad)) fix();
+    };
+    auto no_nan = [](float& v) { v = __builtin_isnan(v) ? 0.f : v; };
 
     const int wu = min(wv + 1, NW - 1), wd = max(wv - 1, 0);
     for (int t = 0; t < nst; ++t) {
@@ -448,9 +455,22 @@ __device__ __forceinline__ void tile_wave(const RegTile& tile, const DevSim* __r
         const float s = SRC ? read_lane(sw, t) : 0.f;
         lds.ez[b][wv][0][lane] = ez[0];
         lds.ez[b][wv][1][lane] = ez[R - 1];
-        // what needs no neighbour: H of all rows but the top one, E of the rows in between
+        // what needs no neighbour covers the exchange: H of all rows but the top
+        // one before the barrier, E of the rows in between while the reads return
 #pragma unroll
         for (int i = 0; i + 1 < R; ++i) hs(i, ez[i + 1]);
+        if constexpr (REF) {
+            bool bad = false;
+#pragma unroll
+            for (int i = 0; i + 1 < R; ++i) bad |= __builtin_isunordered(hx[i], hy[i]);
+            clamp_nan(bad, [&] {
+#pragma unroll
+                for (int i = 0; i + 1 < R; ++i) {
+                    no_nan(hx[i]);
+                    no_nan(hy[i]);
+                }
+            });
+        }
         const float ez0 = ez[0];
 #pragma unroll
         for (int i = 1; i + 1 < R; ++i) e_step(i, hx[i - 1], n, s, E(i), false);
@@ -462,8 +482,23 @@ __device__ __forceinline__ void tile_wave(const RegTile& tile, const DevSim* __r
         }
         h_step(ez_dn, ez0, hxb, nullptr, nullptr, &phyb, H(-1));
         hs(R - 1, ez_up);
+        if constexpr (REF)
+            clamp_nan(__builtin_isunordered(hx[R - 1], hy[R - 1]) || __builtin_isnan(hxb), [&] {
+                no_nan(hx[R - 1]);
+                no_nan(hy[R - 1]);
+                no_nan(hxb);
+            });
         e_step(0, hxb, n, s, E(0), bot);
         e_step(R - 1, hx[R - 2], n, s, E(R - 1), top);
+        if constexpr (REF) {
+            bool bad = false;
+#pragma unroll
+            for (int i = 0; i < R; i += 2) bad |= __builtin_isunordered(ez[i], ez[i + 1]);
+            clamp_nan(bad, [&] {
+#pragma unroll
+                for (int i = 0; i < R; ++i) no_nan(ez[i]);
+            });
+        }
         if (extra) {
             if constexpr (!MAT && !REF) {
                 // a source in vacuum: Jp does not see it, so it can be added to the finished row
@@ -481,45 +516,40 @@ __device__ __forceinline__ void tile_wave(const RegTile& tile, const DevSim* __r
 
     // ---- owned cells to the other buffer
     const int keep = opaque(mine);
-    if (!own) return;
-    gfloat* fe = (gfloat*)Sp->fbase + (size_t)(par ^ 1) * ps;
-    gfloat* fx = fe + 2 * (size_t)ps;
-    gfloat* fy = fe + 4 * (size_t)ps;
+    const unsigned wx = own ? vx : kOff, we4 = own ? ve : kOff, wh4 = own ? vh : kOff;
+    const int po = opaque(par ^ 1), yo = opaque(yb);
 #pragma unroll
     for (int i = 0; i < R; ++i) {
         if (!(keep >> i & 1)) continue;  // wave-uniform
-        to(fe, o0 + i * op, ez[i]);
-        to(fx, o0 + i * op, hx[i]);
-        to(fy, o0 + i * op, hy[i]);
-        const int y = yb + i;
-        if constexpr (MAT) {
-            kcint* span = (kcint*)Sp->span;
-            gfloat* jout = (gfloat*)Sp->jbase + (size_t)(par ^ 1) * Sp->js;
-            const int lo = span[3 * y], hi = span[3 * y + 1], off = span[3 * y + 2];
-            if (x >= lo && x < hi) to(jout, (unsigned)(off - lo + x) * 4u, jp[i]);
-        }
+        const int y = yo + i, o = po * plane + y * row4;
+        st(F, wx, o, ez[i]);
+        st(F, wx, o + 2 * plane, hx[i]);
+        st(F, wx, o + 4 * plane, hy[i]);
+        if constexpr (MAT) st(Jb, own ? jp_off(y) : kOff, po * Sp->js * 4, jp[i]);
         if constexpr (XS) {
-            gfloat* pe = (gfloat*)Sp->xbase + (size_t)(par ^ 1) * Sp->xs;
-            gfloat* ph = pe + 2 * (size_t)Sp->xs;
-            if (je >= 0) pe[y * w2 + je] = pex[i];
-            if (jh >= 0) ph[y * w2 + jh] = phx[i];
+            const int q = (po * Sp->xs + y * w2) * 4;
+            st(Q, we4, q, pex[i]);
+            st(Q, wh4, q + Sp->xs * 8, phx[i]);
         }
         if constexpr (YS) {
-            gfloat* pe = (gfloat*)Sp->ybase + (size_t)(par ^ 1) * Sp->ys;
-            gfloat* ph = pe + 2 * (size_t)Sp->ys;
-            if (row_e(y)) pe[(y + re0) * pitch + x] = pey[i];
-            if (row_h(y)) ph[(y + rh0) * pitch + x] = phy[i];
+            if (row_e(y)) st(Y, wx, (po * Sp->ys + (y + re0) * pitch) * 4, pey[i]);
+            if (row_h(y)) st(Y, wx, ((po + 2) * Sp->ys + (y + rh0) * pitch) * 4, phy[i]);
         }
     }
 }
 
+// Workgroups are dealt to the eight XCDs round-robin: XCD g walks the g-th
+// contiguous eighth of the tile list, so that tiles that share halo rows and
+// columns share an L2 (64 simulations of 512^2: 640 -> 237 MB read per launch,
+// 203 -> 193 us; 4 x 401^2 20.2 -> 17.5 us).
 template <int MODE, int NW>
 __global__ __launch_bounds__(NW* kLane) __attribute__((amdgpu_waves_per_eu(4))) void k_rtile(
-    const RegTile* __restrict__ tiles, const LaunchItem* __restrict__ items, const DevSim* __restrict__ sims, int ordinal,
+    const RegTile* __restrict__ tiles, int ntiles, const LaunchItem* __restrict__ items, const DevSim* __restrict__ sims, int ordinal,
     int tsteps) {
-    __shared__ TileLds<NW> lds;
-    const RegTile tile = tiles[blockIdx.x];
-    if (tile.sim < 0) return;
+    __shared__ TileLds<MODE == TOMO_MODE_REF_COMPAT, NW> lds;
+    const int ti = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    if (ti >= ntiles) return;
+    const RegTile tile = tiles[ti];
     const LaunchItem it = items[tile.item];
     const DevSim* Sp = sims + tile.sim;
     const int nst = min(tsteps, it.nsteps - ordinal * tsteps);
@@ -527,32 +557,39 @@ __global__ __launch_bounds__(NW* kLane) __attribute__((amdgpu_waves_per_eu(4))) 
     const int lane = threadIdx.x & (kLane - 1);
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kLane);
     const int par = it.parity0 ^ (ordinal & 1), step0 = it.step0 + ordinal * tsteps, k0 = ordinal * tsteps;
+    const int nx = Sp->nx, ny = Sp->ny, nc = Sp->nc;
+    const int rows = tile.rows, yb = tile.yl + wv * rows;
     const bool mat = (tile.matmask >> wv) & 1;
-#define TW(R, XS, YS, MAT, SRC) \
-    tile_wave<MODE, R, NW, XS, YS, MAT, SRC>(tile, Sp, lds, par, step0, k0, nst, wv, lane, tables, frows)
-    if (tile.rows == kTileRowsClean) {
-        const bool tables = tile.matmask != 0, frows = false;
-        if constexpr (MODE == TOMO_MODE_PHYSICAL) {  // (reference-mode material takes 4-row tiles)
-            if (mat) {
-                TW(kTileRowsClean, false, false, true, false);
-                return;
-            }
-        }
-        TW(kTileRowsClean, false, false, false, false);
-        return;
-    }
-    constexpr int R = kTileRowsEdge;
-    const int nx = Sp->nx, ny = Sp->ny, nc = Sp->nc, yb = tile.yl + wv * R;
     const bool xs = tile.xl <= nc || tile.xl + kLane > nx - nc;  // lanes reach a strip or an edge
-    const bool tys = tile.yl <= nc + 1 || tile.yl + NW * R > ny - nc;
+    const bool tys = tile.yl <= nc + 1 || tile.yl + NW * rows > ny - nc;
     // rows reach a strip or an edge (the row below the wave is advanced too)
-    const bool ys = yb <= nc + 1 || yb + R > ny - nc;
-    const bool tsrc = MODE == TOMO_MODE_PHYSICAL && Sp->sy >= tile.yl && Sp->sy < tile.yl + NW * R &&
+    const bool ys = yb <= nc + 1 || yb + rows > ny - nc;
+    const bool tsrc = MODE == TOMO_MODE_PHYSICAL && Sp->sy >= tile.yl && Sp->sy < tile.yl + NW * rows &&
                       Sp->sx >= tile.xl && Sp->sx < tile.xl + kLane;
-    const bool src = tsrc && mat && Sp->sy >= yb && Sp->sy < yb + R;
+    const bool src = tsrc && mat && Sp->sy >= yb && Sp->sy < yb + rows;
     // row profiles: also where the source lies in material, whose wave takes the general stage
     const bool frows = tys || (tsrc && tile.matmask);
     const bool tables = tile.matmask || frows;
+#define TW(R, XS, YS, MAT, SRC) \
+    tile_wave<MODE, R, NW, XS, YS, MAT, SRC>(tile, Sp, lds, par, step0, k0, nst, wv, lane, tables, frows)
+    if (rows == kTileRowsTall) {
+        TW(kTileRowsTall, false, false, false, false);
+        return;
+    }
+    if (rows == kTileRowsClean) {  // at the strips of one axis at most, material clear of them
+        constexpr int R = kTileRowsClean;
+        if constexpr (MODE == TOMO_MODE_PHYSICAL) {  // (reference-mode material takes 4-row tiles)
+            if (mat) {
+                TW(R, false, false, true, false);
+                return;
+            }
+        }
+        if (xs) TW(R, true, false, false, false);
+        else if (ys) TW(R, false, true, false, false);
+        else TW(R, false, false, false, false);
+        return;
+    }
+    constexpr int R = kTileRowsEdge;
     if (src) TW(R, true, true, true, true);
     else if (mat) {
         if (xs) {
@@ -573,11 +610,11 @@ __global__ __launch_bounds__(NW* kLane) __attribute__((amdgpu_waves_per_eu(4))) 
 hipError_t launch_rtile(int mode, int waves, const RegTile* tiles, int ntiles, const LaunchItem* items, const DevSim* sims,
                         int ordinal, int tsteps, hipStream_t st) {
     if (ntiles <= 0) return hipErrorInvalidValue;
-    dim3 g(ntiles), b(waves * kLane);
-#define TT(MM, WW)                                                                                \
-    if (mode == MM && waves == WW) {                                                              \
-        TIMED_LAUNCH((k_rtile<MM, WW>), g, b, 0, st, tiles, items, sims, ordinal, tsteps);        \
-        return hipGetLastError();                                                                 \
+    dim3 g((ntiles + 7) / 8 * 8), b(waves * kLane);
+#define TT(MM, WW)                                                                            \
+    if (mode == MM && waves == WW) {                                                          \
+        TIMED_LAUNCH((k_rtile<MM, WW>), g, b, 0, st, tiles, ntiles, items, sims, ordinal, tsteps);    \
+        return hipGetLastError();                                                             \
     }
     TT(TOMO_MODE_PHYSICAL, 8) TT(TOMO_MODE_PHYSICAL, 16) TT(TOMO_MODE_REF_COMPAT, 8) TT(TOMO_MODE_REF_COMPAT, 16)
 #undef TT
