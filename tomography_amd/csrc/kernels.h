@@ -85,11 +85,41 @@ hipError_t launch_project_mfma(const int* sim_idx, int n_sims, int n_freq, const
 hipError_t launch_fitness(const float* D, const float* Pph, const float* tgt, const float* tgt_phase, int L,
                           int n_eval, double norm, int terms, double* fit, hipStream_t st);
 
-// Material rasterisation (bit-exact with the oracle).
+// Start state of one simulation, in one launch: copies its tables and its
+// DevSim out of pinned host memory (src: table_bytes, then entry_bytes; both
+// multiples of 8, any of them 0), zeroes [zero, zero + zero_bytes) (a multiple
+// of 16) and, when mat is given, rasterises the phantom `g` of physical mode
+// (bit-exact with the oracle).
+struct SlotInit {
+    const void* src;
+    void* tables;
+    size_t table_bytes;
+    void* entry;
+    size_t entry_bytes;
+    void* zero;
+    size_t zero_bytes;
+    uint8_t* mat;
+    int pitch, nx, ny;
+    float dxf, dyf;
+    PhantomGeom g;
+};
+hipError_t launch_slot_init(const SlotInit& a, hipStream_t st);
+
+// Material map of the reference-compatible mode, from its uploaded tables
+// (bit-exact with the oracle).
 hipError_t launch_raster_ref(uint8_t* mat, int pitch, int nx, int ny, const int* lo, const int* hi,
                              const int* xc, const int* yc, int npatch, hipStream_t st);
-hipError_t launch_raster_phys(uint8_t* mat, int pitch, int nx, int ny, float dxf, float dyf,
-                              const PhantomGeom& g, hipStream_t st);
+
+// Dense copies of the rows [y0, y1) of a simulation's fields, written to
+// pinned host memory: Ez and Jp nx + 1 wide over rows 0..ny, Hx and Hy nx wide
+// over rows 0..ny - 1.  A null `out` skips that field.
+struct FieldPack {
+    const float *ez, *hx, *hy, *jp;  // device planes; jp is the compact row-span storage
+    const int* span;
+    int nx, ny, pitch, y0, y1;
+    float* out[4];  // Ez, Hx, Hy, Jp: destination of row y0
+};
+hipError_t launch_field_pack(const FieldPack& a, hipStream_t st);
 
 // Zero-fill (a kernel, so that it is safe inside captured graphs).
 hipError_t launch_zero(void* p, size_t bytes, hipStream_t st);

@@ -7,7 +7,9 @@
 //   k_project_mfma  far-field projection on the matrix cores
 //               (N2FPostProcess, FDTD_GPU.cu:553-634)
 //   k_fitness   FP64 fitness reduction (FDTD_GPU.cu:1004-1018)
-//   k_raster_*  material map (FDTD_GPU.cu:718-743 / the seeded phantom)
+//   k_slot_init start state, tables and the seeded phantom's material map
+//   k_raster_ref    the reference's material map (FDTD_GPU.cu:718-743)
+//   k_field_pack    dense field copies for the host
 //
 // k_tblock layout: one wave64 owns a band of 64 consecutive Ez columns and
 // sweeps the rows of its tile bottom to top.  The wave keeps T time levels in
@@ -2348,28 +2350,69 @@ __device__ __forceinline__ bool in_ellipse(float X, float Y, const float* e) {
     return q <= 1.0f;
 }
 
-__global__ void k_raster_phys(uint8_t* __restrict__ mat, int pitch, int nx, int ny, float dxf, float dyf,
-                              PhantomGeom g) {
+__device__ __forceinline__ uint8_t phantom_material(int x, int y, int nx, int ny, float dxf, float dyf,
+                                                    const PhantomGeom& g) {
 #pragma clang fp contract(off)
-    const int x = blockIdx.x * blockDim.x + threadIdx.x;
-    const int y = blockIdx.y;
-    if (x >= pitch || y > ny) return;
     uint8_t m = 0;
-    if (x <= nx) {
-        const float X = (float)(x - nx / 2) * dxf;
-        const float Y = (float)(y - ny / 2) * dyf;
-        if (in_circle(X, Y, 0.f, 0.f, g.ro2)) {
-            m = 1;
-            if (in_circle(X, Y, 0.f, 0.f, g.ri2)) {
-                m = 2;
-                for (int e = 0; e < 3; ++e)
-                    if (in_ellipse(X, Y, g.ell[e])) m = 3;
-                for (int k = 0; k < g.ntum; ++k)
-                    if (in_circle(X, Y, g.tum[k][0], g.tum[k][1], g.tum[k][2])) m = (uint8_t)(4 + k);
-            }
+    const float X = (float)(x - nx / 2) * dxf;
+    const float Y = (float)(y - ny / 2) * dyf;
+    if (in_circle(X, Y, 0.f, 0.f, g.ro2)) {
+        m = 1;
+        if (in_circle(X, Y, 0.f, 0.f, g.ri2)) {
+            m = 2;
+            for (int e = 0; e < 3; ++e)
+                if (in_ellipse(X, Y, g.ell[e])) m = 3;
+            for (int k = 0; k < g.ntum; ++k)
+                if (in_circle(X, Y, g.tum[k][0], g.tum[k][1], g.tum[k][2])) m = (uint8_t)(4 + k);
         }
     }
-    mat[(size_t)y * pitch + x] = m;
+    return m;
+}
+
+// One thread per material cell; the same threads first share out the table
+// copy and the zero fill.  Bound by the launch on small grids (one launch in
+// place of two zero fills, a raster launch and four to seven copies from
+// pageable memory: 64 simulations of 128^2 evaluated in 3.3 ms, before in 5.1,
+// the row spans kept per configuration included) and by the zero fill's writes
+// on large ones.
+__global__ void k_slot_init(SlotInit a) {
+    const int x = blockIdx.x * blockDim.x + threadIdx.x;
+    const int y = blockIdx.y;
+    const size_t n = (size_t)gridDim.x * gridDim.y * blockDim.x;
+    const size_t t = (size_t)y * gridDim.x * blockDim.x + x;
+    const size_t nt = a.table_bytes / 8, nc = nt + a.entry_bytes / 8;
+    const uint2* src = (const uint2*)a.src;
+    for (size_t i = t; i < nc; i += n) {
+        const uint2 v = src[i];
+        if (i < nt) ((uint2*)a.tables)[i] = v;
+        else ((uint2*)a.entry)[i - nt] = v;
+    }
+    for (size_t i = t; i < a.zero_bytes / 16; i += n) ((uint4*)a.zero)[i] = make_uint4(0, 0, 0, 0);
+    if (a.mat && x < a.pitch && y <= a.ny)
+        a.mat[(size_t)y * a.pitch + x] =
+            x <= a.nx ? phantom_material(x, y, a.nx, a.ny, a.dxf, a.dyf, a.g) : (uint8_t)0;
+}
+
+// One thread per value of a field row; blockIdx.z is the field.  Bound by the
+// writes to host memory: 42 us for the four fields of a 128^2 grid, launch and
+// wait included, against 2.7 ms for strided copies of the planes, which go row
+// by row.
+__global__ void k_field_pack(FieldPack a) {
+    const int x = blockIdx.x * blockDim.x + threadIdx.x;
+    const int y = a.y0 + blockIdx.y;
+    const int k = blockIdx.z;
+    const bool h = k == 1 || k == 2;
+    const int w = a.nx + (h ? 0 : 1);
+    if (!a.out[k] || x >= w || y >= a.y1 || (h && y >= a.ny)) return;
+    float v;
+    if (k == 3) {
+        const int lo = a.span[3 * y], hi = a.span[3 * y + 1], off = a.span[3 * y + 2];
+        v = x >= lo && x < hi ? a.jp[off + x - lo] : 0.f;
+    } else {
+        const float* f = k == 0 ? a.ez : k == 1 ? a.hx : a.hy;
+        v = f[(size_t)y * a.pitch + x];
+    }
+    a.out[k][(size_t)blockIdx.y * w + x] = v;
 }
 
 __global__ void k_zero(uint4* __restrict__ p, size_t n16) {
@@ -2568,10 +2611,16 @@ hipError_t launch_raster_ref(uint8_t* mat, int pitch, int nx, int ny, const int*
     return hipGetLastError();
 }
 
-hipError_t launch_raster_phys(uint8_t* mat, int pitch, int nx, int ny, float dxf, float dyf, const PhantomGeom& g_,
-                              hipStream_t st) {
-    dim3 g((pitch + 255) / 256, ny + 1), b(256);
-    hipLaunchKernelGGL(k_raster_phys, g, b, 0, st, mat, pitch, nx, ny, dxf, dyf, g_);
+hipError_t launch_slot_init(const SlotInit& a, hipStream_t st) {
+    if ((uintptr_t)a.src % 8 || (uintptr_t)a.tables % 8 || (uintptr_t)a.entry % 8 || (uintptr_t)a.zero % 16 ||
+        a.table_bytes % 8 || a.entry_bytes % 8 || a.zero_bytes % 16)
+        return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_slot_init, dim3((a.pitch + 255) / 256, a.ny + 1), dim3(256), 0, st, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_field_pack(const FieldPack& a, hipStream_t st) {
+    hipLaunchKernelGGL(k_field_pack, dim3((a.nx + 256) / 256, a.y1 - a.y0, 4), dim3(256), 0, st, a);
     return hipGetLastError();
 }
 

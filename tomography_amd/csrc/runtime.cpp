@@ -42,19 +42,7 @@ double now_s() {
 
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// Device buffer freed when it leaves scope (so early error returns leak nothing).
-struct DevMem {
-    void* p = nullptr;
-    DevMem() = default;
-    DevMem(const DevMem&) = delete;
-    DevMem& operator=(const DevMem&) = delete;
-    ~DevMem() {
-        if (p) (void)hipFree(p);
-    }
-    hipError_t alloc(size_t bytes) { return hipMalloc(&p, bytes); }
-    template <class X>
-    X* as() const { return (X*)p; }
-};
+
 
 struct Slot {
     SimSetup su;
@@ -72,7 +60,6 @@ struct Slot {
     // algorithmic bytes per step of the corner, row-edge, column-edge and
     // interior tile classes
     double cls_cells[4] = {0, 0, 0, 0}, cls_bytes[4] = {0, 0, 0, 0};
-    std::vector<float> hpos;  // host copy of the contour positions (source of an async upload)
 };
 
 // Bytes one simulation slot occupies on the device.
@@ -194,6 +181,10 @@ struct tomo_ctx {
     // device memory of destroyed slots, kept for reuse by size
     std::map<size_t, std::vector<char*>> cache;
     size_t cached_bytes = 0;
+    // pinned host memory of kArenaBytes that small uploads and field copies go
+    // through; [0, arena_used) may still be read by work queued on the stream
+    char* arena = nullptr;
+    size_t arena_used = 0;
     // side streams: the three edge-tile kernels run beside the interior one;
     // ev_side[k] marks side stream k's block done, ev_bar all of a block done
     hipStream_t side[3] = {nullptr, nullptr, nullptr};
@@ -294,6 +285,81 @@ void release_cache(tomo_ctx* c) {
     c->cached_bytes = 0;
 }
 
+// Pinned memory for one upload on the context's stream.  The arena is handed
+// out front to back; when it is used up the stream is waited for and it starts
+// over.
+constexpr size_t kArenaBytes = 4u << 20;
+
+int arena_take(tomo_ctx* c, size_t bytes, void** out) {
+    bytes = align256(bytes);
+    if (bytes > kArenaBytes) return fail(TOMO_E_INVALID, "internal: upload larger than the arena");
+    if (c->arena_used + bytes > kArenaBytes) {
+        HIPCHK(hipStreamSynchronize(c->stream));
+        c->arena_used = 0;
+    }
+    *out = c->arena + c->arena_used;
+    c->arena_used += bytes;
+    return TOMO_OK;
+}
+
+// Copy host memory, which may be released on return, to the device.
+int upload(tomo_ctx* c, void* dst, const void* src, size_t bytes) {
+    for (size_t off = 0; off < bytes;) {
+        const size_t n = std::min(bytes - off, kArenaBytes);
+        void* p = nullptr;
+        int rc = arena_take(c, n, &p);
+        if (rc) return rc;
+        std::memcpy(p, (const char*)src + off, n);
+        HIPCHK(hipMemcpyAsync((char*)dst + off, p, n, hipMemcpyHostToDevice, c->stream));
+        off += n;
+    }
+    return TOMO_OK;
+}
+
+// Device memory of one call, from the cache of released memory and returned to
+// it, in stream order like a slot's (an allocation and its release cost a
+// small evaluation about 0.1 ms).  Sizes are powers of two, so that calls of
+// like size find each other's.  It is not charged to `used`.
+struct Work {
+    tomo_ctx* c;
+    char* p = nullptr;
+    size_t bytes = 0;
+    explicit Work(tomo_ctx* c_) : c(c_) {}
+    Work(const Work&) = delete;
+    Work& operator=(const Work&) = delete;
+    int take(size_t need) {
+        size_t b = 64 << 10;
+        while (b < need) b *= 2;
+        auto hit = c->cache.find(b);
+        if (hit != c->cache.end() && !hit->second.empty()) {
+            p = hit->second.back();
+            hit->second.pop_back();
+            c->cached_bytes -= b;
+        } else if (hipMalloc(&p, b) != hipSuccess) {
+            (void)hipGetLastError();
+            release_cache(c);
+            b = need;
+            HIPCHK(hipMalloc(&p, b));
+        }
+        bytes = b;
+        return TOMO_OK;
+    }
+    ~Work() {
+        if (!p) return;
+        c->cache[bytes].push_back(p);
+        c->cached_bytes += bytes;
+        if (c->used + c->cached_bytes > c->budget) release_cache(c);
+    }
+    // The next `n` values of type X (256-byte aligned).
+    size_t at = 0;
+    template <class X>
+    X* carve(size_t n) {
+        X* r = (X*)(p + at);
+        at += align256(n * sizeof(X));
+        return r;
+    }
+};
+
 void slot_destroy(tomo_ctx* c, Slot* s);
 int slot_fill(tomo_ctx* c, Slot* s, DevSim* d_entry);
 
@@ -348,8 +414,7 @@ int slot_create(tomo_ctx* c, const tomo_sim_config& cfg, const double* p, size_t
 
 // Lay out a slot in s->mem (s->bytes), zero its state and accumulators, upload
 // its tables and rasterise its material map, and write its DevSim to d_entry
-// (all on the context's stream; the uploads read host memory owned by the
-// slot, which must outlive them).
+// (all on the context's stream).
 int slot_fill(tomo_ctx* c, Slot* s, DevSim* d_entry) {
     const SimSetup& su = s->su;
     const size_t bytes = s->bytes;
@@ -366,7 +431,6 @@ int slot_fill(tomo_ctx* c, Slot* s, DevSim* d_entry) {
     for (int k = 0; k < 2; ++k) d.phx[k] = (float*)take(rows * 2 * nc * 4);
     for (int k = 0; k < 2; ++k) d.pey[k] = (float*)take(2 * nc * pitch * 4);
     for (int k = 0; k < 2; ++k) d.phy[k] = (float*)take(2 * nc * pitch * 4);
-    char* state_end = m;
     d.fbase = d.ez[0];
     d.ps = (int)(d.ez[1] - d.ez[0]);
     d.jbase = d.jp[0];
@@ -378,16 +442,17 @@ int slot_fill(tomo_ctx* c, Slot* s, DevSim* d_entry) {
     if (d.hx[0] != d.fbase + 2 * (size_t)d.ps || d.hy[1] != d.fbase + 5 * (size_t)d.ps ||
         d.phx[1] != d.xbase + 3 * (size_t)d.xs || d.phy[1] != d.ybase + 3 * (size_t)d.ys)
         return fail(TOMO_E_INVALID, "internal: slot planes are not equally strided");
-    uint8_t* mat = (uint8_t*)take(rows * pitch);
-    int* span = (int*)take(3 * rows * 4);
-    d.samp = (float*)take(3 * (size_t)c->K * P * 4);
-    char* acc0 = m;
     d.accJ = take((size_t)cf.n_freq * P * 16);
     d.accM = take((size_t)cf.n_freq * P * 16);
-    char* acc1 = m;
-    float* srcw = (float*)take((size_t)std::max(cf.steps, 1) * 4);
+    char* zero_end = m;
+    char* tables = m;
+    int* span = (int*)take(3 * rows * 4);
     float* pos = (float*)take(2 * P * 4);
+    float* srcw = (float*)take((size_t)std::max(cf.steps, 1) * 4);
     int* rr = (int*)take((2 * rows + (size_t)cf.nx + 1 + rows) * 4);
+    char* tables_end = m;
+    uint8_t* mat = (uint8_t*)take(rows * pitch);
+    d.samp = (float*)take(3 * (size_t)c->K * P * 4);
     if ((size_t)(m - s->mem) > bytes) return fail(TOMO_E_INVALID, "internal: slot layout overflow");
     d.mat = mat;
     d.span = span;
@@ -414,9 +479,10 @@ int slot_fill(tomo_ctx* c, Slot* s, DevSim* d_entry) {
     // calculate_JandM signs (FDTD_GPU.cu:251-276): yn +, xp +, yp -, xn -
     d.sgn_dt[0] = dtf; d.sgn_dt[1] = dtf; d.sgn_dt[2] = -dtf; d.sgn_dt[3] = -dtf;
 
+    // the tables, as they lie on the device, then the DevSim
     // contour positions (N2FPostProcess geometry, FDTD_GPU.cu:584-621)
-    std::vector<float>& hpos = s->hpos;
-    hpos.resize(2 * P);
+    std::vector<char> host((size_t)(tables_end - tables) + sizeof(DevSim));
+    float* hpos = (float*)(host.data() + ((char*)pos - tables));
     {
         const int D = cf.ntff_offset, nx = cf.nx, ny = cf.ny;
         for (int p = 0; p < (int)P; ++p) {
@@ -439,29 +505,60 @@ int slot_fill(tomo_ctx* c, Slot* s, DevSim* d_entry) {
             hpos[P + p] = (float)py;
         }
     }
-    hipStream_t st = c->stream;
-    // zero the dynamic state and accumulators
-    HIPCHK(launch_zero(s->mem, (size_t)(state_end - s->mem), st));
-    HIPCHK(launch_zero(acc0, (size_t)(acc1 - acc0), st));
-    HIPCHK(hipMemcpyAsync(span, su.span.data(), 3 * rows * 4, hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(pos, hpos.data(), 2 * P * 4, hipMemcpyHostToDevice, st));
+    auto put = [&](const void* at, const void* src, size_t n) {
+        std::memcpy(host.data() + ((const char*)at - tables), src, n);
+    };
+    put(span, su.span.data(), 3 * rows * 4);
+    int *lo = rr, *hi = rr + rows, *xc = rr + 2 * rows, *yc = xc + cf.nx + 1;
     if (cf.mode == TOMO_MODE_PHYSICAL) {
-        HIPCHK(hipMemcpyAsync(srcw, su.srcw.data(), (size_t)cf.steps * 4, hipMemcpyHostToDevice, st));
-        HIPCHK(launch_raster_phys(mat, su.pitch, cf.nx, cf.ny, (float)cf.dx, (float)cf.dy, su.geom, st));
+        put(srcw, su.srcw.data(), (size_t)cf.steps * 4);
     } else {
-        int* lo = rr;
-        int* hi = rr + rows;
-        int* xc = rr + 2 * rows;
-        int* yc = xc + cf.nx + 1;
-        HIPCHK(hipMemcpyAsync(lo, su.ref.lo.data(), rows * 4, hipMemcpyHostToDevice, st));
-        HIPCHK(hipMemcpyAsync(hi, su.ref.hi.data(), rows * 4, hipMemcpyHostToDevice, st));
-        HIPCHK(hipMemcpyAsync(xc, su.ref.xc.data(), ((size_t)cf.nx + 1) * 4, hipMemcpyHostToDevice, st));
-        HIPCHK(hipMemcpyAsync(yc, su.ref.yc.data(), rows * 4, hipMemcpyHostToDevice, st));
-        HIPCHK(launch_raster_ref(mat, su.pitch, cf.nx, cf.ny, lo, hi, xc, yc, cf.numpatches, st));
+        put(lo, su.ref.lo.data(), rows * 4);
+        put(hi, su.ref.hi.data(), rows * 4);
+        put(xc, su.ref.xc.data(), ((size_t)cf.nx + 1) * 4);
+        put(yc, su.ref.yc.data(), rows * 4);
     }
-    HIPCHK(hipMemcpyAsync(d_entry, &s->d, sizeof(DevSim), hipMemcpyHostToDevice, st));
-    // the uploads above read host memory owned by the slot, which outlives them
-    // (slot_destroy waits for the stream before releasing it)
+    static_assert(sizeof(DevSim) % 8 == 0, "copied in 8-byte words");
+    std::memcpy(host.data() + (tables_end - tables), &s->d, sizeof(DevSim));
+    // Through the pinned arena; tables beyond its room go in several launches.
+    SlotInit in{};
+    in.pitch = su.pitch;
+    in.nx = cf.nx;
+    in.ny = cf.ny;
+    size_t off = 0;
+    const size_t ntab = (size_t)(tables_end - tables);
+    while (host.size() - off > kArenaBytes) {
+        const size_t n = std::min(ntab - off, kArenaBytes);
+        void* p = nullptr;
+        int rc = arena_take(c, n, &p);
+        if (rc) return rc;
+        std::memcpy(p, host.data() + off, n);
+        in.src = p;
+        in.tables = tables + off;
+        in.table_bytes = n;
+        HIPCHK(launch_slot_init(in, c->stream));
+        off += n;
+    }
+    void* p = nullptr;
+    int rc = arena_take(c, host.size() - off, &p);
+    if (rc) return rc;
+    std::memcpy(p, host.data() + off, host.size() - off);
+    in.src = p;
+    in.tables = tables + off;
+    in.table_bytes = ntab - off;
+    in.entry = d_entry;
+    in.entry_bytes = sizeof(DevSim);
+    in.zero = s->mem;  // the dynamic state and the accumulators
+    in.zero_bytes = (size_t)(zero_end - s->mem);
+    if (cf.mode == TOMO_MODE_PHYSICAL) {
+        in.mat = mat;
+        in.dxf = (float)cf.dx;
+        in.dyf = (float)cf.dy;
+        in.g = su.geom;
+    }
+    HIPCHK(launch_slot_init(in, c->stream));
+    if (cf.mode != TOMO_MODE_PHYSICAL)
+        HIPCHK(launch_raster_ref(mat, su.pitch, cf.nx, cf.ny, lo, hi, xc, yc, cf.numpatches, c->stream));
     return TOMO_OK;
 }
 
@@ -476,9 +573,6 @@ void slot_destroy(tomo_ctx* c, Slot* s) {
         if (c->used + c->cached_bytes > c->budget) release_cache(c);
     }
     if (s->idx >= 0) c->free_idx.push_back(s->idx);
-    // the host staging in s (span, waveform, positions) may still be read by
-    // queued uploads: wait before releasing it
-    (void)hipStreamSynchronize(c->stream);
     delete s;
 }
 
@@ -1240,39 +1334,40 @@ static int project(tomo_ctx* c, const std::vector<Slot*>& sl, const std::vector<
         }
         groups.push_back({i, 1});
     }
-    // staging: per group the simulation indices and per frequency {k, normaliser}
-    std::vector<int> idx(sl.size());
+    // tables of the launches: the simulation indices, then per group and
+    // frequency {k, normaliser}
+    const size_t ibytes = align256(sl.size() * sizeof(int));
     std::vector<float2> kinv;
     std::vector<size_t> kofs;
-    for (size_t i = 0; i < sl.size(); ++i) idx[i] = sl[i]->idx;
     for (const Group& g : groups) {
         const SimSetup& su = sl[g.i0]->su;
         kofs.push_back(kinv.size());
         for (int f = 0; f < su.cfg.n_freq; ++f)
             kinv.push_back(make_float2((float)(2 * kPI * su.freq[f] / c0()), (float)su.inv_norm[f]));
     }
-    const size_t bytes = align256(idx.size() * sizeof(int)) + kinv.size() * sizeof(float2);
-    char* d = staging;
-    if (d && bytes > staging_cap) return fail(TOMO_E_NOMEM, "projection tables exceed the fixed staging");
-    if (!d) HIPCHK(hipMalloc(&d, bytes));
-    int* d_idx = (int*)d;
-    float2* d_k = (float2*)(d + align256(idx.size() * sizeof(int)));
-    hipError_t e = hipMemcpyAsync(d_idx, idx.data(), idx.size() * sizeof(int), hipMemcpyHostToDevice, c->stream);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(d_k, kinv.data(), kinv.size() * sizeof(float2), hipMemcpyHostToDevice, c->stream);
-    for (size_t gi = 0; gi < groups.size() && e == hipSuccess; ++gi) {
+    std::vector<char> tab(ibytes + kinv.size() * sizeof(float2));
+    for (size_t i = 0; i < sl.size(); ++i) ((int*)tab.data())[i] = sl[i]->idx;
+    std::memcpy(tab.data() + ibytes, kinv.data(), kinv.size() * sizeof(float2));
+    Work w(c);
+    int rc = TOMO_OK;
+    if (staging && tab.size() > staging_cap) return fail(TOMO_E_NOMEM, "projection tables exceed the fixed staging");
+    if (!staging) {
+        rc = w.take(tab.size());
+        if (rc) return rc;
+        staging = w.p;
+    }
+    rc = upload(c, staging, tab.data(), tab.size());
+    if (rc) return rc;
+    const int* d_idx = (const int*)staging;
+    const float2* d_k = (const float2*)(staging + ibytes);
+    for (size_t gi = 0; gi < groups.size(); ++gi) {
         const Group& g = groups[gi];
         const tomo_sim_config& cf = sl[g.i0]->su.cfg;
         LaunchTimer lt(c);
-        e = launch_project_mfma(d_idx + g.i0, (int)g.n, cf.n_freq, d_sims, d_k + kofs[gi], cf.n_angles,
-                                (float)eta0(), dD + out_off[g.i0], dP ? dP + out_off[g.i0] : nullptr, c->stream);
-        if (e == hipSuccess) lt.done(TOMO_KERNEL_PROJECT);
+        HIPCHK(launch_project_mfma(d_idx + g.i0, (int)g.n, cf.n_freq, d_sims, d_k + kofs[gi], cf.n_angles,
+                                   (float)eta0(), dD + out_off[g.i0], dP ? dP + out_off[g.i0] : nullptr, c->stream));
+        lt.done(TOMO_KERNEL_PROJECT);
     }
-    // the uploads read host vectors of this frame
-    const hipError_t es = hipStreamSynchronize(c->stream);
-    if (!staging) (void)hipFree(d);
-    HIPCHK(e);
-    HIPCHK(es);
     return TOMO_OK;
 }
 
@@ -1310,17 +1405,13 @@ static int eval_many(tomo_ctx* c, const tomo_sim_config& cfg, const double* para
         if (rc) return rc;
     }
     const size_t nrec = n_vec * L;
-    DevMem mD, mP, mT, mF;
-    HIPCHK(mD.alloc(nrec * 4 + 256));
-    HIPCHK(mP.alloc(nrec * 4 + 256));
-    HIPCHK(mT.alloc(2 * L * 4 + 256));
-    HIPCHK(mF.alloc(n_vec * 8 + 256));
-    float *dD = mD.as<float>(), *dP = mP.as<float>(), *dT = mT.as<float>();
-    double* dF = mF.as<double>();
-    HIPCHK(hipMemcpyAsync(dT, tgt.data(), L * 4, hipMemcpyHostToDevice, c->stream));
-    if (tph) HIPCHK(hipMemcpyAsync(dT + L, tph, L * 4, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    rc = TOMO_OK;
+    Work w(c);
+    rc = w.take(2 * align256(nrec * 4) + align256(2 * L * 4) + align256(n_vec * 8));
+    if (rc) return rc;
+    float *dD = w.carve<float>(nrec), *dP = w.carve<float>(nrec), *dT = w.carve<float>(2 * L);
+    double* dF = w.carve<double>(n_vec);
+    rc = upload(c, dT, tgt.data(), L * 4);
+    if (!rc && tph) rc = upload(c, dT + L, tph, L * 4);
     if (plain) {
         for (size_t v = 0; v < n_vec && !rc; ++v) {
             for (int e = 0; e < E && !rc; ++e) {
@@ -1381,7 +1472,7 @@ static int eval_many(tomo_ctx* c, const tomo_sim_config& cfg, const double* para
             if (fit_out) fit_out[v] = hf[v];
         }
     }
-    // the copies above completed (or failed) before the buffers are released
+    // the copies above completed (or failed) before the host buffers are released
     (void)hipStreamSynchronize(c->stream);
     return rc;
 }
@@ -1402,17 +1493,19 @@ static int get_target(tomo_ctx* c, const tomo_sim_config& cfg, std::vector<float
         rc = slot_create(c, cfg, tv.data(), tv.size(), e, &s);
         if (!rc) sl.push_back(s);
     }
-    float *dD = nullptr, *dP = nullptr;
-    if (!rc && hipMalloc(&dD, L * 4) != hipSuccess) rc = fail(TOMO_E_HIP, "hipMalloc");
-    if (!rc && hipMalloc(&dP, L * 4) != hipSuccess) rc = fail(TOMO_E_HIP, "hipMalloc");
-    if (!rc) rc = run_and_project(c, sl, dD, dP, true);
+    Work w(c);
+    if (!rc) rc = w.take(2 * align256(L * 4));
     if (!rc) {
-        out.resize(L);
-        if (hipMemcpy(out.data(), dD, L * 4, hipMemcpyDeviceToHost) != hipSuccess) rc = fail(TOMO_E_HIP, "copy");
+        float *dD = w.carve<float>(L), *dP = w.carve<float>(L);
+        rc = run_and_project(c, sl, dD, dP, true);
+        if (!rc) {
+            out.resize(L);
+            if (hipMemcpyAsync(out.data(), dD, L * 4, hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
+                hipStreamSynchronize(c->stream) != hipSuccess)
+                rc = fail(TOMO_E_HIP, "copy");
+        }
     }
     for (Slot* s : sl) slot_destroy(c, s);
-    if (dD) (void)hipFree(dD);
-    if (dP) (void)hipFree(dP);
     if (!rc) c->targets[key] = out;
     return rc;
 }
@@ -1438,28 +1531,22 @@ static int finish_request(tomo_ctx* c, tomo_request* r) {
     int rc = TOMO_OK;
     if (cfg.mode == TOMO_MODE_PHYSICAL) rc = get_target(c, cfg, tgt);
     else rc = fail(TOMO_E_INVALID, "serving needs physical mode");
-    float *dD = nullptr, *dP = nullptr, *dT = nullptr;
-    double* dF = nullptr;
-    if (!rc && (hipMalloc(&dD, L * 4) || hipMalloc(&dP, L * 4) || hipMalloc(&dT, L * 4) || hipMalloc(&dF, 256)))
-        rc = fail(TOMO_E_HIP, "hipMalloc");
+    Work w(c);
+    if (!rc) rc = w.take(3 * align256(L * 4) + 256);
+    double fit = 0;
     if (!rc) {
+        float *dD = w.carve<float>(L), *dP = w.carve<float>(L), *dT = w.carve<float>(L);
+        double* dF = w.carve<double>(1);
         std::vector<int> off;
         for (size_t i = 0; i < r->slots.size(); ++i) off.push_back((int)(i * cfg.n_freq * cfg.n_angles));
         rc = project(c, r->slots, off, dD, dP);
-    }
-    double fit = 0;
-    if (!rc) {
-        if (hipMemcpyAsync(dT, tgt.data(), L * 4, hipMemcpyHostToDevice, c->stream) != hipSuccess ||
-            launch_fitness(dD, dP, dT, nullptr, (int)L, 1, (double)cfg.n_exc * cfg.n_freq, 0, dF, c->stream) !=
-                hipSuccess ||
-            hipMemcpyAsync(&fit, dF, 8, hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
-            hipStreamSynchronize(c->stream) != hipSuccess)
+        if (!rc) rc = upload(c, dT, tgt.data(), L * 4);
+        if (!rc && (launch_fitness(dD, dP, dT, nullptr, (int)L, 1, (double)cfg.n_exc * cfg.n_freq, 0, dF, c->stream) !=
+                        hipSuccess ||
+                    hipMemcpyAsync(&fit, dF, 8, hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
+                    hipStreamSynchronize(c->stream) != hipSuccess))
             rc = fail(TOMO_E_HIP, "fitness");
     }
-    if (dD) (void)hipFree(dD);
-    if (dP) (void)hipFree(dP);
-    if (dT) (void)hipFree(dT);
-    if (dF) (void)hipFree(dF);
     for (Slot* s : r->slots) slot_destroy(c, s);
     r->slots.clear();
     r->fitness = fit;
@@ -1620,19 +1707,21 @@ int eval_noalloc(tomo_ctx* c, char* base, const tomo_sim_config& cfg, const doub
     char* slot_mem = base + slot_off;
     // pageable host staging: a fixed staging waits for the stream before rewriting it
     std::vector<LaunchItem> h_items(kMaxStagedEpochs);
-    std::vector<TileItem> h_tiles((size_t)tiles_cap);
+    // not initialised: only the pages that the tile list covers are ever touched
+    const std::unique_ptr<TileItem[]> h_tiles(new TileItem[(size_t)tiles_cap]);
     Staging st;
     st.fixed = true;
     st.h_items = h_items.data();
     st.d_items = d_items;
     st.items_cap = kMaxStagedEpochs;
-    st.h_tiles = h_tiles.data();
+    st.h_tiles = h_tiles.get();
     st.d_tiles = d_tiles;
     st.tiles_cap = tiles_cap;
     st.d_sims = tbl;
     hipStream_t sm = c->stream;
-    HIPCHK(hipMemcpyAsync(dT, target, L * 4, hipMemcpyHostToDevice, sm));
-    if (tph) HIPCHK(hipMemcpyAsync(dT + L, tph, L * 4, hipMemcpyHostToDevice, sm));
+    rc = upload(c, dT, target, L * 4);
+    if (!rc && tph) rc = upload(c, dT + L, tph, L * 4);
+    if (rc) return rc;
     for (int e = 0; e < E; ++e) {
         Slot* s = slots[e].get();
         s->mem = slot_mem;  // each excitation reuses the slot memory after the previous one's work (stream order)
@@ -1714,6 +1803,7 @@ int tomo_ctx_create(int device, uint64_t hbm_budget, tomo_ctx** out) {
     size_t fr = 0, tot = 0;
     HIPCHK(hipMemGetInfo(&fr, &tot));
     c->budget = hbm_budget ? hbm_budget : (uint64_t)(0.9 * (double)fr);
+    HIPCHK(hipHostMalloc(&c->arena, kArenaBytes, hipHostMallocDefault));
     HIPCHK(hipEventCreateWithFlags(&c->stg.staged, hipEventDisableTiming));
     HIPCHK(hipEventRecord(c->stg.staged, c->stream));
     int rc = ensure_table(c.get(), 256);
@@ -1758,6 +1848,7 @@ int tomo_ctx_destroy(tomo_ctx* c) {
         if (c->side[k]) (void)hipStreamDestroy(c->side[k]);
     }
     if (c->ev_bar) (void)hipEventDestroy(c->ev_bar);
+    if (c->arena) (void)hipHostFree(c->arena);
     for (hipEvent_t e : c->ev_pool) (void)hipEventDestroy(e);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
@@ -2103,21 +2194,27 @@ int tomo_sim_fields(tomo_sim* sim, float* ez, float* hx, float* hy, float* jp) {
     std::lock_guard<std::mutex> g(c->mu);
     const DevSim& d = s->d;
     const int nx = d.nx, ny = d.ny, par = s->parity;
-    hipStream_t st = c->stream;
-    if (ez) HIPCHK(hipMemcpy2DAsync(ez, (nx + 1) * 4, d.ez[par], d.pitch * 4, (nx + 1) * 4, ny + 1, hipMemcpyDeviceToHost, st));
-    if (hx) HIPCHK(hipMemcpy2DAsync(hx, nx * 4, d.hx[par], d.pitch * 4, nx * 4, ny, hipMemcpyDeviceToHost, st));
-    if (hy) HIPCHK(hipMemcpy2DAsync(hy, nx * 4, d.hy[par], d.pitch * 4, nx * 4, ny, hipMemcpyDeviceToHost, st));
-    if (jp) {
-        std::vector<float> cj((size_t)std::max(s->su.jp_len, 1));
-        HIPCHK(hipMemcpyAsync(cj.data(), d.jp[par], cj.size() * 4, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipStreamSynchronize(st));
-        std::fill(jp, jp + (size_t)(nx + 1) * (ny + 1), 0.f);
-        for (int y = 0; y <= ny; ++y) {
-            const int lo = s->su.span[3 * y], hi = s->su.span[3 * y + 1], off = s->su.span[3 * y + 2];
-            for (int x = lo; x < hi; ++x) jp[(size_t)y * (nx + 1) + x] = cj[off + x - lo];
+    (void)hipSetDevice(c->device);
+    float* const dst[4] = {ez, hx, hy, jp};
+    // bands of rows, as many as the arena holds of every field
+    const size_t row = (size_t)(nx + 1) * sizeof(float);
+    const int band = std::max(1, (int)std::min<size_t>((size_t)ny + 1, kArenaBytes / (4 * row)));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    for (int y0 = 0; y0 <= ny; y0 += band) {
+        const int y1 = std::min(ny + 1, y0 + band);
+        FieldPack a{d.ez[par], d.hx[par], d.hy[par], d.jp[par], d.span, nx, ny, d.pitch, y0, y1, {}};
+        for (int k = 0; k < 4; ++k)
+            if (dst[k]) a.out[k] = (float*)(c->arena + k * (size_t)band * row);
+        HIPCHK(launch_field_pack(a, c->stream));
+        HIPCHK(hipStreamSynchronize(c->stream));
+        for (int k = 0; k < 4; ++k) {
+            const bool h = k == 1 || k == 2;
+            const size_t w = (size_t)nx + (h ? 0 : 1);
+            const int ye = h ? std::min(y1, ny) : y1;
+            if (dst[k] && ye > y0) std::memcpy(dst[k] + y0 * w, a.out[k], (ye - y0) * w * sizeof(float));
         }
     }
-    HIPCHK(hipStreamSynchronize(st));
+    c->arena_used = 0;
     return TOMO_OK;
 }
 
@@ -2130,6 +2227,7 @@ int tomo_sim_materials(tomo_sim* sim, uint8_t* mat, float* coef, int* n_mat) {
     }
     std::lock_guard<std::mutex> g(c->mu);
     const DevSim& d = s->d;
+    HIPCHK(hipStreamSynchronize(c->stream));
     if (mat)
         HIPCHK(hipMemcpy2D(mat, d.nx + 1, d.mat, d.pitch, d.nx + 1, d.ny + 1, hipMemcpyDeviceToHost));
     if (coef) std::memcpy(coef, d.coef, sizeof(float) * d.nmat * TOMO_NCOEF);
@@ -2149,6 +2247,7 @@ int tomo_sim_dft(tomo_sim* sim, float* J, float* M) {
     const size_t n = (size_t)d.nfreq * d.P;
     const bool f64 = (d.flags & TOMO_FLAG_DFT_FP64) != 0;
     std::vector<float> a(4 * n), b(4 * n);
+    HIPCHK(hipStreamSynchronize(c->stream));
     HIPCHK(hipMemcpy(a.data(), d.accJ, 16 * n, hipMemcpyDeviceToHost));
     HIPCHK(hipMemcpy(b.data(), d.accM, 16 * n, hipMemcpyDeviceToHost));
     for (size_t i = 0; i < n; ++i) {
@@ -2175,18 +2274,17 @@ int tomo_sim_farfield(tomo_sim* sim, float* D, float* P) {
     }
     std::lock_guard<std::mutex> g(c->mu);
     const size_t L = (size_t)s->su.cfg.n_freq * s->su.cfg.n_angles;
-    float *dD = nullptr, *dP = nullptr;
-    HIPCHK(hipMalloc(&dD, L * 4));
-    HIPCHK(hipMalloc(&dP, L * 4));
+    Work w(c);
+    int rc = w.take(2 * align256(L * 4));
+    if (rc) return rc;
+    float *dD = w.carve<float>(L), *dP = w.carve<float>(L);
     std::vector<Slot*> one{s};
-    int rc = project(c, one, {0}, dD, dP);
-    if (!rc) {
-        if (hipMemcpy(D, dD, L * 4, hipMemcpyDeviceToHost) != hipSuccess) rc = fail(TOMO_E_HIP, "copy");
-        if (!rc && P && hipMemcpy(P, dP, L * 4, hipMemcpyDeviceToHost) != hipSuccess) rc = fail(TOMO_E_HIP, "copy");
-    }
-    (void)hipFree(dD);
-    (void)hipFree(dP);
-    return rc;
+    rc = project(c, one, {0}, dD, dP);
+    if (rc) return rc;
+    HIPCHK(hipMemcpyAsync(D, dD, L * 4, hipMemcpyDeviceToHost, c->stream));
+    if (P) HIPCHK(hipMemcpyAsync(P, dP, L * 4, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    return TOMO_OK;
 }
 
 }  // extern "C"

@@ -428,8 +428,8 @@ static void phys_cpml(const tomo_sim_config& c, SimSetup& s) {
 }
 
 // Products of the configuration alone (shared by every simulation of it):
-// the physical source waveform and its spectrum normaliser, the reference
-// disc extents and patch coordinates.
+// the physical source waveform and its spectrum normaliser, the row spans of
+// the tissue discs, the reference's patch coordinates.
 struct ConfigProducts {
     std::vector<float> srcw;
     double inv_norm[TOMO_MAX_FREQ] = {};
@@ -539,7 +539,6 @@ int build_setup(const tomo_sim_config& c, const double* p, size_t np, int exc, S
         if ((rc = build_phantom(c, p, np, s))) return rc;
         if ((int)s.tissues.size() > TOMO_MAX_MAT) return fail(TOMO_E_INVALID, "too many materials");
         phys_coefs(c, s);
-        physical_spans(c, s);
         phys_cpml(c, s);
         s.chy = (float)(dt / (kMU0 * c.dx));
         s.chx = (float)(dt / (kMU0 * c.dy));
@@ -566,9 +565,16 @@ int build_setup(const tomo_sim_config& c, const double* p, size_t np, int exc, S
                 }
                 cp->inv_norm[f] = 1.0 / (8 * kPI * eta0() * std::norm(S));
             }
+            physical_spans(c, s);
+            cp->span = s.span;
+            cp->mspan = s.mspan;
+            cp->jp_len = s.jp_len;
             cp->has_phys = true;
         }
         s.srcw = cp->srcw;
+        s.span = cp->span;
+        s.mspan = cp->mspan;
+        s.jp_len = cp->jp_len;
         for (int f = 0; f < c.n_freq; ++f) s.inv_norm[f] = cp->inv_norm[f];
         s.tJ = 0.5;
         s.tM = 1.0;
