@@ -74,9 +74,9 @@ hipError_t launch_fold(bool fp64, const LaunchItem* items, int nitems, const Dev
                        hipStream_t st);
 
 // Far-field projection of a group of simulations that share grid, contour and
-// frequencies, on the matrix cores: D/P at [(sim * n_freq + f) * n_angles + a];
+// frequencies: D/P at [(sim * n_freq + f) * n_angles + a];
 // kinv[f] = {wavenumber, far-field normaliser}.
-hipError_t launch_project_mfma(const int* sim_idx, int n_sims, int n_freq, const DevSim* sims, const float2* kinv,
+hipError_t launch_project(const int* sim_idx, int n_sims, int n_freq, const DevSim* sims, const float2* kinv,
                                int n_angles, float eta0, float* D, float* Pph, hipStream_t st);
 
 // FP64 fitness reduction, one block per evaluation:

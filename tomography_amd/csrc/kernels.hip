@@ -4,8 +4,8 @@
 //               E_field_update + calculate_JandM's sampling, FDTD_GPU.cu:231-434)
 //   k_fold      running DFT of one chunk of surface samples (calculate_JandM's
 //               accumulation, FDTD_GPU.cu:231-280), Kahan FP32 or FP64
-//   k_project_mfma  far-field projection on the matrix cores
-//               (N2FPostProcess, FDTD_GPU.cu:553-634)
+//   k_project_mfma, k_project_chain  far-field projection of many / few
+//               simulations (N2FPostProcess, FDTD_GPU.cu:553-634)
 //   k_fitness   FP64 fitness reduction (FDTD_GPU.cu:1004-1018)
 //   k_slot_init start state, tables and the seeded phantom's material map
 //   k_raster_ref    the reference's material map (FDTD_GPU.cu:718-743)
@@ -2164,17 +2164,19 @@ __global__ __launch_bounds__(256) void k_fold(const LaunchItem* __restrict__ ite
 // register r of lane l holds C[8(r/4) + 4(l/32) + r%4][l%32], so a lane ends
 // up holding all four rows of simulations 2q + l/32 (q = r/4) at angle l%32
 // and forms D and the phase without leaving its registers.
-// Few simulations (SPLIT): the four waves share 8 simulations and take one
-// 32-angle tile each, so a lone simulation keeps four waves busy instead of
-// one.  Every output element sees the same products in the same order in
-// both layouts, so the results are identical.
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kProjAngleTiles = 4;                 // 32-angle tiles per workgroup
 constexpr int kProjAngles = 32 * kProjAngleTiles;
 constexpr int kProjChunk = 16;                     // contour points per LDS phase tile
 constexpr int kProjWaves = 4;                      // waves (8 simulations each) per workgroup
 
-template <bool SPLIT>
+// Far field of one angle from its N and L sums.
+__device__ __forceinline__ float2 far_field(float Nr, float Ni, float Lyr, float Lyi, float Lxr, float Lxi, float cph,
+                                            float sph, float eta0) {
+    const float Lr = -sph * Lyr + cph * Lxr, Li = -sph * Lyi + cph * Lxi;
+    return make_float2(Lr + eta0 * Nr, Li + eta0 * Ni);
+}
+
 __global__ __launch_bounds__(64 * kProjWaves) void k_project_mfma(const int* __restrict__ sim_idx, int n_sims,
                                                                   const DevSim* __restrict__ sims,
                                                                   const float2* __restrict__ kinv, int A,
@@ -2183,9 +2185,8 @@ __global__ __launch_bounds__(64 * kProjWaves) void k_project_mfma(const int* __r
     __shared__ float2 wt[2][kProjChunk][kProjAngles];  // phase tiles {cos, sin}, double-buffered
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int a0 = blockIdx.x * kProjAngles, f = blockIdx.z;
-    constexpr int AT = SPLIT ? 1 : kProjAngleTiles;     // 32-angle tiles per wave
-    const int s0 = SPLIT ? blockIdx.y * 8 : (blockIdx.y * kProjWaves + wv) * 8;  // this wave's first simulation
-    const int mt0 = SPLIT ? wv : 0;                      // this wave's first angle tile
+    constexpr int AT = kProjAngleTiles;                  // 32-angle tiles per wave
+    const int s0 = (blockIdx.y * kProjWaves + wv) * 8;   // this wave's first simulation
     const DevSim* G = sims + sim_idx[0];                 // geometry shared by the group
     const int P = G->P, L1 = G->L1, L2 = G->L2, L3 = G->L3, F = G->nfreq;
     const bool fp64 = (G->flags & TOMO_FLAG_DFT_FP64) != 0;
@@ -2257,7 +2258,7 @@ __global__ __launch_bounds__(64 * kProjWaves) void k_project_mfma(const int* __r
         for (int j = 0; j < kProjChunk / 2; ++j) {
 #pragma unroll
             for (int m = 0; m < AT; ++m) {
-                const float2 w = wt[b][2 * j + kh][32 * (mt0 + m) + (lane & 31)];
+                const float2 w = wt[b][2 * j + kh][32 * m + (lane & 31)];
                 cre[m] = __builtin_amdgcn_mfma_f32_32x32x2f32(xr[j], w.x, cre[m], 0, 0, 0);
                 cre[m] = __builtin_amdgcn_mfma_f32_32x32x2f32(-xi[j], w.y, cre[m], 0, 0, 0);
                 cim[m] = __builtin_amdgcn_mfma_f32_32x32x2f32(xr[j], w.y, cim[m], 0, 0, 0);
@@ -2272,7 +2273,7 @@ __global__ __launch_bounds__(64 * kProjWaves) void k_project_mfma(const int* __r
     const float inv = ki.y;
 #pragma unroll
     for (int m = 0; m < AT; ++m) {
-        const int ab = a0 + 32 * (mt0 + m) + (lane & 31);
+        const int ab = a0 + 32 * m + (lane & 31);
         if (ab >= A) continue;
         float cph, sph;
         sincosf(6.283185307179586f * (float)ab / (float)A, &sph, &cph);
@@ -2283,13 +2284,135 @@ __global__ __launch_bounds__(64 * kProjWaves) void k_project_mfma(const int* __r
             const float Nr = cre[m][4 * q], Ni = cim[m][4 * q];
             const float Lyr = cre[m][4 * q + 1], Lyi = cim[m][4 * q + 1];
             const float Lxr = cre[m][4 * q + 2], Lxi = cim[m][4 * q + 2];
-            const float Lr = -sph * Lyr + cph * Lxr, Li = -sph * Lyi + cph * Lxi;
-            const float Er = Lr + eta0 * Nr, Ei = Li + eta0 * Ni;
+            const float2 e = far_field(Nr, Ni, Lyr, Lyi, Lxr, Lxi, cph, sph, eta0);
             const size_t o = ((size_t)s * F + f) * A + ab;
-            D[o] = k * k * (Er * Er + Ei * Ei) * inv;
-            if (Pph) Pph[o] = atan2f(Ei, Er);
+            D[o] = k * k * (e.x * e.x + e.y * e.y) * inv;
+            if (Pph) Pph[o] = atan2f(e.y, e.x);
         }
     }
+}
+
+// The same projection for few simulations, on the vector units.  A matrix
+// product over P contour points is one serial chain per output element, and
+// few simulations fill few of the chain's 32 rows: a lone one takes 3.  The
+// f32 matrix instruction rounds after each of its two products (the same bits
+// as two fmaf over 14 million random sums, subnormal ones included), so
+// multiply-adds in the order of the kernel above give its results: per pair
+// of points (xr wr)_0, (xr wr)_1, (-xi wi)_0, (-xi wi)_1 for the real part,
+// (xr wi)_0, (xr wi)_1, (xi wr)_0, (xi wr)_1 for the imaginary one.  Bound by
+// the phases' sine and cosine and that chain of 2 P multiply-adds, so a
+// workgroup takes only kChainAngles angles (184 workgroups for 8 frequencies
+// of 180 angles): all its waves evaluate the phase tile of kChainPoints
+// points, and wave w runs the chains of simulation w of the group, one per
+// lane: 8 angles x {N, L_y, L_x, spare} x {re, im}.  Measured on 8 frequencies
+// of 180 angles, one simulation (before: four waves sharing the kernel above's
+// 32 rows): 256^2 202 -> 20 us, 512^2 430 -> 37, 1024^2 887 -> 72; 64
+// simulations of 512^2 770 -> 248.
+constexpr int kChainAngles = 8, kChainPoints = 64, kChainSims = 8;  // per workgroup / tile / workgroup
+
+__global__ __launch_bounds__(64 * kChainSims) void k_project_chain(const int* __restrict__ sim_idx, int n_sims,
+                                                                   const DevSim* __restrict__ sims,
+                                                                   const float2* __restrict__ kinv, int A,
+                                                                   float eta0, float* __restrict__ D,
+                                                                   float* __restrict__ Pph) {
+    constexpr int kPairs = kChainPoints / 2;
+    // per pair of points and angle {c0, c1, -s0, -s1, s0, s1, c0, c1}: a lane
+    // reads the half of its part
+    __shared__ __align__(16) float wt[2][kPairs][kChainAngles][8];
+    // per pair of points and row (N, L_y, L_x) {xr0, xr1, xi0, xi1}
+    __shared__ __align__(16) float xt[2][kChainSims][kPairs][3][4];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int a0 = blockIdx.x * kChainAngles, f = blockIdx.z;
+    const int s = blockIdx.y * kChainSims + wv;  // this wave's simulation
+    const DevSim* G = sims + sim_idx[0];         // geometry shared by the group
+    const int P = G->P, L1 = G->L1, L2 = G->L2, L3 = G->L3, F = G->nfreq;
+    const bool fp64 = (G->flags & TOMO_FLAG_DFT_FP64) != 0;
+    const float2 ki = kinv[f];
+    const float k = ki.x;
+    const float dxf = G->dxf, dyf = G->dyf;
+    const float* __restrict__ px = G->pos;
+    const float* __restrict__ py = G->pos + P;
+    const void *accJ = nullptr, *accM = nullptr;
+    if (s < n_sims) {
+        const DevSim* S = sims + sim_idx[s];
+        accJ = S->accJ;
+        accM = S->accM;
+    }
+    // filler: one phase (angle fa, point fp of the tile) and, per wave, one
+    // point's current values of its simulation
+    const int fa = threadIdx.x % kChainAngles, fp = threadIdx.x / kChainAngles;
+    float fc = 0.f, fs = 0.f;
+    sincosf(6.283185307179586f * (float)(a0 + fa) / (float)A, &fs, &fc);
+    float qx, qy, jr, ji, mr, mi;
+    auto load = [&](int c0) {
+        const int p = c0 + fp, q = c0 + lane;
+        qx = qy = jr = ji = mr = mi = 0.f;
+        if (p < P) { qx = px[p]; qy = py[p]; }
+        if (q < P && accJ) {
+            const size_t o = (size_t)f * P + q;
+            if (fp64) {
+                const double2 a = ((const double2*)accJ)[o], b = ((const double2*)accM)[o];
+                jr = (float)a.x; ji = (float)a.y; mr = (float)b.x; mi = (float)b.y;
+            } else {
+                const float2 a = ((const float2*)accJ)[2 * o], b = ((const float2*)accM)[2 * o];
+                jr = a.x; ji = a.y; mr = b.x; mi = b.y;
+            }
+        }
+    };
+    auto fill = [&](int c0, int b) {
+        float sn = 0.f, cs = 0.f;
+        if (c0 + fp < P && a0 + fa < A) sincosf(k * (qx * fc + qy * fs), &sn, &cs);
+        float* w = wt[b][fp >> 1][fa] + (fp & 1);
+        w[0] = cs;
+        w[2] = -sn;
+        w[4] = sn;
+        w[6] = cs;
+        if (s < n_sims) {
+            const int p = c0 + lane;
+            const bool ysf = p < L1 || (p >= L2 && p < L3);
+            const float sj = (ysf ? dxf : dyf) * -1.f, sm = (ysf ? dxf : dyf) * 1.f;
+            float* x = xt[b][wv][lane >> 1][0] + (lane & 1);
+            x[0] = sj * jr;
+            x[2] = sj * ji;
+            x[4] = ysf ? sm * mr : 0.f;
+            x[6] = ysf ? sm * mi : 0.f;
+            x[8] = ysf ? 0.f : sm * mr;
+            x[10] = ysf ? 0.f : sm * mi;
+        }
+    };
+    const int row = min((lane >> 1) & 3, 2), half = lane & 1, an = lane >> 3;
+    float acc = 0.f;
+    load(0);
+    fill(0, 0);
+    for (int c0 = 0, b = 0; c0 < P; c0 += kChainPoints, b ^= 1) {
+        __syncthreads();  // tile b is complete; tile b ^ 1 is no longer read
+        const bool more = c0 + kChainPoints < P;
+        if (more) load(c0 + kChainPoints);
+        if (s < n_sims) {
+#pragma unroll 8
+            for (int j = 0; j < kPairs; ++j) {
+                const float4 w = *(const float4*)(wt[b][j][an] + 4 * half);
+                const float4 x = *(const float4*)xt[b][wv][j][row];
+                acc = fmaf(x.x, w.x, acc);
+                acc = fmaf(x.y, w.y, acc);
+                acc = fmaf(x.z, w.z, acc);
+                acc = fmaf(x.w, w.w, acc);
+            }
+        }
+        if (more) fill(c0 + kChainPoints, b ^ 1);
+    }
+    if (s >= n_sims) return;
+    const int l0 = lane & ~7, ab = a0 + an;
+    const float Nr = __shfl(acc, l0), Ni = __shfl(acc, l0 + 1);
+    const float Lyr = __shfl(acc, l0 + 2), Lyi = __shfl(acc, l0 + 3);
+    const float Lxr = __shfl(acc, l0 + 4), Lxi = __shfl(acc, l0 + 5);
+    if ((lane & 7) || ab >= A) return;
+    float cph, sph;
+    sincosf(6.283185307179586f * (float)ab / (float)A, &sph, &cph);
+    const float2 e = far_field(Nr, Ni, Lyr, Lyi, Lxr, Lxi, cph, sph, eta0);
+    const size_t o = ((size_t)s * F + f) * A + ab;
+    D[o] = k * k * (e.x * e.x + e.y * e.y) * ki.y;
+    if (Pph) Pph[o] = atan2f(e.y, e.x);
 }
 
 // ---------------------------------------------------------------- fitness (FP64)
@@ -2571,13 +2694,22 @@ hipError_t launch_tres(int T, int rows_per_wave, const ResTile* tiles, int ntile
     return hipLaunchCooperativeKernel(f, dim3(ntiles), dim3(kResWaves * kWave), args, 0, st);
 }
 
-hipError_t launch_project_mfma(const int* sim_idx, int n_sims, int n_freq, const DevSim* sims, const float2* kinv,
+hipError_t launch_project(const int* sim_idx, int n_sims, int n_freq, const DevSim* sims, const float2* kinv,
                                int n_angles, float eta0, float* D, float* Pph, hipStream_t st) {
-    const bool split = n_sims < 8 * kProjWaves;
-    const int per_wg = split ? 8 : 8 * kProjWaves;  // simulations per workgroup
-    dim3 g((n_angles + kProjAngles - 1) / kProjAngles, (n_sims + per_wg - 1) / per_wg, n_freq), b(64 * kProjWaves);
-    if (split) TIMED_LAUNCH(k_project_mfma<true>, g, b, 0, st, sim_idx, n_sims, sims, kinv, n_angles, eta0, D, Pph);
-    else TIMED_LAUNCH(k_project_mfma<false>, g, b, 0, st, sim_idx, n_sims, sims, kinv, n_angles, eta0, D, Pph);
+    // Workgroups of either kernel.  Both times grow with the contour; on 512^2
+    // (8 frequencies of 180 angles) a round of up to 256 matrix-core
+    // workgroups takes 760 to 780 us and a vector workgroup 0.16 us of the
+    // device (128 simulations: 488 us against 778; 256: 923 against 783).
+    const int chain = (n_angles + kChainAngles - 1) / kChainAngles * n_freq * ((n_sims + kChainSims - 1) / kChainSims);
+    const int mfma = (n_angles + kProjAngles - 1) / kProjAngles * n_freq * ((n_sims + 8 * kProjWaves - 1) / (8 * kProjWaves));
+    if (chain < 5000 * ((mfma + 255) / 256)) {
+        dim3 g((n_angles + kChainAngles - 1) / kChainAngles, (n_sims + kChainSims - 1) / kChainSims, n_freq);
+        TIMED_LAUNCH(k_project_chain, g, dim3(64 * kChainSims), 0, st, sim_idx, n_sims, sims, kinv, n_angles, eta0, D,
+                     Pph);
+    } else {
+        dim3 g((n_angles + kProjAngles - 1) / kProjAngles, (n_sims + 8 * kProjWaves - 1) / (8 * kProjWaves), n_freq);
+        TIMED_LAUNCH(k_project_mfma, g, dim3(64 * kProjWaves), 0, st, sim_idx, n_sims, sims, kinv, n_angles, eta0, D, Pph);
+    }
     return hipGetLastError();
 }
 

@@ -1305,7 +1305,7 @@ static int check_uniform_precision(const std::vector<Slot*>& sl) {
 // Project the far field of `sl` into D/P (device, [slot][freq][angle] at
 // offset out_off[i]).  Consecutive simulations that share grid, contour,
 // frequencies and angles and whose records are contiguous form one group: one
-// matrix-core launch per group.
+// launch per group.
 // The kernels index `d_sims` (the context's table by default); `staging`, when
 // given, holds the launch's small tables instead of a device allocation.
 static int project(tomo_ctx* c, const std::vector<Slot*>& sl, const std::vector<int>& out_off, float* dD,
@@ -1364,7 +1364,7 @@ static int project(tomo_ctx* c, const std::vector<Slot*>& sl, const std::vector<
         const Group& g = groups[gi];
         const tomo_sim_config& cf = sl[g.i0]->su.cfg;
         LaunchTimer lt(c);
-        HIPCHK(launch_project_mfma(d_idx + g.i0, (int)g.n, cf.n_freq, d_sims, d_k + kofs[gi], cf.n_angles,
+        HIPCHK(launch_project(d_idx + g.i0, (int)g.n, cf.n_freq, d_sims, d_k + kofs[gi], cf.n_angles,
                                    (float)eta0(), dD + out_off[g.i0], dP ? dP + out_off[g.i0] : nullptr, c->stream));
         lt.done(TOMO_KERNEL_PROJECT);
     }
