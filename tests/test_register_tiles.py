@@ -103,3 +103,60 @@ def test_division_by_known_kappa_is_the_division():
         with np.errstate(all="ignore"):
             assert np.array_equal((x[:, None].astype(np.float64) * (1.0 / k.astype(np.float64))).astype(np.float32),
                                   x[:, None] / k)
+
+
+def least_budget(cfg, p):
+    """Smallest memory budget (to 4 KiB) under which the simulation is accepted."""
+    lo, hi = 0, t.request_bytes(cfg) * 2 // 4096
+    while hi - lo > 1:
+        mid = (lo + hi) // 2
+        try:
+            with t.Context(hbm_budget=mid * 4096) as c:
+                c.set_schedule(tsteps=4, chunk=60)
+                c.sim(cfg, p).close()
+            hi = mid
+        except t.TomoError:
+            lo = mid
+    return hi * 4096
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("chunk", [4, 32, 64])
+@pytest.mark.parametrize("name", ["one tile exactly", "wide", "thick CPML", "FP64 running DFT"])
+def test_fold_in_the_next_epoch_equals_its_own_launch(name, chunk):
+    """Evaluations fold an epoch's samples in the next epoch's first launch,
+    stepped simulations in a launch of their own: the same far field, for
+    chunks shorter than the longest block, runs that end in a partial chunk and
+    several simulations together."""
+    cfg, p, exc = CASES[name]
+    cfg = cfg.copy(steps=cfg.steps + 3 * chunk)
+    T = np.zeros(cfg.farfield_len(), np.float32)
+    with t.Context() as c:
+        c.set_schedule(tsteps=4, chunk=chunk, form=t.FORM_FUSED)
+        want = []
+        for e in range(cfg.n_exc):
+            g = c.sim(cfg, p, exc=e)
+            g.step(cfg.steps)
+            want.append(g.farfield()[0].ravel())
+            g.close()
+        want = np.concatenate(want)
+        for many in (1, 3):
+            D = c.eval_batch(cfg, np.tile(p, (many, 1)), target=T, want_farfield=True)[1]
+            assert np.abs(want).max() > 0
+            for d in D:
+                assert np.array_equal(d.ravel(), want)
+
+
+@pytest.mark.gpu
+def test_a_budget_without_room_for_spare_sample_rows():
+    """A budget that just holds the simulation is still enough, and its result
+    is the same."""
+    cfg = wide(nx=200, ny=200, n_exc=1)
+    T = np.zeros(cfg.farfield_len(), np.float32)
+    got = []
+    for budget in (0, least_budget(cfg, PHYS_PARAMS)):
+        with t.Context(hbm_budget=budget) as c:
+            c.set_schedule(tsteps=4, chunk=60)
+            got.append(c.eval_batch(cfg, PHYS_PARAMS, target=T, want_farfield=True)[1])
+    assert np.abs(got[0]).max() > 0
+    assert np.array_equal(*got)

@@ -24,6 +24,7 @@
 #include <type_traits>
 
 #include "device.h"
+#include "fold.h"
 #include "kernels.h"
 
 namespace tomo {
@@ -662,7 +663,7 @@ __global__ __launch_bounds__(512) void k_tblock(const TileItem* __restrict__ til
         S.par = it.parity0 ^ (ordinal & 1);
         S.nx = Sp->nx; S.ny = Sp->ny; S.pitch = Sp->pitch; S.nc = Sp->nc; S.D = Sp->D; S.P = Sp->P;
         S.L1 = Sp->L1; S.L2 = Sp->L2; S.L3 = Sp->L3; S.cx_hi = Sp->cx_hi; S.cy_lo = Sp->cy_lo;
-        S.sx = Sp->sx; S.sy = Sp->sy; S.flags = Sp->flags; S.K = Sp->chunk;
+        S.sx = Sp->sx; S.sy = Sp->sy; S.flags = Sp->flags; S.K = Sp->srows;
         S.chx = Sp->chx; S.chy = Sp->chy; S.chx_d = Sp->chx_d; S.chy_d = Sp->chy_d; S.dxf = Sp->dxf;
         S.dyf = Sp->dyf; S.inc_dt = Sp->inc_dt; S.inc_c = Sp->inc_c; S.inc_ax = Sp->inc_ax;
         S.inc_ay = Sp->inc_ay; S.inc_itau = Sp->inc_itau; S.inc_abs = Sp->inc_abs_origin;
@@ -753,7 +754,7 @@ __device__ __forceinline__ void body_edge(const TileItem& tile, const LaunchItem
     S.par = it.parity0 ^ (ordinal & 1);
     S.nx = Sp->nx; S.ny = Sp->ny; S.pitch = Sp->pitch; S.nc = Sp->nc; S.D = Sp->D; S.P = Sp->P;
     S.L1 = Sp->L1; S.L2 = Sp->L2; S.L3 = Sp->L3; S.cx_hi = Sp->cx_hi; S.cy_lo = Sp->cy_lo;
-    S.sx = Sp->sx; S.sy = Sp->sy; S.flags = Sp->flags; S.K = Sp->chunk;
+    S.sx = Sp->sx; S.sy = Sp->sy; S.flags = Sp->flags; S.K = Sp->srows;
     S.chx = Sp->chx; S.chy = Sp->chy; S.dxf = Sp->dxf; S.dyf = Sp->dyf;
     const int nx = S.nx, ny = S.ny, nc = S.nc;
     const int bx = tile.x0 + wv * V;
@@ -1023,7 +1024,7 @@ __global__ __launch_bounds__(kResWaves * kWave, 1) void k_tres(const ResTile* __
     S.ps = Sp->ps; S.js = Sp->js; S.xs = Sp->xs; S.ys = Sp->ys;
     S.nx = Sp->nx; S.ny = Sp->ny; S.pitch = Sp->pitch; S.nc = Sp->nc; S.D = Sp->D; S.P = Sp->P;
     S.L1 = Sp->L1; S.L2 = Sp->L2; S.L3 = Sp->L3; S.cx_hi = Sp->cx_hi; S.cy_lo = Sp->cy_lo;
-    S.sx = Sp->sx; S.sy = Sp->sy; S.flags = Sp->flags; S.K = Sp->chunk;
+    S.sx = Sp->sx; S.sy = Sp->sy; S.flags = Sp->flags; S.K = Sp->srows;
     S.chx = Sp->chx; S.chy = Sp->chy; S.dxf = Sp->dxf; S.dyf = Sp->dyf;
     const int nx = S.nx, ny = S.ny, nc = S.nc, D = S.D;
     const int x0 = tile.x0 - T;  // first lane's column
@@ -1257,7 +1258,7 @@ __global__ __launch_bounds__(kTileWaves * kWave) __attribute__((amdgpu_waves_per
         S.par = it.parity0 ^ (ordinal & 1);
         S.nx = Sp->nx; S.ny = Sp->ny; S.pitch = Sp->pitch; S.nc = Sp->nc; S.D = Sp->D; S.P = Sp->P;
         S.L1 = Sp->L1; S.L2 = Sp->L2; S.L3 = Sp->L3; S.cx_hi = Sp->cx_hi; S.cy_lo = Sp->cy_lo;
-        S.sx = Sp->sx; S.sy = Sp->sy; S.flags = Sp->flags; S.K = Sp->chunk;
+        S.sx = Sp->sx; S.sy = Sp->sy; S.flags = Sp->flags; S.K = Sp->srows;
         S.chx = Sp->chx; S.chy = Sp->chy; S.chx_d = Sp->chx_d; S.chy_d = Sp->chy_d; S.dxf = Sp->dxf;
         S.dyf = Sp->dyf;
         const int nx = S.nx, ny = S.ny, nc = S.nc, D = S.D;
@@ -1433,7 +1434,7 @@ __device__ __forceinline__ void body_row(const TileItem& tile, const LaunchItem&
     const bool wsrc = (sx >= x0 && sx <= x0 + kWave - 1);
     kcfloat* srcw = (kcfloat*)Sp->srcw;
     // y-face NTFF rows (FDTD_common.cxx:4-46 legs yn, yp)
-    const int D = Sp->D, P = Sp->P, K = Sp->chunk, L2 = Sp->L2, cx_hi = Sp->cx_hi;
+    const int D = Sp->D, P = Sp->P, K = Sp->srows, L2 = Sp->L2, cx_hi = Sp->cx_hi;
     const bool xr = (x >= D + 1 && x <= cx_hi);
     gfloat* samp = (gfloat*)Sp->samp;
     const int y0 = tile.y0, y1 = tile.y1;
@@ -1686,7 +1687,7 @@ __device__ __forceinline__ void body_col(const TileItem& tile, const LaunchItem&
     const float axh = lcx[4 * TOMO_MAX_NC + ixh], bxh = lcx[5 * TOMO_MAX_NC + ixh];
     const bool hok = (x >= 0 && x < nx), eok = (x >= 1 && x <= nx - 1);
     // x-face NTFF contour columns (FDTD_common.cxx:4-46 legs xp, xn)
-    const int D = Sp->D, ny = Sp->ny, P = Sp->P, K = Sp->chunk;
+    const int D = Sp->D, ny = Sp->ny, P = Sp->P, K = Sp->srows;
     const bool ccol = (x == nx - D - 1 || x == nx - D || x == D || x == D + 1);
     const bool wcc = (x0 <= D + 1 && x0 + kWave - 1 >= D) || (x0 <= nx - D && x0 + kWave - 1 >= nx - D - 1);
     gfloat* samp = (gfloat*)Sp->samp;
@@ -2018,130 +2019,24 @@ __global__ __launch_bounds__(256, kFusedWgPerCu<T>) void k_tfused(const TileItem
 }
 
 // ---------------------------------------------------------------- running DFT fold
-// Phase e^{-j w (step + t0) dt}: evaluated in FP64 for every step of the chunk
-// (<= 64 steps) into an LDS table and rounded once to FP32; the chunk is summed
-// in FP32 and added to the long-running accumulator with Kahan compensation.
-// Block (x, item, z) folds contour points [256 x, 256 x + 256) of one item
-// for frequencies [z fpb, z fpb + fpb), kFoldGroup at a time.  Few items
-// (one simulation) take fpb = kFoldGroup = 1, so the frequencies spread over
-// more blocks; many items take fpb = all frequencies with kFoldGroup = 8, so
-// each sample is read once per 8 frequencies.  Every frequency's sum runs in
-// the same order either way.
+// One launch's share: block (x, item, z) folds contour points [256 x, 256 x +
+// 256) of one item for frequencies [z fpb, z fpb + fpb), kFoldGroup at a time
+// (fold.h; items of the other precision are skipped).
 template <bool FP64, int kFoldGroup>
 __global__ __launch_bounds__(256) void k_fold(const LaunchItem* __restrict__ items,
                                               const DevSim* __restrict__ sims, int fpb) {
     const LaunchItem it = items[blockIdx.y];
     const DevSim* S = sims + it.sim;
-    const int P = S->P, K = S->chunk;
-    const int fb = blockIdx.z * fpb, F = min(S->nfreq, fb + fpb);
-    const int nk = min(it.nsteps, K);
-    if (nk <= 0 || fb >= F || ((S->flags & TOMO_FLAG_DFT_FP64) != 0) != FP64) return;
-    const int nf = F - fb;
-    __shared__ float2 wJ[FP64 ? 1 : TOMO_MAX_FREQ * 64];
-    __shared__ float2 wM[FP64 ? 1 : TOMO_MAX_FREQ * 64];
-    __shared__ double2 dJ[FP64 ? TOMO_MAX_FREQ * 64 : 1];
-    __shared__ double2 dRot[FP64 ? TOMO_MAX_FREQ : 1];
-    if (!FP64) {
-        // every phase of the chunk evaluated in FP64 and rounded once to FP32
-        // (a rotation recurrence would drift by an ulp per step)
-        for (int i = threadIdx.x; i < 2 * nf * nk; i += blockDim.x) {
-            const int which = i / (nf * nk), f = fb + (i / nk) % nf, k = i % nk;
-            double s0, c0;
-            sincos(-S->wdt[f] * ((double)it.step0 + k + (which ? S->tM : S->tJ)), &s0, &c0);
-            (which ? wM : wJ)[f * 64 + k] = make_float2((float)c0, (float)s0);
-        }
-    } else {
-        // FP64 study mode: exact phases; the M phase is the J phase rotated by
-        // -w (tM - tJ).
-        for (int i = threadIdx.x; i < nf * nk; i += blockDim.x) {
-            const int f = fb + i / nk, k = i % nk;
-            double s, c;
-            sincos(-S->wdt[f] * ((double)it.step0 + k + S->tJ), &s, &c);
-            dJ[f * 64 + k] = make_double2(c, s);
-        }
-        if (threadIdx.x < nf) {
-            double s, c;
-            sincos(-S->wdt[fb + threadIdx.x] * (S->tM - S->tJ), &s, &c);
-            dRot[fb + threadIdx.x] = make_double2(c, s);
-        }
-    }
-    __syncthreads();
+    const int fb = blockIdx.z * fpb, nf = min(S->nfreq, fb + fpb) - fb;
+    const int nk = min(it.nsteps, S->chunk);
+    if (nk <= 0 || nf <= 0 || ((S->flags & TOMO_FLAG_DFT_FP64) != 0) != FP64) return;
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= P) return;
-    const int leg = p < S->L1 ? 0 : (p < S->L2 ? 1 : (p < S->L3 ? 2 : 3));
-    const float sdt = S->sgn_dt[leg];
-    // global-address-space views (flat loads would also count against the LDS
-    // counter, so every phase-table wait would drain the sample loads)
-    gcfloat* hs = (gcfloat*)S->samp + p;
-    gcfloat* e0 = (gcfloat*)S->samp + (size_t)K * P + p;
-    gcfloat* e1 = (gcfloat*)S->samp + (size_t)2 * K * P + p;
-    // Frequencies in groups of kFoldGroup: each sample is read once per group
-    // (coalesced over p) and multiplied into every frequency of the group.
-    for (int f0 = fb; f0 < F; f0 += kFoldGroup) {
-        if (!FP64) {
-            float jr[kFoldGroup], ji[kFoldGroup], mr[kFoldGroup], mi[kFoldGroup];
-#pragma unroll
-            for (int q = 0; q < kFoldGroup; ++q) jr[q] = ji[q] = mr[q] = mi[q] = 0.f;
-            // unrolled so that several steps' samples are in flight at once
-            // (the accumulation order is unchanged); one frequency per thread
-            // leaves the registers for 20 steps' loads
-#pragma unroll (kFoldGroup == 1 ? 20 : 8)
-            for (int k = 0; k < nk; ++k) {
-                const float h = hs[(size_t)k * P];
-                const float e = (e0[(size_t)k * P] + e1[(size_t)k * P]) / 2;
-#pragma unroll
-                for (int q = 0; q < kFoldGroup; ++q) {
-                    const float2 a = wJ[(f0 + q) * 64 + k], b = wM[(f0 + q) * 64 + k];
-                    jr[q] += h * a.x;
-                    ji[q] += h * a.y;
-                    mr[q] += e * b.x;
-                    mi[q] += e * b.y;
-                }
-            }
-#pragma unroll
-            for (int q = 0; q < kFoldGroup; ++q) {
-                if (f0 + q >= F) break;
-                float4* aJ = (float4*)S->accJ + (size_t)(f0 + q) * P + p;
-                float4* aM = (float4*)S->accM + (size_t)(f0 + q) * P + p;
-                float4 vJ = *aJ, vM = *aM;
-                // Kahan: value (x, y), compensation (z, w)
-                float yv, tv;
-                yv = sdt * jr[q] - vJ.z; tv = vJ.x + yv; vJ.z = (tv - vJ.x) - yv; vJ.x = tv;
-                yv = sdt * ji[q] - vJ.w; tv = vJ.y + yv; vJ.w = (tv - vJ.y) - yv; vJ.y = tv;
-                yv = sdt * mr[q] - vM.z; tv = vM.x + yv; vM.z = (tv - vM.x) - yv; vM.x = tv;
-                yv = sdt * mi[q] - vM.w; tv = vM.y + yv; vM.w = (tv - vM.y) - yv; vM.y = tv;
-                *aJ = vJ;
-                *aM = vM;
-            }
-        } else {
-            double jr[kFoldGroup], ji[kFoldGroup], mr[kFoldGroup], mi[kFoldGroup];
-#pragma unroll
-            for (int q = 0; q < kFoldGroup; ++q) jr[q] = ji[q] = mr[q] = mi[q] = 0.0;
-#pragma unroll 8
-            for (int k = 0; k < nk; ++k) {
-                const double h = hs[(size_t)k * P];
-                const double e = 0.5 * ((double)e0[(size_t)k * P] + (double)e1[(size_t)k * P]);
-#pragma unroll
-                for (int q = 0; q < kFoldGroup; ++q) {
-                    const double2 a = dJ[(f0 + q) * 64 + k], r = dRot[f0 + q];
-                    const double2 b = make_double2(a.x * r.x - a.y * r.y, a.x * r.y + a.y * r.x);
-                    jr[q] += h * a.x;
-                    ji[q] += h * a.y;
-                    mr[q] += e * b.x;
-                    mi[q] += e * b.y;
-                }
-            }
-#pragma unroll
-            for (int q = 0; q < kFoldGroup; ++q) {
-                if (f0 + q >= F) break;
-                double2* aJ = (double2*)S->accJ + (size_t)(f0 + q) * P + p;
-                double2* aM = (double2*)S->accM + (size_t)(f0 + q) * P + p;
-                double2 vJ = *aJ, vM = *aM;
-                vJ.x += sdt * jr[q]; vJ.y += sdt * ji[q]; vM.x += sdt * mr[q]; vM.y += sdt * mi[q];
-                *aJ = vJ;
-                *aM = vM;
-            }
-        }
+    if constexpr (!FP64) {
+        __shared__ float2 wJ[TOMO_MAX_FREQ * 64], wM[TOMO_MAX_FREQ * 64];
+        fold_fp32<kFoldGroup>(S, it, nk, fb, nf, p, wJ, wM);
+    } else {
+        __shared__ double2 dJ[TOMO_MAX_FREQ * 64], dRot[TOMO_MAX_FREQ];
+        fold_fp64<kFoldGroup>(S, it, nk, fb, nf, p, dJ, dRot);
     }
 }
 

@@ -49,6 +49,7 @@ struct Slot {
     DevSim d{};
     char* mem = nullptr;
     size_t bytes = 0;
+    int srows = 0;      // sample rows
     int idx = -1;       // DevSim table index
     int done = 0;       // steps completed
     int parity = 0;     // buffer holding the current state
@@ -62,8 +63,12 @@ struct Slot {
     double cls_cells[4] = {0, 0, 0, 0}, cls_bytes[4] = {0, 0, 0, 0};
 };
 
-// Bytes one simulation slot occupies on the device.
-size_t slot_bytes(const SimSetup& s, int chunk) {
+// Sample rows beyond a chunk: the longest block of the register tiles, which
+// writes them while the chunk's own rows are folded (run_epochs).
+constexpr int kRoundRows = 24;
+
+// Bytes one simulation slot with `srows` sample rows occupies on the device.
+size_t slot_bytes(const SimSetup& s, int srows) {
     const tomo_sim_config& c = s.cfg;
     const size_t rows = (size_t)c.ny + 1, pitch = s.pitch, nc = c.ncpml, P = s.P;
     size_t b = 0;
@@ -73,7 +78,7 @@ size_t slot_bytes(const SimSetup& s, int chunk) {
     b += 4 * align256(2 * nc * pitch * 4);                    // pey, phy x2
     b += align256(rows * pitch);                              // mat
     b += align256(3 * rows * 4);                              // span
-    b += align256(3 * (size_t)chunk * P * 4);                 // samples
+    b += align256(3 * (size_t)srows * P * 4);                 // samples
     b += 2 * align256((size_t)c.n_freq * P * 16);             // accJ, accM
     b += align256((size_t)std::max(c.steps, 1) * 4);          // source waveform
     b += align256(2 * P * 4);                                 // contour positions
@@ -364,13 +369,19 @@ void slot_destroy(tomo_ctx* c, Slot* s);
 int slot_fill(tomo_ctx* c, Slot* s, DevSim* d_entry);
 
 // Build the device-resident simulation for one excitation of one phantom.
-int slot_create(tomo_ctx* c, const tomo_sim_config& cfg, const double* p, size_t np, int exc, Slot** out) {
+// together > 0: it is the first of that many alike that an evaluation creates
+// and runs within one call; they take spare sample rows where the budget
+// admits all of them with these, so that the rows refuse nothing.  Simulations
+// that outlive a call, or advance an epoch per call, have no use for them.
+int slot_create(tomo_ctx* c, const tomo_sim_config& cfg, const double* p, size_t np, int exc, int together, Slot** out) {
     std::unique_ptr<Slot> s(new Slot());
     int rc = build_setup(cfg, p, np, exc, s->su);
     if (rc) return rc;
     const SimSetup& su = s->su;
     if (c->K % c->T) return fail(TOMO_E_INVALID, "chunk must be a multiple of the fused step count");
-    const size_t bytes = slot_bytes(su, c->K);
+    s->srows = c->K;
+    if (together > 0 && c->used + together * slot_bytes(su, c->K + kRoundRows) <= c->budget) s->srows += kRoundRows;
+    const size_t bytes = slot_bytes(su, s->srows);
     if (c->used + bytes > c->budget) return fail(TOMO_E_NOMEM, "HBM budget exceeded");
     auto hit = c->cache.find(bytes);
     if (hit != c->cache.end() && !hit->second.empty()) {
@@ -452,7 +463,7 @@ int slot_fill(tomo_ctx* c, Slot* s, DevSim* d_entry) {
     int* rr = (int*)take((2 * rows + (size_t)cf.nx + 1 + rows) * 4);
     char* tables_end = m;
     uint8_t* mat = (uint8_t*)take(rows * pitch);
-    d.samp = (float*)take(3 * (size_t)c->K * P * 4);
+    d.samp = (float*)take(3 * (size_t)s->srows * P * 4);
     if ((size_t)(m - s->mem) > bytes) return fail(TOMO_E_INVALID, "internal: slot layout overflow");
     d.mat = mat;
     d.span = span;
@@ -462,7 +473,7 @@ int slot_fill(tomo_ctx* c, Slot* s, DevSim* d_entry) {
     d.D = cf.ntff_offset; d.P = su.P; d.L1 = su.L1; d.L2 = su.L2; d.L3 = su.L3;
     d.cx_hi = su.cx_hi; d.cy_lo = su.cy_lo;
     d.sx = su.sx; d.sy = su.sy; d.mode = cf.mode; d.flags = cf.flags;
-    d.nmat = su.nmat; d.nfreq = cf.n_freq; d.chunk = c->K; d.steps = cf.steps;
+    d.nmat = su.nmat; d.nfreq = cf.n_freq; d.chunk = c->K; d.steps = cf.steps; d.srows = s->srows;
     std::memcpy(d.coef, su.coef, sizeof(d.coef));
     for (int i = 0; i < TOMO_MAX_NC; ++i) {
         d.ike[i] = su.ike[i]; d.ae[i] = su.ae[i]; d.be[i] = su.be[i];
@@ -1019,6 +1030,15 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st, bool toge
             // the host staging is rewritten below: wait for its last upload
             if (st.staged) HIPCHK(hipEventSynchronize(st.staged));
             else HIPCHK(hipStreamSynchronize(c->stream));
+            // An epoch's samples are folded by further workgroups of the next
+            // epoch's first launch, which writes the sample rows after them, so
+            // only the last staged epoch's fold is a launch of its own (each takes 7
+            // to 8 us; 1024^2 in 60-step epochs 16.6 ms per evaluation -> 15.5,
+            // 363^2 in 32-step ones 8.1 -> 6.6, 64 of 512^2 90.5 -> 88.3).  Captured
+            // epochs stay whole, and simulations without the spare rows or in FP64
+            // fold by themselves.
+            bool around = rtile && !fp64_any && E > 1 && Tb <= kRoundRows && Tb <= K;
+            for (Slot* s : ms) around = around && s->srows >= K + Tb;
             int maxP = 0, maxF = 0;
             for (int i = 0; i < nsim; ++i) {
                 Slot* s = ms[i];
@@ -1028,6 +1048,7 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st, bool toge
                     it.step0 = s->done + e * K;
                     it.parity0 = s->parity ^ ((e * ((K + Tb - 1) / Tb)) & 1);  // epochs before the last are full
                     it.nsteps = std::min(K, s->target - s->done - e * K);
+                    it.samp0 = around ? (int)((int64_t)e * K % s->srows) : 0;
                 }
                 maxP = std::max(maxP, s->d.P);
                 maxF = std::max(maxF, s->d.nfreq);
@@ -1072,6 +1093,8 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st, bool toge
             const LaunchItem* h_it = st.h_items;
             LaunchItem* d_it = st.d_items;
             int nl = 0;  // time blocks of that epoch
+            FoldRun before{};         // the previous epoch, folded by this one's first launch
+            bool fold_after = true;  // this epoch's fold is a launch of its own
             // tile classes: corners (general kernel), row-edge, column-edge, interior
             const int n0 = st.n_corner, nr = st.n_rowedge, ncl = n_edge - n0 - nr;
             const int cnt[3] = {n0, nr, ncl};
@@ -1095,7 +1118,7 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st, bool toge
             auto launch_epoch = [&]() -> int {
                 if (multi) HIPCHK(hipEventRecord(c->ev_bar, c->stream));
                 double ucells = 0, ubytes = 0;
-                hipEvent_t first = nullptr;  // start of the update phase: its first launch
+                hipEvent_t first = nullptr, last = nullptr;  // start of the update phase's first launch, end of its last
                 if (resident) {
                     // every time block of the epoch in one launch; the counters start at zero
                     for (int o = 0; o < nl; ++o)
@@ -1143,10 +1166,11 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st, bool toge
                     if (rtile) {
                         LaunchTimer lt(c);
                         HIPCHK(launch_rtile(mode, plan.waves, (const RegTile*)st.d_tiles, st.ntiles, d_it, st.d_sims, o, Tb,
-                                            c->stream));
+                                            o == 0 ? before : FoldRun{}, c->stream));
                         const int k = mode == TOMO_MODE_PHYSICAL ? TILE_INNER : TILE_CORNER;
                         lt.done(mode == TOMO_MODE_PHYSICAL ? TOMO_KERNEL_FUSED : TOMO_KERNEL_GENERAL, cells[k], bytes[k]);
                         if (!first) first = lt.a;
+                        last = lt.b;
                         continue;
                     }
                     if (mode != TOMO_MODE_PHYSICAL) {  // (the resident form skipped this loop)
@@ -1209,13 +1233,14 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st, bool toge
                 }
                 // the fold runs after every update launch of the epoch: its start ends the update phase
                 hipEvent_t fold_start = nullptr;
-                for (int prec = 0; prec < 2; ++prec) {
+                for (int prec = 0; prec < 2 && fold_after; ++prec) {
                     if (!(prec ? fp64_any : fp32_any)) continue;
                     LaunchTimer lt(c);
                     HIPCHK(launch_fold(prec == 1, d_it, (int)ms.size(), st.d_sims, maxP, maxF, c->stream));
                     lt.done(TOMO_KERNEL_FOLD);
                     if (!fold_start) fold_start = lt.a;
                 }
+                if (!fold_after) fold_start = last;
                 if (c->prof && first && fold_start) c->pending.push_back({first, fold_start, -1, ucells, ubytes, false});
                 return TOMO_OK;
             };
@@ -1231,6 +1256,8 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st, bool toge
                     minn = std::min(minn, h_it[i].nsteps);
                 }
                 nl = (maxn + Tb - 1) / Tb;
+                fold_after = !around || e == E - 1;
+                before = around && e > 0 ? FoldRun{st.d_items + (e - 1) * nsim, nsim, maxP, maxF} : FoldRun{};
                 if (c->use_graph && !st.fixed && !resident && !c->prof && minn == K) {
                     const std::vector<int64_t> gk = {mode, T, S, c->Si, W, c->Wi, c->ER, c->form, K, c->grid_mult, ntiles, maxP,
                                                      fp32_any, fp64_any, (int64_t)ms.size(), plan.T, plan.waves, plan.tall, (int64_t)(intptr_t)d_it,
@@ -1416,7 +1443,7 @@ static int eval_many(tomo_ctx* c, const tomo_sim_config& cfg, const double* para
         for (size_t v = 0; v < n_vec && !rc; ++v) {
             for (int e = 0; e < E && !rc; ++e) {
                 Slot* s = nullptr;
-                rc = slot_create(c, cfg, params + v * dim, dim, e, &s);
+                rc = slot_create(c, cfg, params + v * dim, dim, e, 1, &s);
                 if (rc) break;
                 std::vector<Slot*> one{s};
                 rc = run_and_project(c, one, dD + v * L + (size_t)e * F * A, dP + v * L + (size_t)e * F * A, false);
@@ -1433,7 +1460,7 @@ static int eval_many(tomo_ctx* c, const tomo_sim_config& cfg, const double* para
                 std::vector<Slot*> mine;
                 for (int e = 0; e < E; ++e) {
                     Slot* s = nullptr;
-                    int r2 = slot_create(c, cfg, params + v * dim, dim, e, &s);
+                    int r2 = slot_create(c, cfg, params + v * dim, dim, e, E - e, &s);
                     if (r2) {
                         for (Slot* m : mine) slot_destroy(c, m);
                         if (r2 == TOMO_E_NOMEM && !sl.empty()) goto run_pass;
@@ -1490,7 +1517,7 @@ static int get_target(tomo_ctx* c, const tomo_sim_config& cfg, std::vector<float
     int rc = TOMO_OK;
     for (int e = 0; e < cfg.n_exc && !rc; ++e) {
         Slot* s = nullptr;
-        rc = slot_create(c, cfg, tv.data(), tv.size(), e, &s);
+        rc = slot_create(c, cfg, tv.data(), tv.size(), e, cfg.n_exc - e, &s);
         if (!rc) sl.push_back(s);
     }
     Work w(c);
@@ -1578,7 +1605,7 @@ static int progress_once(tomo_ctx* c, int* n_active) {
         int rc = TOMO_OK;
         for (int e = 0; e < r->cfg.n_exc && !rc; ++e) {
             Slot* s = nullptr;
-            rc = slot_create(c, r->cfg, r->params.data(), r->params.size(), e, &s);
+            rc = slot_create(c, r->cfg, r->params.data(), r->params.size(), e, 0, &s);
             if (!rc) { s->req = (long)r->ticket; r->slots.push_back(s); }
         }
         if (rc) {
@@ -1680,12 +1707,14 @@ int eval_noalloc(tomo_ctx* c, char* base, const tomo_sim_config& cfg, const doub
     if (c->K % c->T) return fail(TOMO_E_INVALID, "chunk must be a multiple of the fused step count");
     // host setup of every excitation first: it sizes the slot
     std::vector<std::unique_ptr<Slot>> slots;
-    size_t sbytes = 0;
+    size_t sbytes = 0, round_bytes = 0;  // without and with the spare sample rows
     for (int e = 0; e < E; ++e) {
         std::unique_ptr<Slot> s(new Slot());
         rc = build_setup(cfg, params, n_params, e, s->su);
         if (rc) return rc;
+        s->srows = c->K;
         sbytes = std::max(sbytes, slot_bytes(s->su, c->K));
+        round_bytes = std::max(round_bytes, slot_bytes(s->su, c->K + kRoundRows));
         slots.push_back(std::move(s));
     }
     size_t off = 0;
@@ -1698,6 +1727,11 @@ int eval_noalloc(tomo_ctx* c, char* base, const tomo_sim_config& cfg, const doub
     char* pstage = carve(kNoallocProjBytes);
     LaunchItem* d_items = (LaunchItem*)carve(sizeof(LaunchItem) * kMaxStagedEpochs);
     const size_t total = TOMO_NOALLOC_SCRATCH_BYTES;
+    // the spare rows where they leave 4 MiB (131072 tiles) for the tile list
+    if (round_bytes + off + (4u << 20) <= total) {
+        sbytes = round_bytes;
+        for (auto& s : slots) s->srows = c->K + kRoundRows;
+    }
     const size_t slot_off = (total - sbytes) & ~(size_t)255;
     if (sbytes > total || slot_off < off + align256(64 * sizeof(TileItem)))
         return fail(TOMO_E_NOMEM, "configuration needs " + std::to_string(off + sbytes) +
@@ -1931,7 +1965,7 @@ int tomo_autotune(tomo_ctx* c, const tomo_sim_config* cfg, int n_sims, tomo_sche
     int rc = TOMO_OK;
     for (int i = 0; i < n_sims && !rc; ++i) {
         Slot* s = nullptr;
-        rc = slot_create(c, tc, p.data(), p.size(), i % tc.n_exc, &s);
+        rc = slot_create(c, tc, p.data(), p.size(), i % tc.n_exc, 0, &s);
         if (!rc) sl.push_back(s);
     }
     const bool prof = c->prof;
@@ -2145,7 +2179,7 @@ int tomo_sim_create(tomo_ctx* c, const tomo_sim_config* cfg, const double* param
     if (!c || !cfg || !out) return fail(TOMO_E_INVALID, "null argument");
     std::lock_guard<std::mutex> g(c->mu);
     Slot* s = nullptr;
-    int rc = slot_create(c, *cfg, params, n, exc, &s);
+    int rc = slot_create(c, *cfg, params, n, exc, 0, &s);
     if (rc) return rc;
     std::shared_ptr<SimLink> link = std::make_shared<SimLink>();
     link->ctx = c;

@@ -44,7 +44,7 @@ struct DevSim {
     int ps, js, xs, ys;
     const uint8_t* mat;
     const int* span;       // lo, hi, off per row
-    float* samp;           // 3 x K x P
+    float* samp;           // 3 x srows x P
     void* accJ;            // F x P
     void* accM;
     const float* srcw;     // physical source waveform per step (nullptr in ref mode)
@@ -55,6 +55,7 @@ struct DevSim {
     int sx, sy;            // physical source cell
     int mode, flags;
     int nmat, nfreq, chunk, steps;
+    int srows, pad;        // sample rows: chunk, or more where a chunk's samples outlive its epoch (LaunchItem::samp0)
     float coef[TOMO_MAX_MAT * TOMO_NCOEF];
     // CPML 1-D profiles: E (inverse kappa, a, b) and H (inverse kappa, a, b)
     float ike[TOMO_MAX_NC], ae[TOMO_MAX_NC], be[TOMO_MAX_NC];
@@ -78,6 +79,7 @@ struct LaunchItem {
     int step0;     // first step of this epoch
     int parity0;   // buffer holding the state at step0
     int nsteps;    // steps to do in this epoch (<= chunk)
+    int samp0;     // sample row of the epoch's first step; the rows go round after srows
 };
 
 // Tile classes of physical-mode simulations (TileItem::cls).

@@ -28,6 +28,7 @@
 // row in material costs 3 times a vacuum one).  Spilled prologues cost more than
 // shorter tiles (16 rows at the strips: 169 -> 270 us).
 #include "device.h"
+#include "fold.h"
 #include "kernels.h"
 
 namespace tomo {
@@ -257,7 +258,7 @@ __device__ __forceinline__ void tile_wave(const RegTile& tile, const DevSim* __r
     }
 
     // ---- contour samples: face rows / columns hold H and Ez, their outer neighbours Ez
-    const int D = Sp->D, P = Sp->P, K = Sp->chunk, cx_hi = Sp->cx_hi, cy_lo = Sp->cy_lo;
+    const int D = Sp->D, P = Sp->P, K = Sp->srows, cx_hi = Sp->cx_hi, cy_lo = Sp->cy_lo;
     const bool own = x >= tile.x0 && x < tile.xe;
     const Buffer Z = buffer_of(Sp->samp, (size_t)3 * K * P * 4);
     // rows of the wave that the tile owns: [ra, rb)
@@ -282,7 +283,7 @@ __device__ __forceinline__ void tile_wave(const RegTile& tile, const DevSim* __r
     const unsigned zx1 = x_lane && x_face ? zx0 + (unsigned)kp4 : kOff;
     const int L2 = Sp->L2;
     auto sample = [&](int k) {
-        const int o = k * P * 4, f = opaque(m_face), g = opaque(m_out), xr = opaque(m_x);
+        const int o = (k >= K ? k - K : k) * P * 4, f = opaque(m_face), g = opaque(m_out), xr = opaque(m_x);
         if (f | g) {
 #pragma unroll
             for (int i = 0; i < R; ++i) {
@@ -542,12 +543,39 @@ __device__ __forceinline__ void tile_wave(const RegTile& tile, const DevSim* __r
 // contiguous eighth of the tile list, so that tiles that share halo rows and
 // columns share an L2 (64 simulations of 512^2: 640 -> 237 MB read per launch,
 // 203 -> 193 us; 4 x 401^2 20.2 -> 17.5 us).
+// Workgroups of a launch, after the tiles', that fold the previous epoch's
+// samples: bx blocks of contour points x bz groups of fpb frequencies per item.
+// The tiles of this launch write other sample rows (LaunchItem::samp0).  A fold
+// is bound by its launch and the latency of its loads; beside the tiles it
+// costs one simulation nothing that can be measured.
+constexpr int kFoldFreqs = 8;
+struct FoldShare {
+    const LaunchItem* items;
+    int blocks, bx, bz, fpb;
+};
+
 template <int MODE, int NW>
 __global__ __launch_bounds__(NW* kLane) __attribute__((amdgpu_waves_per_eu(4))) void k_rtile(
     const RegTile* __restrict__ tiles, int ntiles, const LaunchItem* __restrict__ items, const DevSim* __restrict__ sims, int ordinal,
-    int tsteps) {
-    __shared__ TileLds<MODE == TOMO_MODE_REF_COMPAT, NW> lds;
-    const int ti = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    int tsteps, FoldShare fold) {
+    __shared__ union {
+        TileLds<MODE == TOMO_MODE_REF_COMPAT, NW> tile;
+        struct { float2 wJ[kFoldFreqs * 64], wM[kFoldFreqs * 64]; } fold;
+    } u;
+    TileLds<MODE == TOMO_MODE_REF_COMPAT, NW>& lds = u.tile;
+    const int tblocks = gridDim.x - fold.blocks;
+    if ((int)blockIdx.x >= tblocks) {
+        const int b = blockIdx.x - tblocks, z = b / fold.bx, item = z / fold.bz;
+        const LaunchItem it = fold.items[item];
+        const DevSim* S = sims + it.sim;
+        const int fb = (z - item * fold.bz) * fold.fpb, nf = min(S->nfreq, fb + fold.fpb) - fb;
+        const int nk = min(it.nsteps, S->chunk), p = (b - z * fold.bx) * (NW * kLane) + threadIdx.x;
+        if (nk <= 0 || nf <= 0) return;
+        if (fold.fpb == 1) fold_fp32<1>(S, it, nk, fb, nf, p, u.fold.wJ, u.fold.wM);
+        else fold_fp32<kFoldFreqs>(S, it, nk, fb, nf, p, u.fold.wJ, u.fold.wM);
+        return;
+    }
+    const int ti = (blockIdx.x & 7) * (tblocks >> 3) + (blockIdx.x >> 3);
     if (ti >= ntiles) return;
     const RegTile tile = tiles[ti];
     const LaunchItem it = items[tile.item];
@@ -556,7 +584,7 @@ __global__ __launch_bounds__(NW* kLane) __attribute__((amdgpu_waves_per_eu(4))) 
     if (nst <= 0) return;  // uniform over the workgroup
     const int lane = threadIdx.x & (kLane - 1);
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kLane);
-    const int par = it.parity0 ^ (ordinal & 1), step0 = it.step0 + ordinal * tsteps, k0 = ordinal * tsteps;
+    const int par = it.parity0 ^ (ordinal & 1), step0 = it.step0 + ordinal * tsteps, k0 = it.samp0 + ordinal * tsteps;
     const int nx = Sp->nx, ny = Sp->ny, nc = Sp->nc;
     const int rows = tile.rows, yb = tile.yl + wv * rows;
     const bool mat = (tile.matmask >> wv) & 1;
@@ -608,13 +636,23 @@ __global__ __launch_bounds__(NW* kLane) __attribute__((amdgpu_waves_per_eu(4))) 
 }  // namespace
 
 hipError_t launch_rtile(int mode, int waves, const RegTile* tiles, int ntiles, const LaunchItem* items, const DevSim* sims,
-                        int ordinal, int tsteps, hipStream_t st) {
+                        int ordinal, int tsteps, const FoldRun& f, hipStream_t st) {
     if (ntiles <= 0) return hipErrorInvalidValue;
-    dim3 g((ntiles + 7) / 8 * 8), b(waves * kLane);
-#define TT(MM, WW)                                                                            \
-    if (mode == MM && waves == WW) {                                                          \
-        TIMED_LAUNCH((k_rtile<MM, WW>), g, b, 0, st, tiles, ntiles, items, sims, ordinal, tsteps);    \
-        return hipGetLastError();                                                             \
+    FoldShare fold{};
+    if (f.n > 0) {
+        const int wg = waves * kLane;
+        fold.items = f.items;
+        fold.bx = (f.max_p + wg - 1) / wg;
+        // fewer than about one block per CU: spread the frequencies too (as launch_fold)
+        fold.fpb = (f.max_p + 255) / 256 * f.n < 256 ? 1 : kFoldFreqs;
+        fold.bz = (f.max_f + fold.fpb - 1) / fold.fpb;
+        fold.blocks = fold.bx * fold.bz * f.n;
+    }
+    dim3 g((ntiles + 7) / 8 * 8 + fold.blocks), b(waves * kLane);
+#define TT(MM, WW)                                                                                        \
+    if (mode == MM && waves == WW) {                                                                      \
+        TIMED_LAUNCH((k_rtile<MM, WW>), g, b, 0, st, tiles, ntiles, items, sims, ordinal, tsteps, fold);  \
+        return hipGetLastError();                                                                         \
     }
     TT(TOMO_MODE_PHYSICAL, 8) TT(TOMO_MODE_PHYSICAL, 16) TT(TOMO_MODE_REF_COMPAT, 8) TT(TOMO_MODE_REF_COMPAT, 16)
 #undef TT
