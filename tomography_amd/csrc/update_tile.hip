@@ -436,8 +436,26 @@ __device__ __forceinline__ void tile_wave(const RegTile& tile, const DevSim* __r
     };
     const Profile<REF>* we = lds.row_e + wv * R;      // E row i
     const Profile<REF>* wh = lds.row_h + wv * R + 1;  // H row i
-    auto E = [&](int i) { return YS ? we[i] : Profile<REF>{}; };
-    auto H = [&](int i) { return YS ? wh[i] : Profile<REF>{}; };
+    // Physical mode holds its rows' profiles in registers for the whole block:
+    // read from LDS in each step, they were 12 to 24 waits on the way of a wave
+    // with one other to hide behind (256^2 2.65 -> 2.36 ms per evaluation, 64 of
+    // 512^2 88.0 -> 85.2).  The reference's, with 64-bit kappa, do not fit.
+    constexpr bool HELD = YS && !REF;
+    Profile<REF> he[HELD ? R : 1], hh[HELD ? R + 1 : 1];
+    if constexpr (HELD) {
+#pragma unroll
+        for (int i = 0; i < R; ++i) he[i] = we[i];
+#pragma unroll
+        for (int i = 0; i <= R; ++i) hh[i] = wh[i - 1];
+    }
+    auto E = [&](int i) {
+        if constexpr (HELD) return he[i];
+        else return YS ? we[i] : Profile<REF>{};
+    };
+    auto H = [&](int i) {
+        if constexpr (HELD) return hh[i + 1];
+        else return YS ? wh[i] : Profile<REF>{};
+    };
     auto hs = [&](int i, float up) {
         h_step(ez[i], up, hx[i], &hy[i], XS ? &phx[XS ? i : 0] : nullptr, YS ? &phy[YS ? i : 0] : nullptr, H(i));
     };
