@@ -56,13 +56,14 @@ hipError_t launch_twave(int T, int rows_per_wave, const TileItem* tiles, int nti
 constexpr int kTileRowsEdge = 4, kTileRowsClean = 8, kTileRowsTall = 16;
 // `fold`: the previous epoch's items (n of them, FP32 running DFT), whose
 // samples further workgroups of the launch fold; this launch must write other
-// sample rows (LaunchItem::samp0).
+// sample rows (LaunchItem::samp0).  `lone`: the description of the launch's only
+// simulation, null when there are several (a hint: it changes no result).
 struct FoldRun {
     const LaunchItem* items;
     int n, max_p, max_f;
 };
 hipError_t launch_rtile(int mode, int waves, const RegTile* tiles, int ntiles, const LaunchItem* items, const DevSim* sims,
-                        int ordinal, int tsteps, const FoldRun& fold, hipStream_t st);
+                        int ordinal, int tsteps, const DevSim* lone, const FoldRun& fold, hipStream_t st);
 
 // Resident update form: one cooperative launch advances every simulation of
 // `items` by its epoch (all time blocks), one workgroup per ResTile, all

@@ -1166,7 +1166,7 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st, bool toge
                     if (rtile) {
                         LaunchTimer lt(c);
                         HIPCHK(launch_rtile(mode, plan.waves, (const RegTile*)st.d_tiles, st.ntiles, d_it, st.d_sims, o, Tb,
-                                            o == 0 ? before : FoldRun{}, c->stream));
+                                            nsim == 1 ? st.d_sims + ms[0]->idx : nullptr, o == 0 ? before : FoldRun{}, c->stream));
                         const int k = mode == TOMO_MODE_PHYSICAL ? TILE_INNER : TILE_CORNER;
                         lt.done(mode == TOMO_MODE_PHYSICAL ? TOMO_KERNEL_FUSED : TOMO_KERNEL_GENERAL, cells[k], bytes[k]);
                         if (!first) first = lt.a;
