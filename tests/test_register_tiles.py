@@ -160,3 +160,26 @@ def test_a_budget_without_room_for_spare_sample_rows():
             got.append(c.eval_batch(cfg, PHYS_PARAMS, target=T, want_farfield=True)[1])
     assert np.abs(got[0]).max() > 0
     assert np.array_equal(*got)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n, many", [(830, 1), (1030, 1), (401, 8), (140, 40), (259, 24)])
+def test_tile_order_changes_no_result(n, many):
+    """Sets of more tiles than compute units are dealt by work: one grid in pairs
+    of tiles, many in several rounds, 8 and 16 waves; against the row sweeps."""
+    cfg = wide(nx=n, ny=n, n_exc=1, steps=70)
+    V = np.tile(PHYS_PARAMS, (many, 1))
+    V[:, 0] += np.linspace(-1, 1, many)
+    T = np.zeros(cfg.farfield_len(), np.float32)
+    with t.Context() as c:
+        c.set_schedule(tsteps=4, chunk=60, form=t.FORM_FUSED)
+        D = c.eval_batch(cfg, V, target=T, want_farfield=True)[1]
+    with t.Context() as c:
+        c.set_schedule(tsteps=4, seg_rows=16, edge_waves=2, chunk=60, form=t.FORM_STREAMS)
+        for i in sorted({0, many // 2, many - 1}):
+            g = c.sim(cfg, V[i])
+            g.step(cfg.steps)
+            want = g.farfield()[0]
+            g.close()
+            assert np.abs(want).max() > 0
+            assert np.array_equal(D[i].ravel(), want.ravel())

@@ -53,6 +53,7 @@ hipError_t launch_twave(int T, int rows_per_wave, const TileItem* tiles, int nti
 // and the row below); kTileRowsClean for vacuum at the strips of one axis, and
 // for physical-mode material clear of them and of the source; else
 // kTileRowsEdge.  The six field planes take less than 2 GiB together.
+// A tile of item -1 is an unused place.
 constexpr int kTileRowsEdge = 4, kTileRowsClean = 8, kTileRowsTall = 16;
 // `fold`: the previous epoch's items (n of them, FP32 running DFT), whose
 // samples further workgroups of the launch fold; this launch must write other

@@ -840,11 +840,13 @@ void build_reg_tiles(Slot* sl, int item, const TilePlan& p, std::vector<RegTile>
 // cell and need enough nodes to fill the device; 16 waves give short grids a
 // whole column of tiles each.  Measured us per step on MI355X (steps x waves,
 // t: tall; chunks of 60 steps):
-//   one 256^2  12x8 1.15, 8x8 1.28, 12x8t 1.32    one 512^2  10x8 1.10, 12x8 1.18, 12x8t 1.32
-//   one 1024^2 12x8t 1.88, 10x8 2.07, 12x16 2.3   one 2048^2 12x8t 3.95, 8x8t 4.39, 8x8 4.88
-//   64 x 128^2 15x16 3.08, 12x16 3.40, 6x8 3.99   8 x 256^2  12x16 1.59, 8x8 1.69, 15x16 1.95
-//   8 x 725^2  12x8t 4.61, 8x8t 5.11, 8x8 5.34    reference 4 x 401^2 6x8 2.08, 10x8t 2.56;
-//   reference 16 x 401^2 10x8t 5.65, 6x8 6.10
+//   one 256^2  12x8 1.04, 10x8 1.20, 12x8t 1.23   one 512^2  12x8 1.06, 10x8 1.08, 12x8t 1.31
+//   one 725^2  10x8 1.27, 12x8t 1.31, 12x8 1.37   one 1024^2 12x8t 1.65, 10x8 1.79, 15x16t 1.92
+//   one 2048^2 12x8t 3.68, 8x8t 4.21, 10x8 4.52   8 x 725^2  12x8t 4.38, 8x8t 4.58, 10x8 5.35
+//   64 x 128^2 15x16 2.90, 12x16 3.22, 20x16 3.68 8 x 256^2  12x16 1.56, 15x16 1.58, 6x8 1.73
+//   32 x 256^2 12x16 4.45, 6x8t 4.62              16 x 512^2 12x8t 5.03, 12x16 5.69, 6x8 5.92
+//   reference 4 x 201^2 12x8 1.60, 8x8 1.80; 4 x 401^2 6x8 2.10, 10x8t 2.28; 16 x 401^2
+//   10x8t 5.21, 6x8 5.38
 TilePlan plan_reg_tiles(const std::vector<Slot*>& ms, int K) {
     int64_t nodes = 0;
     int longest = 0;
@@ -861,18 +863,74 @@ TilePlan plan_reg_tiles(const std::vector<Slot*>& ms, int K) {
     if (ms[0]->d.mode != TOMO_MODE_PHYSICAL) {
         p.waves = 8;
         p.tall = nodes > 1000000;
-        deep = p.tall ? 10 : 6;
+        deep = p.tall ? 10 : nodes < 300000 ? 12 : 6;
     } else if (fit16 && ms.size() > 1 && longest <= 300) {
         p.waves = 16;
         deep = longest <= 160 ? 15 : 12;
     } else {
         p.waves = 8;
-        p.tall = nodes > 500000;
-        deep = p.tall || nodes < 200000 ? 12 : 10;
+        p.tall = nodes > 600000;
+        deep = p.tall || nodes < 300000 ? 12 : 10;
     }
     const int launches = (K + deep - 1) / deep;
     p.T = (K + launches - 1) / launches;
     return p;
+}
+
+// Order of the register tiles.  The kernel deals the list to the eight XCDs in
+// contiguous eighths (update_tile.hip), one tile after the other as compute
+// units come free, so the order decides which tiles share a unit and which
+// start last.  A launch that gives no unit more than one tile keeps the
+// list's order.  Otherwise the eighths take equal work instead of equal
+// counts, and in each
+// - where two 8-wave tiles fit a unit and no unit needs a third, the heaviest
+//   tiles run alone and the others in pairs of a heavy and a light one
+//   (1024^2: 397 tiles on 256 units, 15.1 -> 13.6 ms per evaluation);
+// - where more follow, the heaviest start first, so that the launch ends on
+//   light ones (requests of 512^2 16.2 -> 14.3 ms, 64 of 512^2 85.0 -> 83.3,
+//   reference 16 x 401^2 10.5 -> 10.0).
+// Unused places of an eighth hold tiles of item -1.  Work: vector instructions
+// per row and step of the tile's stages, measured from the compiled loops.
+void order_tiles(const std::vector<Slot*>& ms, int waves, int cus, std::vector<RegTile>& v) {
+    const int xcus = cus / 8;
+    if (xcus < 1 || (int)v.size() <= 8 * xcus) return;
+    struct Weighed { int work, tile; };
+    std::vector<Weighed> g[8];
+    std::vector<int> work(v.size());
+    int64_t total = 0, sum = 0;
+    for (size_t i = 0; i < v.size(); ++i) {
+        const RegTile& t = v[i];
+        const DevSim& d = ms[t.item]->d;
+        const bool xs = t.xl <= d.nc || t.xl + 64 > d.nx - d.nc;
+        for (int w = 0; w < waves; ++w) {
+            const int y = t.yl + w * t.rows;
+            const bool ys = y <= d.nc + 1 || y + t.rows > d.ny - d.nc;
+            work[i] += t.rows * (10 + 11 * xs + 11 * ys + 8 * (t.matmask >> w & 1));
+        }
+        total += work[i];
+    }
+    for (size_t i = 0; i < v.size(); ++i) {
+        g[(sum + work[i] / 2) * 8 / total].push_back({work[i], (int)i});
+        sum += work[i];
+    }
+    size_t per = 0;
+    for (auto& x : g) per = std::max(per, x.size());
+    RegTile none{};
+    none.item = -1;
+    std::vector<RegTile> out(8 * per, none);
+    for (int k = 0; k < 8; ++k) {
+        RegTile* o = out.data() + k * per;
+        const int n = (int)g[k].size();
+        std::stable_sort(g[k].begin(), g[k].end(), [](const Weighed& a, const Weighed& b) { return a.work > b.work; });
+        const bool pairs = waves == 8 && n > xcus && n <= 2 * xcus;
+        const int two = pairs ? n - xcus : 0, one = pairs ? xcus - two : n;
+        for (int i = 0; i < one; ++i) o[two + i] = v[g[k][i].tile];
+        for (int i = 0; i < two; ++i) {
+            o[i] = v[g[k][one + i].tile];
+            o[xcus + i] = v[g[k][n - 1 - i].tile];
+        }
+    }
+    v.swap(out);
 }
 
 // The resident launches' error word: 16-byte aligned past the counters.
@@ -995,6 +1053,7 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st, bool toge
                     st.plan = plan_reg_tiles(ms, K);
                 if (st.plan.T) {
                     for (size_t i = 0; i < ms.size(); ++i) build_reg_tiles(ms[i], (int)i, st.plan, trg);
+                    if (st.plan.T) order_tiles(ms, st.plan.waves, c->cus, trg);
                     if (st.fixed && trg.size() * sizeof(RegTile) > st.tiles_cap * sizeof(TileItem)) {
                         st.plan = TilePlan{};  // the row sweeps' list is the smaller one
                         trg.clear();

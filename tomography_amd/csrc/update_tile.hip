@@ -617,6 +617,7 @@ __global__ __launch_bounds__(NW* kLane) __attribute__((amdgpu_waves_per_eu(4))) 
     if (ti >= ntiles) return;
     const RegTile tile = tiles[ti];
     if constexpr (MODE == TOMO_MODE_PHYSICAL) warm(lone, items);
+    if (tile.item < 0) return;  // an unused place of an XCD's share
     const LaunchItem it = items[tile.item];
     const DevSim* Sp = sims + tile.sim;
     const int nst = min(tsteps, it.nsteps - ordinal * tsteps);
