@@ -167,7 +167,8 @@ def test_a_budget_without_room_for_spare_sample_rows():
 def test_tile_order_changes_no_result(n, many):
     """Sets of more tiles than compute units are dealt by work: one grid in pairs
     of tiles, many in several rounds, 8 and 16 waves; against the row sweeps."""
-    cfg = wide(nx=n, ny=n, n_exc=1, steps=70)
+    # (the contour 20 cells outside the source, so that 70 steps reach it)
+    cfg = wide(nx=n, ny=n, n_exc=1, steps=70, ntff_offset=max(n // 2 - 80, 15))
     V = np.tile(PHYS_PARAMS, (many, 1))
     V[:, 0] += np.linspace(-1, 1, many)
     T = np.zeros(cfg.farfield_len(), np.float32)
