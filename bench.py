@@ -100,15 +100,16 @@ def traffic_for(workload, kernel, schedule):
     return rec.get("kernels", {}).get(kernel, {}).get("hbm_bytes_per_launch")
 
 
-def add_traffic(rl, traffic, tsteps):
+def add_traffic(rl, traffic, cells):
     """Counter-measured HBM bytes per launch beside the algorithmic figure:
-    the real HBM fraction, and the time-blocked minimum (a launch advances
-    tsteps steps, so the least it can move is the algorithmic bytes / tsteps,
-    the state read and written once)."""
+    the real HBM fraction, and the time-blocked minimum (a launch advances the
+    workload's `cells` by cell_steps / cells steps, so the least it can move is
+    the algorithmic bytes over that, the state read and written once)."""
     if not rl:
         return rl
     rl["traffic"] = traffic
-    tmin = rl["alg_bytes_per_launch"] / tsteps
+    rl["steps_per_launch"] = round(rl["cell_steps_per_launch"] / cells, 2)
+    tmin = rl["alg_bytes_per_launch"] / max(1.0, rl["cell_steps_per_launch"] / cells)
     rl["blocked_min_bytes"] = round(tmin, 1)
     if traffic:
         avg_s = rl["avg_launch_us"] / 1e6
@@ -600,7 +601,7 @@ def main():
            "ms_per_step_profiled_pass": round(dt_prof / args.steps * 1e3, 3)}
     rl = roofline_from(st)
     if rl:
-        add_traffic(rl, traffic_for("plain_cfg2", rl["kernel"], tuple(sched.values())), sched["tsteps"])
+        add_traffic(rl, traffic_for("plain_cfg2", rl["kernel"], tuple(sched.values())), float(cfg.nx) * cfg.ny)
     out["roofline"] = rl
     out["kernel_ms_per_step"] = kernel_ms(st, args.steps)
     bsch = dict(BATCH_SCHEDULE)
@@ -611,7 +612,8 @@ def main():
         bcs = cell_steps(bcfg) * nvec
         brl = roofline_from(bst)
         if brl:
-            add_traffic(brl, traffic_for("batched_cfg3", brl["kernel"], tuple(bsched.values())), bsched["tsteps"])
+            add_traffic(brl, traffic_for("batched_cfg3", brl["kernel"], tuple(bsched.values())),
+                        float(bcfg.nx) * bcfg.ny * bcfg.n_exc * nvec)
         out["batched"] = {"workload": "512^2, dx 0.5 mm, 4096 steps; 64 vectors x 16 antennas = 1024 simulations, "
                                       "16 freq x 360 angles (CFG3)",
                           "Mcell_steps_per_s": round(bcs / bdt / 1e6, 1), "evals_per_s": round(nvec / bdt, 3),

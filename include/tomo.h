@@ -173,8 +173,8 @@ int tomo_set_schedule(tomo_ctx *ctx, const tomo_schedule *s);
 int tomo_get_schedule(tomo_ctx *ctx, tomo_schedule *s);
 /* The schedule the FDTD_GPU / FDTD_CPU shims install on their context.  Of its
  * fields the reference-compatible simulations (register tiles under every form)
- * take the 64-step DFT chunk.  The DFT chunk sets the FP32 partial sums of the running DFT,
- * so contexts compare bit for bit only under equal chunks. */
+ * take the 64-step DFT chunk.  The chunk sets the FP32 partial sums of the
+ * running DFT, so contexts compare bit for bit only under equal chunks. */
 #define TOMO_DROPIN_SCHEDULE {8, 12, 1, 1, 64, 16, TOMO_FORM_RESIDENT, 1, 0}
 
 /* Autotuner: time candidate schedules on n_sims resident simulations of

@@ -24,6 +24,8 @@ import re
 import sys
 from collections import defaultdict
 
+# name in a trace of the register-tile kernels, by the kernel class the library reports them under
+REGISTER_TILES = {"k_tfused": "k_rtile<1, 8>", "k_tblock": "k_rtile<0, 8>"}
 _NAME = re.compile(r"(k_[a-z0-9_]+)(?:<([^>]*)>)?")
 
 
@@ -133,7 +135,9 @@ def traffic(fetch_path, write_path, bench_path, copy_mb, command):
     from a FETCH_SIZE and a WRITE_SIZE summary (`pmc` output, each with the
     timed region's dispatches) and the bench line of the profiled command.
     Each counter is scaled by what it reads for the largest copy dispatch of
-    the run (bench.py --calib-copy-mb copy_mb: a copy of copy_mb MiB)."""
+    the run (bench.py --calib-copy-mb copy_mb: a copy of copy_mb MiB).  The
+    register tiles run under one name in every leg (REGISTER_TILES): their last
+    dispatches are the last leg's, so the plain leg needs a --no-batched run."""
     fetch, write = json.load(open(fetch_path)), json.load(open(write_path))
     lines = [l for l in open(bench_path) if l.lstrip().startswith("{")]
     bench = json.loads(lines[-1])
@@ -153,6 +157,8 @@ def traffic(fetch_path, write_path, bench_path, copy_mb, command):
         kern = {}
         for r in [rl] + list(rl.get("other_kernels", [])):
             key = f"{r['kernel']}<{T}>"
+            if key not in fetch["kernels"] and name == legs[-1][0]:
+                key = REGISTER_TILES.get(r["kernel"], key)
             fk = fetch["kernels"].get(key, {}).get("avg_kib_last")
             wk = write["kernels"].get(key, {}).get("avg_kib_last")
             if fk is None or wk is None:
