@@ -1044,7 +1044,7 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st, bool toge
                 // Register tiles wherever the grids allow them (64 columns and 32
                 // rows at least): reference-compatible simulations, the fused form,
                 // and the streams form for simulations that advance together (64 of
-                // 512^2: 131 ms against 174 on four streams; 64 of 128^2: 5.3
+                // 512^2: 83.5 ms against 174 on four streams; 64 of 128^2: 3.0
                 // against 21).  One simulation by itself under an installed streams
                 // schedule keeps that form's four kernels, as its name says.
                 const bool streams_alone = c->form == TOMO_FORM_STREAMS && c->form_set && !together;

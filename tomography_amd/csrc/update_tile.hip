@@ -557,10 +557,6 @@ __device__ __forceinline__ void tile_wave(const RegTile& tile, const DevSim* __r
     }
 }
 
-// Workgroups are dealt to the eight XCDs round-robin: XCD g walks the g-th
-// contiguous eighth of the tile list, so that tiles that share halo rows and
-// columns share an L2 (64 simulations of 512^2: 640 -> 237 MB read per launch,
-// 203 -> 193 us; 4 x 401^2 20.2 -> 17.5 us).
 // Bring the lines of a lone simulation's description that a tile reads, and its
 // launch item, into the scalar cache while the tile itself is on its way (they
 // are found through it: without this, three round trips before the first load
@@ -592,6 +588,10 @@ struct FoldShare {
     int blocks, bx, bz, fpb;
 };
 
+// Workgroups are dealt to the eight XCDs round-robin: XCD g walks the g-th
+// contiguous eighth of the tile list, so that tiles that share halo rows and
+// columns share an L2 (64 simulations of 512^2: 640 -> 237 MB read per launch,
+// 203 -> 193 us; 4 x 401^2 20.2 -> 17.5 us).
 template <int MODE, int NW>
 __global__ __launch_bounds__(NW* kLane) __attribute__((amdgpu_waves_per_eu(4))) void k_rtile(
     const RegTile* __restrict__ tiles, int ntiles, const LaunchItem* __restrict__ items, const DevSim* __restrict__ sims, int ordinal,
