@@ -231,6 +231,7 @@ __device__ __forceinline__ void tile_wave(const RegTile& tile, const DevSim* __r
     const float chx = Sp->chx, chy = Sp->chy, dxf = Sp->dxf, dyf = Sp->dyf, chx_d = Sp->chx_d, chy_d = Sp->chy_d;
     const float cb0 = Sp->coef[1];  // vacuum curl coefficient (the vacuum Ez coefficient is exactly 1)
     const bool clamp = REF && !(Sp->flags & TOMO_FLAG_NO_NAN_CLAMP);
+    const bool debye = !(Sp->flags & TOMO_FLAG_CPU_COEFS);  // the CPU form has no Jp: an infinite Ez must not make one
     const bool ex_ok = !XS || (x >= 1 && x < nx);
     const bool bot = YS && yb == 0, top = YS && yb + R - 1 == ny;  // PEC rows: the wave's first, its last
     Profile<REF> Le, Lh;
@@ -381,8 +382,10 @@ __device__ __forceinline__ void tile_wave(const RegTile& tile, const DevSim* __r
                 const float f1 = expf(-a1 * a1), fo = f0[i];
                 f0[i] = f1;
                 en = A.x * e0 + A.y * dHy - A.y * dHx + A.z * f1 + A.w * fo - B.x * jp[i];
-                const float jn = B.y * jp[i] + B.z * (en - e0 + f1 - fo);
-                jp[i] = (XS || YS) ? (eok ? jn : 0.f) : jn;
+                if (debye) {  // wave-uniform
+                    const float jn = B.y * jp[i] + B.z * (en - e0 + f1 - fo);
+                    jp[i] = (XS || YS) ? (eok ? jn : 0.f) : jn;
+                }
             } else {
                 const float u = A.y * dHy;
                 const float v = e0 + u;
