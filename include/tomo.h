@@ -144,12 +144,13 @@ const char *tomo_last_error(void);
  * at least 64 x 32 nodes, whose block depth and tile shape the library picks
  * for the chunk, else row sweeps under the schedule's own fields).  A context
  * whose caller has chosen no form, and reference-compatible simulations under
- * any, take the register tiles too;
+ * any (on grids large enough), take the register tiles too;
  * edge_rows: output rows per corner and row-edge tile (the latency-critical
  * boundary tiles; at most seg_rows). */
 #define TOMO_FORM_STREAMS 1
 #define TOMO_FORM_FUSED 2
-/* TOMO_FORM_RESIDENT (physical mode): one cooperative launch per DFT chunk in which each
+/* TOMO_FORM_RESIDENT (physical mode, and reference-compatible grids too small
+ * for register tiles): one cooperative launch per DFT chunk in which each
  * workgroup keeps one tile of a simulation (a 64-lane band, seg_rows rows per
  * wave, 8 waves) in registers through every time block, exchanging only a
  * T-deep frame with its neighbours; seg_rows 8 or 12, tsteps 2, 4 or 8.  Runs
@@ -171,9 +172,9 @@ typedef struct tomo_schedule {
 } tomo_schedule;
 int tomo_set_schedule(tomo_ctx *ctx, const tomo_schedule *s);
 int tomo_get_schedule(tomo_ctx *ctx, tomo_schedule *s);
-/* The schedule the FDTD_GPU / FDTD_CPU shims install on their context.  Of its
- * fields the reference-compatible simulations (register tiles under every form)
- * take the 64-step DFT chunk.  The chunk sets the FP32 partial sums of the
+/* The schedule the FDTD_GPU / FDTD_CPU shims install on their context.  The
+ * reference's own grids run register tiles, which take the 64-step DFT chunk of
+ * it; reference-compatible grids under 64 columns run the resident form.  The chunk sets the FP32 partial sums of the
  * running DFT, so contexts compare bit for bit only under equal chunks. */
 #define TOMO_DROPIN_SCHEDULE {8, 12, 1, 1, 64, 16, TOMO_FORM_RESIDENT, 1, 0}
 

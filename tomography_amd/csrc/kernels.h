@@ -73,8 +73,8 @@ hipError_t launch_rtile(int mode, int waves, const RegTile* tiles, int ntiles, c
 constexpr int kResidentWaves = 8;  // waves per workgroup of the resident kernel
 bool tres_supported(int T, int rows_per_wave);
 // Tiles one cooperative launch can hold on `cus` compute units (0: none).
-int tres_max_tiles(int T, int rows_per_wave, int cus);
-hipError_t launch_tres(int T, int rows_per_wave, const ResTile* tiles, int ntiles,
+int tres_max_tiles(int T, int rows_per_wave, int mode, int cus);
+hipError_t launch_tres(int T, int rows_per_wave, int mode, const ResTile* tiles, int ntiles,
                        const LaunchItem* items, const DevSim* sims, int* done, int* err, int spin_limit,
                        hipStream_t st);
 

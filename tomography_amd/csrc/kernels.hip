@@ -997,7 +997,7 @@ struct RCell {
     int mat;
 };
 
-template <int T, int RW>
+template <int T, int RW, int MODE>
 __global__ __launch_bounds__(kResWaves * kWave, 1) void k_tres(const ResTile* __restrict__ tiles,
                                                               const LaunchItem* __restrict__ items,
                                                               const DevSim* __restrict__ sims, int* done,
@@ -1015,7 +1015,17 @@ __global__ __launch_bounds__(kResWaves * kWave, 1) void k_tres(const ResTile* __
     const DevSim* Sp = sims + it.sim;
     const int lane = threadIdx.x & (kWave - 1);
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);  // wave-uniform
-    fill_edge<T, false>(Sp, lc4, lcp, nullptr);
+    if constexpr (MODE == TOMO_MODE_PHYSICAL) {
+        fill_edge<T, false>(Sp, lc4, lcp, nullptr);
+    } else {
+        // the reference's tables as they are (its stage divides by kappa)
+        float* lcf = (float*)lc4;
+        for (int i = threadIdx.x; i < Sp->nmat * TOMO_NCOEF; i += blockDim.x) lcf[i] = Sp->coef[i];
+        for (int i = threadIdx.x; i < Sp->nc; i += blockDim.x) {
+            CP(0, i) = Sp->ke[i]; CP(1, i) = Sp->km[i]; CP(2, i) = Sp->ike[i]; CP(3, i) = Sp->ikm[i];
+            CP(4, i) = Sp->ae[i]; CP(5, i) = Sp->be[i]; CP(6, i) = Sp->am[i]; CP(7, i) = Sp->bm[i];
+        }
+    }
     if (threadIdx.x == 0) s_abort = 0;
     __syncthreads();
     SimView S;
@@ -1025,7 +1035,9 @@ __global__ __launch_bounds__(kResWaves * kWave, 1) void k_tres(const ResTile* __
     S.nx = Sp->nx; S.ny = Sp->ny; S.pitch = Sp->pitch; S.nc = Sp->nc; S.D = Sp->D; S.P = Sp->P;
     S.L1 = Sp->L1; S.L2 = Sp->L2; S.L3 = Sp->L3; S.cx_hi = Sp->cx_hi; S.cy_lo = Sp->cy_lo;
     S.sx = Sp->sx; S.sy = Sp->sy; S.flags = Sp->flags; S.K = Sp->srows;
-    S.chx = Sp->chx; S.chy = Sp->chy; S.dxf = Sp->dxf; S.dyf = Sp->dyf;
+    S.chx = Sp->chx; S.chy = Sp->chy; S.chx_d = Sp->chx_d; S.chy_d = Sp->chy_d; S.dxf = Sp->dxf; S.dyf = Sp->dyf;
+    S.inc_dt = Sp->inc_dt; S.inc_c = Sp->inc_c; S.inc_ax = Sp->inc_ax; S.inc_ay = Sp->inc_ay;
+    S.inc_itau = Sp->inc_itau; S.inc_abs = Sp->inc_abs_origin;
     const int nx = S.nx, ny = S.ny, nc = S.nc, D = S.D;
     const int x0 = tile.x0 - T;  // first lane's column
     const int x = x0 + lane;
@@ -1037,8 +1049,8 @@ __global__ __launch_bounds__(kResWaves * kWave, 1) void k_tres(const ResTile* __
     wf.xs = (x0 <= nc) || (x0 + kWave - 1 >= nx - nc);
     wf.ccol = (x0 <= D + 1 && x0 + kWave - 1 >= D) || (x0 <= nx - D && x0 + kWave - 1 >= nx - D - 1);
     wf.src = (S.sx >= x0 && S.sx <= x0 + kWave - 1);
-    ResLane L;
-    {
+    ResLane L{};
+    if constexpr (MODE == TOMO_MODE_PHYSICAL) {
         const int ixe = (x >= 1 && x <= nc) ? nc - x : ((x >= nx - nc && x <= nx - 1) ? x - nx + nc : ID);
         const int ixh = (x >= 0 && x < nc) ? nc - 1 - x : ((x >= nx - nc && x < nx) ? x - nx + nc : ID);
         L.kxe = CP(2, ixe); L.axe = CP(4, ixe); L.bxe = CP(5, ixe);
@@ -1053,7 +1065,7 @@ __global__ __launch_bounds__(kResWaves * kWave, 1) void k_tres(const ResTile* __
     // Yee/Debye stage; the others the general one with psi in LDS.
     const int cbot = max(nc, D + 1) + 1, ctop = min(ny - nc, ny - D - 1) - 1;
     const int cl = max(nc, D + 1) + 1, cr = min(nx - nc, nx - D - 1) - 1;
-    const bool clean = yb >= cbot && yb + RW - 1 <= ctop && x0 >= cl &&
+    const bool clean = MODE == TOMO_MODE_PHYSICAL && yb >= cbot && yb + RW - 1 <= ctop && x0 >= cl &&
                        x0 + kWave - 1 <= cr;
     const int nblocks = (it.nsteps + T - 1) / T;
     RCell rows[RW];
@@ -1137,7 +1149,8 @@ __global__ __launch_bounds__(kResWaves * kWave, 1) void k_tres(const ResTile* __
                 int yt = __builtin_amdgcn_readfirstlane(yb + RW - 1);
                 asm volatile("" : "+s"(yt));
                 Cell tc = get(RW - 1);
-                res_h(S, lcp, L, tc, ez_top, yt, htx, hty);
+                if constexpr (MODE == TOMO_MODE_PHYSICAL) res_h(S, lcp, L, tc, ez_top, yt, htx, hty);
+                else stage_h<MODE>(S, lcp, wf, tc, ez_top, x, yt, htx, hty);
                 psi[(RW - 1) * kWave] = make_float4(tc.pex, tc.phx, tc.pey, tc.phy);
             }
             hxt[wv][lane] = htx;
@@ -1180,8 +1193,13 @@ __global__ __launch_bounds__(kResWaves * kWave, 1) void k_tres(const ResTile* __
                     Cell c = get(i);
                     asm volatile("" : "+v"(c.mat));
                     float hx = htx, hy = hty;
-                    if (i + 1 < RW) res_h(S, lcp, L, c, rows[i + 1].ez, y, hx, hy);
-                    res_e(S, lc4, lcp, L, c, hx, hy, hxp, y, x, n, wf.src);
+                    if constexpr (MODE == TOMO_MODE_PHYSICAL) {
+                        if (i + 1 < RW) res_h(S, lcp, L, c, rows[i + 1].ez, y, hx, hy);
+                        res_e(S, lc4, lcp, L, c, hx, hy, hxp, y, x, n, wf.src);
+                    } else {
+                        if (i + 1 < RW) stage_h<MODE>(S, lcp, wf, c, rows[i + 1].ez, x, y, hx, hy);
+                        stage_e<MODE>(S, lc4, lcp, wf, c, hx, hy, hxp, x, y, n);
+                    }
                     put(i, c);
                     if (y >= y0 && y < y1 && xown) write_samples(S, wf, c, x, y, k0 + t);
                 }
@@ -2563,26 +2581,32 @@ bool tres_supported(int T, int rows_per_wave) {
     return (T == 2 || T == 4 || T == 8) && (rows_per_wave == 8 || rows_per_wave == 12);
 }
 
-static const void* tres_kernel(int T, int RW) {
+template <int T, int RW>
+static const void* tres_fn(int mode) {
+    return mode == TOMO_MODE_PHYSICAL ? reinterpret_cast<const void*>(&k_tres<T, RW, TOMO_MODE_PHYSICAL>)
+                                      : reinterpret_cast<const void*>(&k_tres<T, RW, TOMO_MODE_REF_COMPAT>);
+}
+
+static const void* tres_kernel(int T, int RW, int mode) {
 #define TR(TT, RR) \
-    if (T == TT && RW == RR) return reinterpret_cast<const void*>(&k_tres<TT, RR>);
+    if (T == TT && RW == RR) return tres_fn<TT, RR>(mode);
     TR(2, 8) TR(2, 12) TR(4, 8) TR(4, 12) TR(8, 8) TR(8, 12)
 #undef TR
     return nullptr;
 }
 
-int tres_max_tiles(int T, int rows_per_wave, int cus) {
-    const void* f = tres_kernel(T, rows_per_wave);
+int tres_max_tiles(int T, int rows_per_wave, int mode, int cus) {
+    const void* f = tres_kernel(T, rows_per_wave, mode);
     if (!f) return 0;
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, kResWaves * kWave, 0) != hipSuccess) return 0;
     return per_cu * cus;
 }
 
-hipError_t launch_tres(int T, int rows_per_wave, const ResTile* tiles, int ntiles,
+hipError_t launch_tres(int T, int rows_per_wave, int mode, const ResTile* tiles, int ntiles,
                        const LaunchItem* items, const DevSim* sims, int* done, int* err, int spin_limit,
                        hipStream_t st) {
-    const void* f = tres_kernel(T, rows_per_wave);
+    const void* f = tres_kernel(T, rows_per_wave, mode);
     if (!f) return hipErrorInvalidValue;
     t_start = t_stop = nullptr;  // a cooperative launch carries no events
     void* args[] = {(void*)&tiles, (void*)&items, (void*)&sims, (void*)&done, (void*)&err, (void*)&spin_limit};

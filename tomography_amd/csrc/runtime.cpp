@@ -1035,11 +1035,15 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st, bool toge
             std::vector<RegTile> trg;
             if (rebuild) {
                 // resident form: every tile of the set in one cooperative launch,
-                // when they fit on the device at once (else the fused form runs)
-                if (c->form == TOMO_FORM_RESIDENT && mode == TOMO_MODE_PHYSICAL && tres_supported(T, S) && !st.fixed &&
-                    !c->res_refused) {
+                // when they fit on the device at once (else the fused form runs).
+                // Reference-compatible simulations take it on grids too small
+                // for register tiles (512 steps of 40^2 under the drop-in's
+                // schedule: 4 excitations in turn 32 ms against the row sweep's
+                // 59, four vectors together 9 against 15).
+                if (c->form == TOMO_FORM_RESIDENT && tres_supported(T, S) && !st.fixed && !c->res_refused &&
+                    (mode == TOMO_MODE_PHYSICAL || !plan_reg_tiles(ms, K).T)) {
                     for (size_t i = 0; i < ms.size(); ++i) build_res_tiles(ms[i], (int)i, T, S, trs);
-                    if ((int)trs.size() > tres_max_tiles(T, S, c->cus)) trs.clear();
+                    if ((int)trs.size() > tres_max_tiles(T, S, mode, c->cus)) trs.clear();
                 }
                 // Register tiles wherever the grids allow them (64 columns and 32
                 // rows at least): reference-compatible simulations, the fused form,
@@ -1049,7 +1053,7 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st, bool toge
                 // schedule keeps that form's four kernels, as its name says.
                 const bool streams_alone = c->form == TOMO_FORM_STREAMS && c->form_set && !together;
                 st.plan = TilePlan{};
-                if (mode != TOMO_MODE_PHYSICAL || (!wave && trs.empty() && !streams_alone))
+                if (trs.empty() && (mode != TOMO_MODE_PHYSICAL || (!wave && !streams_alone)))
                     st.plan = plan_reg_tiles(ms, K);
                 if (st.plan.T) {
                     for (size_t i = 0; i < ms.size(); ++i) build_reg_tiles(ms[i], (int)i, st.plan, trg);
@@ -1192,7 +1196,7 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st, bool toge
                     HIPCHK(launch_zero(st.d_flags, (sizeof(int) * st.nres + 15) & ~(size_t)15, c->stream));
                     hipEvent_t a = c->prof ? pool_event(c) : nullptr, b = c->prof ? pool_event(c) : nullptr;
                     if (a && b) HIPCHK(hipEventRecord(a, c->stream));
-                    const hipError_t le = launch_tres(T, S, st.d_res, st.nres, d_it, st.d_sims, st.d_flags,
+                    const hipError_t le = launch_tres(T, S, mode, st.d_res, st.nres, d_it, st.d_sims, st.d_flags,
                                                       res_err(st), kResSpinLimit, c->stream);
                     if (le == hipSuccess) {
                         if (a && b) {
