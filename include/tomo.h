@@ -181,7 +181,10 @@ int tomo_get_schedule(tomo_ctx *ctx, tomo_schedule *s);
 /* Autotuner: time candidate schedules on n_sims resident simulations of
  * `cfg` (coordinate descent over form, tsteps, seg_rows, inner_rows,
  * edge_rows, edge/inner waves and grid_mult; the chunk is kept), install the fastest and return it with its
- * measured update rate in cell-steps per second. */
+ * measured update rate in cell-steps per second.  Register tiles take nothing
+ * but the chunk from a schedule: where they win, the fields are left as they
+ * are (or as the first candidate that led to them) and the form is
+ * TOMO_FORM_FUSED, under which any number of simulations takes them. */
 int tomo_autotune(tomo_ctx *ctx, const tomo_sim_config *cfg, int n_sims, tomo_schedule *best,
                   double *cell_steps_per_s);
 

@@ -1,0 +1,72 @@
+"""The autotuner where register tiles carry the launches: they depend on the
+DFT chunk and the grids alone, so nothing but the form is left to choose, and a
+context that took its advice runs no simulation on slower kernels than one that
+asked for none."""
+import numpy as np
+import pytest
+
+import tomography_amd as t
+from cases import PHYS_PARAMS, phys_small, ref_params, ref_small
+
+SWEEPS = ("k_tblock", "k_tedge", "k_trow", "k_tcol", "k_tinner")
+
+
+def lone_launches(c, cfg, p):
+    c.profile(True)
+    g = c.sim(cfg, p)
+    g.step(64)
+    g.close()
+    st = c.stats()
+    c.profile(False)
+    return {k: v["launches"] for k, v in st.items() if k.startswith("k_t") and v["launches"]}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_sims", [1, 2])
+@pytest.mark.parametrize("before", [{}, dict(form=t.FORM_FUSED, tsteps=2, seg_rows=9)])
+def test_register_tiles_leave_only_the_form_to_choose(n_sims, before):
+    cfg = phys_small(steps=64, n=128)
+    with t.Context() as c:
+        if before:
+            c.set_schedule(**before)
+        old = c.schedule()
+        sched, rate = c.autotune(cfg, n_sims)
+        assert rate > 0 and c.schedule() == sched
+        assert sched == old[:6] + (t.FORM_FUSED,) + old[7:]
+        assert set(lone_launches(c, cfg, PHYS_PARAMS)) == {"k_tfused"}
+    with t.Context() as c:  # and so does a context that installs the answer
+        c.set_schedule(**dict(zip(("tsteps", "seg_rows", "edge_waves", "inner_waves", "chunk", "grid_mult", "form",
+                                   "edge_rows", "inner_rows"), sched)))
+        assert set(lone_launches(c, cfg, PHYS_PARAMS)) == {"k_tfused"}
+
+
+@pytest.mark.gpu
+def test_an_installed_streams_form_is_tuned_away_from():
+    """One simulation under an installed streams schedule runs the row sweeps;
+    register tiles, several times faster, win the comparison."""
+    cfg = phys_small(steps=64, n=256)
+    with t.Context() as c:
+        c.set_schedule(tsteps=4, seg_rows=16, edge_waves=2, chunk=32, form=t.FORM_STREAMS)
+        assert "k_tfused" not in lone_launches(c, cfg, PHYS_PARAMS)
+        assert c.autotune(cfg, 1)[0][6] == t.FORM_FUSED
+        assert set(lone_launches(c, cfg, PHYS_PARAMS)) == {"k_tfused"}
+
+
+@pytest.mark.gpu
+def test_reference_grids_of_register_tiles_keep_their_schedule():
+    cfg = ref_small(steps=64, n=101)
+    with t.Context() as c:
+        old = c.schedule()
+        sched, rate = c.autotune(cfg, 2)
+        assert rate > 0 and sched == old == c.schedule()
+        assert set(lone_launches(c, phys_small(steps=64, n=128), PHYS_PARAMS)) == {"k_tfused"}
+
+
+@pytest.mark.gpu
+def test_small_grids_are_still_tuned():
+    cfg = phys_small(steps=64, n=48, n_exc=1).copy(breast_radius=0.006, skin_thickness=0.001, src_radius=0.008)
+    with t.Context() as c:
+        sched, rate = c.autotune(cfg, 1)
+        assert rate > 0 and c.schedule() == sched
+        ran = lone_launches(c, cfg, PHYS_PARAMS)
+        assert any(k in SWEEPS for k in ran) or "k_tfused" in ran

@@ -877,6 +877,16 @@ TilePlan plan_reg_tiles(const std::vector<Slot*>& ms, int K) {
     return p;
 }
 
+// Whether simulations take register tiles, where their grids allow them (64
+// columns and 32 rows at least), under the context's streams or fused form:
+// reference-compatible ones, the fused form, and the streams form for
+// simulations that advance together (64 of 512^2: 83.5 ms against 174 on four
+// streams; 64 of 128^2: 3.0 against 21).  One simulation by itself under an
+// installed streams schedule keeps that form's four kernels, as its name says.
+bool form_takes_tiles(const tomo_ctx* c, int mode, bool together) {
+    return mode != TOMO_MODE_PHYSICAL || !(c->form == TOMO_FORM_STREAMS && c->form_set && !together);
+}
+
 // Order of the register tiles.  The kernel deals the list to the eight XCDs in
 // contiguous eighths (update_tile.hip), one tile after the other as compute
 // units come free, so the order decides which tiles share a unit and which
@@ -1045,16 +1055,8 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st, bool toge
                     for (size_t i = 0; i < ms.size(); ++i) build_res_tiles(ms[i], (int)i, T, S, trs);
                     if ((int)trs.size() > tres_max_tiles(T, S, mode, c->cus)) trs.clear();
                 }
-                // Register tiles wherever the grids allow them (64 columns and 32
-                // rows at least): reference-compatible simulations, the fused form,
-                // and the streams form for simulations that advance together (64 of
-                // 512^2: 83.5 ms against 174 on four streams; 64 of 128^2: 3.0
-                // against 21).  One simulation by itself under an installed streams
-                // schedule keeps that form's four kernels, as its name says.
-                const bool streams_alone = c->form == TOMO_FORM_STREAMS && c->form_set && !together;
                 st.plan = TilePlan{};
-                if (trs.empty() && (mode != TOMO_MODE_PHYSICAL || (!wave && !streams_alone)))
-                    st.plan = plan_reg_tiles(ms, K);
+                if (trs.empty() && !wave && form_takes_tiles(c, mode, together)) st.plan = plan_reg_tiles(ms, K);
                 if (st.plan.T) {
                     for (size_t i = 0; i < ms.size(); ++i) build_reg_tiles(ms[i], (int)i, st.plan, trg);
                     if (st.plan.T) order_tiles(ms, st.plan.waves, c->cus, trg);
@@ -1987,7 +1989,8 @@ int tomo_get_schedule(tomo_ctx* c, tomo_schedule* s) {
     return TOMO_OK;
 }
 
-// Seconds for `epochs` epochs of the resident slots under the current schedule.
+// Seconds for `epochs` epochs of the resident slots under the current schedule,
+// run in one call as an evaluation runs them.
 static int time_epochs(tomo_ctx* c, std::vector<Slot*>& sl, int epochs, double* secs) {
     hipEvent_t a = pool_event(c), b = pool_event(c);
     if (!a || !b) return fail(TOMO_E_HIP, "event");
@@ -1995,11 +1998,9 @@ static int time_epochs(tomo_ctx* c, std::vector<Slot*>& sl, int epochs, double* 
     int rc = run_epochs(c, sl, stage(c), sl.size() > 1);  // untimed: rebuilds and uploads the tile list
     if (rc) return rc;
     HIPCHK(hipEventRecord(a, c->stream));
-    for (int e = 0; e < epochs; ++e) {
-        for (Slot* s : sl) s->target = std::min(s->su.cfg.steps, s->done + c->K);
-        rc = run_epochs(c, sl, stage(c), sl.size() > 1);
-        if (rc) return rc;
-    }
+    for (Slot* s : sl) s->target = std::min(s->su.cfg.steps, s->done + c->K * epochs);
+    rc = run_epochs(c, sl, stage(c), sl.size() > 1);
+    if (rc) return rc;
     HIPCHK(hipEventRecord(b, c->stream));
     HIPCHK(hipEventSynchronize(b));
     float ms = 0;
@@ -2028,10 +2029,10 @@ int tomo_autotune(tomo_ctx* c, const tomo_sim_config* cfg, int n_sims, tomo_sche
     int rc = TOMO_OK;
     for (int i = 0; i < n_sims && !rc; ++i) {
         Slot* s = nullptr;
-        rc = slot_create(c, tc, p.data(), p.size(), i % tc.n_exc, 0, &s);
+        rc = slot_create(c, tc, p.data(), p.size(), i % tc.n_exc, n_sims - i, &s);
         if (!rc) sl.push_back(s);
     }
-    const bool prof = c->prof;
+    const bool prof = c->prof, was_set = c->form_set;
     c->prof = false;
     tomo_schedule cur{c->T, c->S, c->W, c->Wi, c->K, c->grid_mult, c->form, c->ER, c->Si};
     // each trial times at least 512 steps: a few launches alone are dominated
@@ -2039,17 +2040,29 @@ int tomo_autotune(tomo_ctx* c, const tomo_sim_config* cfg, int n_sims, tomo_sche
     const int epochs = std::max(2, (512 + c->K - 1) / c->K);
     double cells = 0;
     for (Slot* s : sl) cells += (double)s->d.nx * s->d.ny * c->K * epochs;
+    const tomo_schedule was = cur;
+    const bool together = n_sims > 1, fits = !rc && plan_reg_tiles(sl, c->K).T > 0;
     double best_t = 1e30;
-    auto trial = [&](const tomo_schedule& cand) -> int {
+    // Register tiles follow from the chunk and the grids alone: every schedule
+    // that leads to them makes the same launches.  They are timed once, so that
+    // they compete with the other forms but not, by noise, with themselves.
+    bool tiles_timed = false, best_tiles = false, best_set = true;
+    auto trial = [&](const tomo_schedule& cand, bool form_set = true) -> int {
         int r = set_schedule_locked(c, cand);
         if (r) return r;
+        c->form_set = form_set;
+        if (tiles_timed && fits && form_takes_tiles(c, tc.mode, together) &&
+            (tc.mode != TOMO_MODE_PHYSICAL || cand.form == TOMO_FORM_STREAMS || cand.form == TOMO_FORM_FUSED))
+            return TOMO_OK;
         double t = 0;
         r = time_epochs(c, sl, epochs, &t);
         if (r) return r;
-        if (t < best_t) { best_t = t; cur = cand; }
+        const bool tiles = c->stg.plan.T > 0;
+        if (t < best_t && !(tiles && tiles_timed)) { best_t = t; best_tiles = tiles; best_set = form_set; cur = cand; }
+        tiles_timed = tiles_timed || tiles;
         return TOMO_OK;
     };
-    if (!rc) rc = trial(cur);
+    if (!rc) rc = trial(cur, was_set);
     // Seeds measured on MI355X, so that the descent does not start from a
     // poor corner of the space: one simulation (fused, short tiles) and many
     // (four streams, tall tiles; T = 6 where the chunk allows it).
@@ -2074,7 +2087,14 @@ int tomo_autotune(tomo_ctx* c, const tomo_sim_config* cfg, int n_sims, tomo_sche
         for (int v : Ws) { tomo_schedule x = cur; x.inner_waves = v; if (!rc) rc = trial(x); }
         for (int v : Gs) { tomo_schedule x = cur; x.grid_mult = v; if (!rc) rc = trial(x); }
     }
+    // where register tiles won, the form that gives them to any number of simulations
+    if (best_tiles && tc.mode == TOMO_MODE_PHYSICAL) {
+        cur.form = TOMO_FORM_FUSED;
+        best_set = true;
+    }
     if (!rc) rc = set_schedule_locked(c, cur);
+    if (rc) (void)set_schedule_locked(c, was);
+    c->form_set = rc ? was_set : best_set;
     c->prof = prof;
     for (Slot* s : sl) slot_destroy(c, s);
     c->stg.tile_key.clear();
