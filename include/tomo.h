@@ -170,6 +170,8 @@ typedef struct tomo_schedule {
      * (which then sets the column-edge and the interior tiles alike). */
     int32_t inner_rows;
 } tomo_schedule;
+/* Installing the schedule that tomo_get_schedule returned changes nothing: a
+ * context whose caller has chosen no form keeps none. */
 int tomo_set_schedule(tomo_ctx *ctx, const tomo_schedule *s);
 int tomo_get_schedule(tomo_ctx *ctx, tomo_schedule *s);
 /* The schedule the FDTD_GPU / FDTD_CPU shims install on their context.  The

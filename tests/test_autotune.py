@@ -2,11 +2,11 @@
 DFT chunk and the grids alone, so nothing but the form is left to choose, and a
 context that took its advice runs no simulation on slower kernels than one that
 asked for none."""
-import numpy as np
 import pytest
 
 import tomography_amd as t
-from cases import PHYS_PARAMS, phys_small, ref_params, ref_small
+from cases import PHYS_PARAMS, phys_small, ref_small
+from tomography_amd.workloads import SCHED_KEYS
 
 SWEEPS = ("k_tblock", "k_tedge", "k_trow", "k_tcol", "k_tinner")
 
@@ -35,15 +35,14 @@ def test_register_tiles_leave_only_the_form_to_choose(n_sims, before):
         assert sched == old[:6] + (t.FORM_FUSED,) + old[7:]
         assert set(lone_launches(c, cfg, PHYS_PARAMS)) == {"k_tfused"}
     with t.Context() as c:  # and so does a context that installs the answer
-        c.set_schedule(**dict(zip(("tsteps", "seg_rows", "edge_waves", "inner_waves", "chunk", "grid_mult", "form",
-                                   "edge_rows", "inner_rows"), sched)))
+        c.set_schedule(**dict(zip(SCHED_KEYS, sched)))
         assert set(lone_launches(c, cfg, PHYS_PARAMS)) == {"k_tfused"}
 
 
 @pytest.mark.gpu
 def test_an_installed_streams_form_is_tuned_away_from():
     """One simulation under an installed streams schedule runs the row sweeps;
-    register tiles, several times faster, win the comparison."""
+    register tiles, more than ten times faster, win the comparison."""
     cfg = phys_small(steps=64, n=256)
     with t.Context() as c:
         c.set_schedule(tsteps=4, seg_rows=16, edge_waves=2, chunk=32, form=t.FORM_STREAMS)
@@ -70,3 +69,20 @@ def test_small_grids_are_still_tuned():
         assert rate > 0 and c.schedule() == sched
         ran = lone_launches(c, cfg, PHYS_PARAMS)
         assert any(k in SWEEPS for k in ran) or "k_tfused" in ran
+
+
+@pytest.mark.gpu
+def test_a_schedule_put_back_changes_nothing():
+    """The schedule read from a context that chose no form, installed again, is
+    no choice of the streams form; naming that form is one."""
+    cfg = phys_small(steps=64, n=128)
+    with t.Context() as c:
+        old = c.schedule()
+        c.set_schedule(**dict(zip(SCHED_KEYS, old)))
+        assert c.schedule() == old
+        assert set(lone_launches(c, cfg, PHYS_PARAMS)) == {"k_tfused"}
+        c.set_schedule(form=t.FORM_STREAMS)
+        assert c.schedule() == old
+        assert "k_tfused" not in lone_launches(c, cfg, PHYS_PARAMS)
+        c.set_schedule(**dict(zip(SCHED_KEYS, old)))
+        assert "k_tfused" not in lone_launches(c, cfg, PHYS_PARAMS)

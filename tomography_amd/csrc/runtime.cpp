@@ -1954,7 +1954,14 @@ int tomo_ctx_destroy(tomo_ctx* c) {
     return TOMO_OK;
 }
 
+static tomo_schedule schedule_of(const tomo_ctx* c) {
+    return {c->T, c->S, c->W, c->Wi, c->K, c->grid_mult, c->form, c->ER, c->Si};
+}
+
 static int set_schedule_locked(tomo_ctx* c, const tomo_schedule& s) {
+    // the schedule that tomo_get_schedule gave out: not a choice of a form
+    const tomo_schedule now = schedule_of(c);
+    if (!std::memcmp(&s, &now, sizeof(s))) return TOMO_OK;
     const int T = s.tsteps ? s.tsteps : c->T, S = s.seg_rows ? s.seg_rows : c->S;
     const int W = s.edge_waves ? s.edge_waves : c->W, Wi = s.inner_waves ? s.inner_waves : c->Wi;
     const int K = s.chunk ? s.chunk : c->K, G = s.grid_mult ? s.grid_mult : c->grid_mult;
@@ -1983,9 +1990,7 @@ int tomo_set_schedule(tomo_ctx* c, const tomo_schedule* s) {
 
 int tomo_get_schedule(tomo_ctx* c, tomo_schedule* s) {
     if (!c || !s) return fail(TOMO_E_INVALID, "null argument");
-    s->tsteps = c->T; s->seg_rows = c->S; s->edge_waves = c->W; s->inner_waves = c->Wi;
-    s->chunk = c->K; s->grid_mult = c->grid_mult; s->form = c->form; s->edge_rows = c->ER;
-    s->inner_rows = c->Si;
+    *s = schedule_of(c);
     return TOMO_OK;
 }
 
@@ -2034,7 +2039,7 @@ int tomo_autotune(tomo_ctx* c, const tomo_sim_config* cfg, int n_sims, tomo_sche
     }
     const bool prof = c->prof, was_set = c->form_set;
     c->prof = false;
-    tomo_schedule cur{c->T, c->S, c->W, c->Wi, c->K, c->grid_mult, c->form, c->ER, c->Si};
+    tomo_schedule cur = schedule_of(c);
     // each trial times at least 512 steps: a few launches alone are dominated
     // by first-launch and dispatch effects
     const int epochs = std::max(2, (512 + c->K - 1) / c->K);
