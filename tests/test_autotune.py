@@ -1,7 +1,7 @@
-"""The autotuner where register tiles carry the launches: they depend on the
-DFT chunk and the grids alone, so nothing but the form is left to choose, and a
-context that took its advice runs no simulation on slower kernels than one that
-asked for none."""
+"""The autotuner, and schedules put back or changed, where register tiles carry
+the launches: they depend on the DFT chunk and the grids alone, so nothing but
+the form is left to choose, and a context that took the autotuner's advice runs
+no simulation on slower kernels than one that asked for none."""
 import pytest
 
 import tomography_amd as t
@@ -86,3 +86,24 @@ def test_a_schedule_put_back_changes_nothing():
         assert "k_tfused" not in lone_launches(c, cfg, PHYS_PARAMS)
         c.set_schedule(**dict(zip(SCHED_KEYS, old)))
         assert "k_tfused" not in lone_launches(c, cfg, PHYS_PARAMS)
+
+
+@pytest.mark.gpu
+def test_a_form_chosen_for_a_live_simulation_takes_effect():
+    """A simulation on register tiles whose context then chooses the streams
+    form advances by that form's kernels, and back."""
+    cfg = phys_small(steps=200, n=128)
+    with t.Context() as c:
+        g = c.sim(cfg, PHYS_PARAMS)
+
+        def ran():
+            c.profile(True)
+            g.step(32)
+            return {k for k, v in c.stats().items() if k.startswith("k_t") and v["launches"]}
+
+        assert ran() == {"k_tfused"}
+        c.set_schedule(form=t.FORM_STREAMS)
+        assert "k_tfused" not in ran()
+        c.set_schedule(form=t.FORM_FUSED)
+        assert ran() == {"k_tfused"}
+        g.close()

@@ -132,7 +132,7 @@ struct Staging {
     int res_cap = 0, nres = 0;
     int* d_flags = nullptr;  // res_cap counters, then the error word (res_err)
     int res_key_form = 0;    // form the tile lists were built for
-    bool key_together = false;
+    bool key_together = false, key_form_set = false;
     TilePlan plan;           // register tiles of the list (T == 0: none)
 };
 }  // namespace
@@ -1037,7 +1037,8 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st, bool toge
             for (Slot* s : ms) key.push_back(s->serial);
             const bool rebuild = key != st.tile_key || st.key_T != T || st.key_S != S || st.key_W != W ||
                                  st.key_Wi != c->Wi || st.key_ER != c->ER || st.key_Si != c->Si ||
-                                 st.res_key_form != c->form || st.key_together != together;
+                                 st.res_key_form != c->form || st.key_form_set != c->form_set ||
+                                 st.key_together != together;
             // tile form: whole register tiles, one workgroup each, in place of the four classes
             const bool wave = c->form == TOMO_FORM_TILE && mode == TOMO_MODE_PHYSICAL && twave_supported(T, S);
             std::vector<TileItem> te, tr, tc, tn;
@@ -1139,6 +1140,7 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st, bool toge
                 st.n_rowedge = (int)tr.size();
                 st.res_key_form = c->form;
                 st.key_together = together;
+                st.key_form_set = c->form_set;
                 st.nres = 0;
                 if (!trs.empty()) {
                     rc = ensure_res_staging(c, st, (int)trs.size());
