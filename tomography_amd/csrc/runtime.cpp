@@ -368,19 +368,36 @@ struct Work {
 void slot_destroy(tomo_ctx* c, Slot* s);
 int slot_fill(tomo_ctx* c, Slot* s, DevSim* d_entry);
 
+// Spare sample rows of the simulations, all alike, that one call creates and
+// runs to their end: `groups` groups of `per` are still to be run, as many
+// whole groups at a time as the budget admits.  The first simulation of a pass
+// decides for the pass: the rows are taken where they make no further pass, so
+// that they refuse nothing, and by all or none, since one simulation without
+// them makes every fold of the pass a launch of its own (run_epochs).
+struct SpareRows {
+    size_t groups;
+    int per;
+    int rows = -1;  // undecided
+    void decide(uint64_t room, size_t bytes, size_t bytes_with) {
+        const uint64_t a = room / (bytes * per), b = room / (bytes_with * per);
+        auto passes = [&](uint64_t fit) { return (groups + fit - 1) / fit; };
+        rows = b && passes(b) == passes(a) ? kRoundRows : 0;
+    }
+};
+
 // Build the device-resident simulation for one excitation of one phantom.
-// together > 0: it is the first of that many alike that an evaluation creates
-// and runs within one call; they take spare sample rows where the budget
-// admits all of them with these, so that the rows refuse nothing.  Simulations
-// that outlive a call, or advance an epoch per call, have no use for them.
-int slot_create(tomo_ctx* c, const tomo_sim_config& cfg, const double* p, size_t np, int exc, int together, Slot** out) {
+// spare: null for simulations that outlive a call or advance an epoch per call,
+// which have no use for the rows.
+int slot_create(tomo_ctx* c, const tomo_sim_config& cfg, const double* p, size_t np, int exc, SpareRows* spare, Slot** out) {
     std::unique_ptr<Slot> s(new Slot());
     int rc = build_setup(cfg, p, np, exc, s->su);
     if (rc) return rc;
     const SimSetup& su = s->su;
     if (c->K % c->T) return fail(TOMO_E_INVALID, "chunk must be a multiple of the fused step count");
     s->srows = c->K;
-    if (together > 0 && c->used + together * slot_bytes(su, c->K + kRoundRows) <= c->budget) s->srows += kRoundRows;
+    if (spare && spare->rows < 0)
+        spare->decide(c->budget > c->used ? c->budget - c->used : 0, slot_bytes(su, c->K), slot_bytes(su, c->K + kRoundRows));
+    if (spare) s->srows += spare->rows;
     const size_t bytes = slot_bytes(su, s->srows);
     if (c->used + bytes > c->budget) return fail(TOMO_E_NOMEM, "HBM budget exceeded");
     auto hit = c->cache.find(bytes);
@@ -1510,7 +1527,8 @@ static int eval_many(tomo_ctx* c, const tomo_sim_config& cfg, const double* para
         for (size_t v = 0; v < n_vec && !rc; ++v) {
             for (int e = 0; e < E && !rc; ++e) {
                 Slot* s = nullptr;
-                rc = slot_create(c, cfg, params + v * dim, dim, e, 1, &s);
+                SpareRows spare{1, 1};
+                rc = slot_create(c, cfg, params + v * dim, dim, e, &spare, &s);
                 if (rc) break;
                 std::vector<Slot*> one{s};
                 rc = run_and_project(c, one, dD + v * L + (size_t)e * F * A, dP + v * L + (size_t)e * F * A, false);
@@ -1522,12 +1540,13 @@ static int eval_many(tomo_ctx* c, const tomo_sim_config& cfg, const double* para
         size_t v0 = 0;
         while (v0 < n_vec && !rc) {
             std::vector<Slot*> sl;
+            SpareRows spare{n_vec - v0, E};
             size_t v = v0;
             for (; v < n_vec && !rc; ++v) {
                 std::vector<Slot*> mine;
                 for (int e = 0; e < E; ++e) {
                     Slot* s = nullptr;
-                    int r2 = slot_create(c, cfg, params + v * dim, dim, e, E - e, &s);
+                    int r2 = slot_create(c, cfg, params + v * dim, dim, e, &spare, &s);
                     if (r2) {
                         for (Slot* m : mine) slot_destroy(c, m);
                         if (r2 == TOMO_E_NOMEM && !sl.empty()) goto run_pass;
@@ -1582,9 +1601,10 @@ static int get_target(tomo_ctx* c, const tomo_sim_config& cfg, std::vector<float
     const size_t L = (size_t)cfg.n_exc * cfg.n_freq * cfg.n_angles;
     std::vector<Slot*> sl;
     int rc = TOMO_OK;
+    SpareRows spare{1, cfg.n_exc};
     for (int e = 0; e < cfg.n_exc && !rc; ++e) {
         Slot* s = nullptr;
-        rc = slot_create(c, cfg, tv.data(), tv.size(), e, cfg.n_exc - e, &s);
+        rc = slot_create(c, cfg, tv.data(), tv.size(), e, &spare, &s);
         if (!rc) sl.push_back(s);
     }
     Work w(c);
@@ -1672,7 +1692,7 @@ static int progress_once(tomo_ctx* c, int* n_active) {
         int rc = TOMO_OK;
         for (int e = 0; e < r->cfg.n_exc && !rc; ++e) {
             Slot* s = nullptr;
-            rc = slot_create(c, r->cfg, r->params.data(), r->params.size(), e, 0, &s);
+            rc = slot_create(c, r->cfg, r->params.data(), r->params.size(), e, nullptr, &s);
             if (!rc) { s->req = (long)r->ticket; r->slots.push_back(s); }
         }
         if (rc) {
@@ -2034,9 +2054,10 @@ int tomo_autotune(tomo_ctx* c, const tomo_sim_config* cfg, int n_sims, tomo_sche
     }
     std::vector<Slot*> sl;
     int rc = TOMO_OK;
+    SpareRows spare{1, n_sims};
     for (int i = 0; i < n_sims && !rc; ++i) {
         Slot* s = nullptr;
-        rc = slot_create(c, tc, p.data(), p.size(), i % tc.n_exc, n_sims - i, &s);
+        rc = slot_create(c, tc, p.data(), p.size(), i % tc.n_exc, &spare, &s);
         if (!rc) sl.push_back(s);
     }
     const bool prof = c->prof, was_set = c->form_set;
@@ -2269,7 +2290,7 @@ int tomo_sim_create(tomo_ctx* c, const tomo_sim_config* cfg, const double* param
     if (!c || !cfg || !out) return fail(TOMO_E_INVALID, "null argument");
     std::lock_guard<std::mutex> g(c->mu);
     Slot* s = nullptr;
-    int rc = slot_create(c, *cfg, params, n, exc, 0, &s);
+    int rc = slot_create(c, *cfg, params, n, exc, nullptr, &s);
     if (rc) return rc;
     std::shared_ptr<SimLink> link = std::make_shared<SimLink>();
     link->ctx = c;
