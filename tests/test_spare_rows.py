@@ -17,7 +17,7 @@ def test_rows_make_no_further_pass():
     V[:, 0] += np.arange(6)
     T = np.zeros(cfg.farfield_len(), np.float32)
     one = least_budget(cfg, PHYS_PARAMS) * cfg.n_exc  # of one vector, without the rows (to 8 KiB)
-    rows = 3 * 24 * 4 * cfg.contour_len() * cfg.n_exc
+    rows = 3 * 15 * 4 * cfg.contour_len() * cfg.n_exc
     assert rows < one / 6 and rows > 16 * 8192
     epochs = -(-cfg.steps // CHUNK)
 

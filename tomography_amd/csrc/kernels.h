@@ -45,7 +45,7 @@ bool twave_supported(int T, int rows_per_wave);
 hipError_t launch_twave(int T, int rows_per_wave, const TileItem* tiles, int ntiles, const LaunchItem* items,
                         const DevSim* sims, int ordinal, int grid, hipStream_t st);
 
-// Register-tile update: one workgroup of `waves` (8 or 16) waves per RegTile
+// Register-tile update: one workgroup of `waves` waves (8, or 16 in physical mode) per RegTile
 // advances it one time block of `tsteps` steps.  Every held node is a node of
 // the grid, and the owned nodes lie at least `tsteps` inside the held ones
 // wherever those do not end at the grid's edge.  rows: kTileRowsTall for a tile
@@ -54,6 +54,7 @@ hipError_t launch_twave(int T, int rows_per_wave, const TileItem* tiles, int nti
 // for physical-mode material clear of them and of the source; else
 // kTileRowsEdge.  The six field planes take less than 2 GiB together.
 // A tile of item -1 is an unused place.
+constexpr int kMaxTileSteps = 15;  // longest block that the planner asks for (runtime.cpp)
 constexpr int kTileRowsEdge = 4, kTileRowsClean = 8, kTileRowsTall = 16;
 // `fold`: the previous epoch's items (n of them, FP32 running DFT), whose
 // samples further workgroups of the launch fold; this launch must write other

@@ -65,7 +65,7 @@ struct Slot {
 
 // Sample rows beyond a chunk: the longest block of the register tiles, which
 // writes them while the chunk's own rows are folded (run_epochs).
-constexpr int kRoundRows = 24;
+constexpr int kRoundRows = kMaxTileSteps;
 
 // Bytes one simulation slot with `srows` sample rows occupies on the device.
 size_t slot_bytes(const SimSetup& s, int srows) {
@@ -883,7 +883,7 @@ TilePlan plan_reg_tiles(const std::vector<Slot*>& ms, int K) {
         deep = p.tall ? 10 : nodes < 300000 ? 12 : 6;
     } else if (fit16 && ms.size() > 1 && longest <= 300) {
         p.waves = 16;
-        deep = longest <= 160 ? 15 : 12;
+        deep = longest <= 160 ? kMaxTileSteps : 12;
     } else {
         p.waves = 8;
         p.tall = nodes > 600000;

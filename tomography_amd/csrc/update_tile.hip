@@ -4,7 +4,7 @@
 //
 // A workgroup of NW waves holds 64 columns times NW * R rows, R rows per wave,
 // one column per lane, in registers; it requests them all at once, advances
-// them up to 24 steps and stores the cells it owns.  A step invalidates one
+// them up to 15 steps and stores the cells it owns.  A step invalidates one
 // lane and one row at each edge of the tile that is not the grid's edge, so
 // tiles overlap by twice the block's steps.  Waves couple through LDS: each
 // publishes its bottom and top Ez rows, advances what needs no neighbour (H of
@@ -697,7 +697,7 @@ hipError_t launch_rtile(int mode, int waves, const RegTile* tiles, int ntiles, c
         TIMED_LAUNCH((k_rtile<MM, WW>), g, b, 0, st, tiles, ntiles, items, sims, ordinal, tsteps, lone, fold);  \
         return hipGetLastError();                                                                         \
     }
-    TT(TOMO_MODE_PHYSICAL, 8) TT(TOMO_MODE_PHYSICAL, 16) TT(TOMO_MODE_REF_COMPAT, 8) TT(TOMO_MODE_REF_COMPAT, 16)
+    TT(TOMO_MODE_PHYSICAL, 8) TT(TOMO_MODE_PHYSICAL, 16) TT(TOMO_MODE_REF_COMPAT, 8)
 #undef TT
     return hipErrorInvalidValue;
 }
