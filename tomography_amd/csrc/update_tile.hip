@@ -231,7 +231,9 @@ __device__ __forceinline__ void tile_wave(const RegTile& tile, const DevSim* __r
     const float chx = Sp->chx, chy = Sp->chy, dxf = Sp->dxf, dyf = Sp->dyf, chx_d = Sp->chx_d, chy_d = Sp->chy_d;
     const float cb0 = Sp->coef[1];  // vacuum curl coefficient (the vacuum Ez coefficient is exactly 1)
     const bool clamp = REF && !(Sp->flags & TOMO_FLAG_NO_NAN_CLAMP);
-    const bool debye = !(Sp->flags & TOMO_FLAG_CPU_COEFS);  // the CPU form has no Jp: an infinite Ez must not make one
+    // the CPU form has no Jp: an infinite Ez must not make one (a mask keeps the
+    // stage one basic block; a branch cost the drop-in objective 1%)
+    const unsigned debye = Sp->flags & TOMO_FLAG_CPU_COEFS ? 0u : ~0u;
     const bool ex_ok = !XS || (x >= 1 && x < nx);
     const bool bot = YS && yb == 0, top = YS && yb + R - 1 == ny;  // PEC rows: the wave's first, its last
     Profile<REF> Le, Lh;
@@ -382,10 +384,8 @@ __device__ __forceinline__ void tile_wave(const RegTile& tile, const DevSim* __r
                 const float f1 = expf(-a1 * a1), fo = f0[i];
                 f0[i] = f1;
                 en = A.x * e0 + A.y * dHy - A.y * dHx + A.z * f1 + A.w * fo - B.x * jp[i];
-                if (debye) {  // wave-uniform
-                    const float jn = B.y * jp[i] + B.z * (en - e0 + f1 - fo);
-                    jp[i] = (XS || YS) ? (eok ? jn : 0.f) : jn;
-                }
+                const float jn = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, B.y * jp[i] + B.z * (en - e0 + f1 - fo)) & debye);
+                jp[i] = (XS || YS) ? (eok ? jn : 0.f) : jn;
             } else {
                 const float u = A.y * dHy;
                 const float v = e0 + u;
@@ -595,8 +595,11 @@ struct FoldShare {
 // contiguous eighth of the tile list, so that tiles that share halo rows and
 // columns share an L2 (64 simulations of 512^2: 640 -> 237 MB read per launch,
 // 203 -> 193 us; 4 x 401^2 20.2 -> 17.5 us).
+// Aligned, so that a change to one instance does not move the others: the same
+// instructions 2 KiB further on were 1.3% slower (mixed requests of 362 to 1448,
+// 51.5 -> 52.2 us a launch).
 template <int MODE, int NW>
-__global__ __launch_bounds__(NW* kLane) __attribute__((amdgpu_waves_per_eu(4))) void k_rtile(
+__global__ __launch_bounds__(NW* kLane) __attribute__((amdgpu_waves_per_eu(4), aligned(4096))) void k_rtile(
     const RegTile* __restrict__ tiles, int ntiles, const LaunchItem* __restrict__ items, const DevSim* __restrict__ sims, int ordinal,
     int tsteps, const DevSim* __restrict__ lone, FoldShare fold) {
     __shared__ union {
