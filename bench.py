@@ -60,6 +60,8 @@ def _kernel_roofline(name, k):
     achieved = bpl / avg_s / 1e9
     return {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None, "kernel": name,
+            "counts": "algorithmic bytes of every step; time blocking keeps them on the chip, so frac may pass 1 and "
+                      "traffic_frac is the share of HBM",
             "launches": k["launches"], "avg_launch_us": round(avg_s * 1e6, 2), "alg_bytes_per_launch": bpl,
             "alg_bytes_per_cell_step": round(k["alg_bytes"] / k["cell_steps"], 3) if k["cell_steps"] else None,
             "cell_steps_per_launch": k["cell_steps"] / k["launches"], "total_ms": round(k["ms"], 2)}
@@ -604,6 +606,7 @@ def main():
         add_traffic(rl, traffic_for("plain_cfg2", rl["kernel"], tuple(sched.values())), float(cfg.nx) * cfg.ny)
     out["roofline"] = rl
     out["kernel_ms_per_step"] = kernel_ms(st, args.steps)
+    out["kernel_classes"] = t.api.KERNEL_CLASSES  # what runs under the names of the classes
     bsch = dict(BATCH_SCHEDULE)
     if args.batch_schedule:
         bsch = dict(zip(SCHED_KEYS, [int(x) for x in args.batch_schedule.split(",")]))

@@ -198,15 +198,15 @@ int tomo_autotune(tomo_ctx *ctx, const tomo_sim_config *cfg, int n_sims, tomo_sc
  * (the psi pair).  `update` is the wall time of the whole update phase (all
  * streams, from the first launch of an epoch to the join of its last block). */
 enum {
-    TOMO_KERNEL_GENERAL = 0, /* reference-compatible simulations: register tiles, or k_tblock on small grids */
+    TOMO_KERNEL_GENERAL = 0, /* reference-compatible simulations: k_rtile (register tiles), or k_tblock on small grids */
     TOMO_KERNEL_CORNER = 1,  /* k_tedge: corner tiles (and all tiles of small physical grids) */
     TOMO_KERNEL_ROW = 2,     /* k_trow: top / bottom frame between the corners */
     TOMO_KERNEL_COL = 3,     /* k_tcol: left / right frame between the corners */
     TOMO_KERNEL_INNER = 4,   /* k_tinner: clean interior bands */
     TOMO_KERNEL_FOLD = 5,    /* k_fold: running-DFT fold of a chunk of samples */
-    TOMO_KERNEL_PROJECT = 6, /* k_project_mfma: far-field projection on the matrix cores */
+    TOMO_KERNEL_PROJECT = 6, /* far-field projection: k_project_chain, or k_project_mfma (matrix cores) for many simulations */
     TOMO_KERNEL_FITNESS = 7, /* k_fitness: FP64 fitness reduction */
-    TOMO_KERNEL_FUSED = 8,   /* physical mode, every tile in one launch: register tiles, or k_tfused on small grids */
+    TOMO_KERNEL_FUSED = 8,   /* physical mode, every tile in one launch: k_rtile, or k_tfused where a grid is small */
     TOMO_KERNEL_RESIDENT = 9, /* k_tres: a whole epoch in one cooperative launch (TOMO_FORM_RESIDENT) */
     TOMO_KERNEL_TILE = 10,    /* k_twave: register tiles, one launch per time block (TOMO_FORM_TILE) */
     TOMO_KERNEL_COUNT = 11

@@ -40,8 +40,15 @@ class Schedule(_c.Structure):
         return tuple(getattr(self, k) for k, _ in self._fields_)
 
 
+# Kernel classes of the statistics, each by the name of the kernel that first
+# carried it (KERNEL_CLASSES: what runs in those that several kernels share).
 KERNEL_NAMES = ("k_tblock", "k_tedge", "k_trow", "k_tcol", "k_tinner", "k_fold", "k_project_mfma", "k_fitness",
                 "k_tfused", "k_tres", "k_twave")
+KERNEL_CLASSES = {
+    "k_tblock": "reference-compatible simulations: k_rtile, or k_tblock on grids under 64 columns",
+    "k_tfused": "every tile of physical-mode simulations: k_rtile, or k_tfused where a grid is under 64 x 32 nodes",
+    "k_project_mfma": "far-field projection: k_project_chain, or k_project_mfma for many simulations",
+}
 
 
 class KernelStats(_c.Structure):

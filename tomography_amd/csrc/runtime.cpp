@@ -97,18 +97,17 @@ struct SimLink {
 };
 
 namespace {
-// Launch staging of the epoch runner: launch items and the tile list (host
-// copies and device copies) and the DevSim table the kernels index.  The
-// context's own staging grows on demand (pinned host memory, device memory);
-// a fixed staging lives in caller-provided memory and never grows.
 // Shape of the register tiles of a launch: T steps per block, `waves` waves
 // per tile.  T == 0: the launch takes the row sweeps.
 struct TilePlan {
     int T = 0, waves = 0;
     bool tall = false;  // vacuum tiles of kTileRowsTall rows per wave
-    bool operator==(const TilePlan& o) const { return T == o.T && waves == o.waves && tall == o.tall; }
 };
 
+// Launch staging of the epoch runner: launch items and the tile list (host
+// copies and device copies) and the DevSim table the kernels index.  The
+// context's own staging grows on demand (pinned host memory, device memory);
+// a fixed staging lives in caller-provided memory and never grows.
 struct Staging {
     LaunchItem* h_items = nullptr;
     LaunchItem* d_items = nullptr;
@@ -1079,7 +1078,7 @@ int run_epochs(tomo_ctx* c, const std::vector<Slot*>& sl, Staging& st, bool toge
                     for (size_t i = 0; i < ms.size(); ++i) build_reg_tiles(ms[i], (int)i, st.plan, trg);
                     if (st.plan.T) order_tiles(ms, st.plan.waves, c->cus, trg);
                     if (st.fixed && trg.size() * sizeof(RegTile) > st.tiles_cap * sizeof(TileItem)) {
-                        st.plan = TilePlan{};  // the row sweeps' list is the smaller one
+                        st.plan = TilePlan{};  // the row sweeps of a schedule with tall tiles need fewer
                         trg.clear();
                     }
                 }

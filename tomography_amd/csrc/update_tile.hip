@@ -26,7 +26,8 @@
 // the 128 VGPRs of four waves per SIMD without spilling: 16 rows of vacuum, 8
 // with one axis' CPML psi or with material coefficients, 4 with both (a corner
 // row in material costs 3 times a vacuum one).  Spilled prologues cost more than
-// shorter tiles (16 rows at the strips: 169 -> 270 us).
+// shorter tiles (16 rows at the strips: 169 -> 270 us).  Reference-compatible
+// mode, with its incident field and 64-bit kappa, spills 11 VGPRs all the same.
 #include "device.h"
 #include "fold.h"
 #include "kernels.h"
@@ -155,7 +156,9 @@ __device__ __forceinline__ void tile_wave(const RegTile& tile, const DevSim* __r
     const int je = (x >= 1 && x <= nc) ? x - 1 : ((x >= nx - nc && x <= nx - 1) ? nc + x - (nx - nc) : -1);
     const int jh = x < nc ? x : ((x >= nx - nc && x < nx) ? nc + x - (nx - nc) : -1);
     // psi rows of the y strips: E node rows 1..nc and ny-nc..ny-1, H rows 0..nc-1
-    // and ny-nc..ny-1 (a wave's rows never reach both strips: ny >= 2 nc + 4)
+    // and ny-nc..ny-1 (no wave reaches both: they are 4 rows apart, ny >= 2 nc + 4,
+    // and tiles of 8-row waves hold 64 rows from an end of the grid or clear of
+    // the strips, so that with nc <= 31 the gap falls between two waves)
     const bool hi = yb + R > ny - nc;
     auto row_e = [&](int y) { return (unsigned)(hi ? y - (ny - nc) : y - 1) < (unsigned)nc; };
     auto row_h = [&](int y) { return (unsigned)(hi ? y - (ny - nc) : y) < (unsigned)nc; };

@@ -35,7 +35,8 @@ SCHED_KEYS = ("tsteps", "seg_rows", "edge_waves", "inner_waves", "chunk", "grid_
 # Default schedules (fixed so that the profiled command and the timed one run
 # the same launches).  On grids of at least 64 x 32 nodes all three run register
 # tiles, of which they set the DFT chunk and the form; the sweep parameters
-# (swept on MI355X for the row sweeps) matter to smaller grids.  The plain one:
+# (swept on MI355X for the row sweeps) matter to smaller grids, and so does the
+# drop-in one's resident form.  The plain one:
 # fused; the batched one: four streams where simulations run by themselves.
 # Both fold the running DFT over 60-step chunks: the chunk sets the FP32 partial
 # sums, so equal chunks make batched and plain results equal bit for bit.  The
