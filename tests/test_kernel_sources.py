@@ -1,40 +1,67 @@
-"""Two facts that other tests restate in Python, held to the kernel sources
-themselves: the rule that picks a far-field projection, and the reference
-stage's division by a known kappa."""
+"""The rule that picks a far-field projection and the reference stage's division
+by a known kappa, compiled for the host from the kernel sources, so that the
+tests that rest on them cannot drift from them."""
 import ctypes
 import os
 import re
 import subprocess
 
 import numpy as np
+import pytest
 
 import test_projection_routes as routes
+import tomography_amd as t
+from cases import PHYS_PARAMS
+from tomography_amd.workloads import seeded_vectors
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "tomography_amd", "csrc")
 
 
-def test_projection_rule_is_the_dispatch_s_own():
-    """The restated rule against launch_project's expressions and constants."""
+def host_build(tmp_path, name, code):
+    src = tmp_path / (name + ".cpp")
+    src.write_text(code)
+    lib = tmp_path / (name + ".so")
+    subprocess.run(["g++", "-std=c++17", "-O2", "-ffp-contract=off", "-shared", "-fPIC", str(src), "-o", str(lib)], check=True)
+    return ctypes.CDLL(str(lib))
+
+
+def project_route(tmp_path):
+    """launch_project's own rule, compiled for the host: 0 the vector units, 1 the
+    matrix cores split, 2 the matrix cores."""
     text = open(os.path.join(CSRC, "kernels.hip")).read()
-    const = {k: int(v) for k, v in re.findall(r"\b(kChain\w+|kProj\w+) = (\d+)\b", text)}
-    const["kProjAngles"] = 32 * const["kProjAngleTiles"]
-    body = text[text.index("hipError_t launch_project("):]
-    rule = dict(re.findall(r"const int (chain|mfma) = ([^;]+);", body))
-    cond = re.search(r"if \((chain < [^{]+)\) \{", body).group(1)
+    const = "".join(re.findall(r"^constexpr int kProj.*;|^constexpr int kChainAngles.*;", text, re.M))
+    const = re.sub(r"//[^;]*?(?=constexpr|$)", "", const)
+    fn = re.search(r"^static int project_route\(.*?^}", text, re.M | re.S).group(0)
+    return host_build(tmp_path, "route", "#include <algorithm>\n%s\n%s\nextern \"C\" int route(int n, int a, int f) "
+                      "{ return project_route(n, a, f); }\n" % (const, fn)).route
 
-    def on_matrix_cores(n_sims, n_angles, n_freq):
-        env = dict(const, n_sims=n_sims, n_angles=n_angles, n_freq=n_freq)
-        for name in ("chain", "mfma"):
-            env[name] = eval(rule[name].replace("/", "//"), {}, env)
-        return not eval(cond.replace("/", "//"), {}, env)
 
-    picks = set()
-    for n in (1, 2, 8, 9, 31, 32, 33, 64, 65, 127, 128, 200, 256, 257, 1024, 4000):
-        for A in (1, 24, 100, 180, 360, 720, 723, 1921, 4096):
-            for F in (1, 3, 8, 16, 32):
-                assert on_matrix_cores(n, A, F) == routes.on_matrix_cores(n, A, F), (n, A, F)
-                picks.add(on_matrix_cores(n, A, F))
-    assert picks == {True, False}
+def test_projection_tests_run_both_kinds(tmp_path):
+    """The sizes of the projection tests lead to the kernels that they compare."""
+    route = project_route(tmp_path)
+    sizes = next(m.args[1] for m in routes.test_both_projections_agree.pytestmark if m.name == "parametrize")
+    for nx, ny, off, A, F, flags in sizes:
+        assert (route(1, A, F), route(9, A, F), route(65, A, F)) == (0, 0, 2)
+    assert [route(n, 4093, 8) for n in (1, 5, 9, 33)] == [0, 1, 1, 2]
+    assert route(1, 180, 8) == route(16, 360, 16) == 0 and route(1024, 360, 16) == 2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nx, ny, off, flags", [(71, 66, 9, 0), (75, 70, 8, t.FLAG_DFT_FP64)])
+def test_all_three_projections_agree(tmp_path, nx, ny, off, flags):
+    """One simulation on the vector units, 5 and 9 on the split matrix cores, 33
+    on the whole ones: the same far fields bit for bit."""
+    route = project_route(tmp_path)
+    cfg = routes.small(nx, ny, off, 4093, 8, flags)
+    V = seeded_vectors(33, 8, 5)
+    V[:, :3] = PHYS_PARAMS[:3]
+    T = np.zeros(cfg.farfield_len(), np.float32)
+    with t.Context() as c:
+        D = {n: c.eval_batch(cfg, V[:n], target=T, want_farfield=True)[1].reshape(n, -1) for n in (33, 9, 5, 1)}
+    assert [route(n, 4093, 8) for n in (33, 9, 5, 1)] == [2, 1, 1, 0]
+    assert np.abs(D[33]).max() > 0 and np.all(np.isfinite(D[33]))
+    for n in (9, 5, 1):
+        assert np.array_equal(D[n], D[33][:n]), n
 
 
 def test_division_by_a_known_divisor(tmp_path):
@@ -43,12 +70,8 @@ def test_division_by_a_known_divisor(tmp_path):
     text = open(os.path.join(CSRC, "update_tile.hip")).read()
     line = re.search(r"float div_known\(float a, double r\) \{[^}]*\}", text).group(0)
     use = re.search(r"p\.k = (1\.0 / \(double\)k\[i\]);", text).group(1)
-    src = tmp_path / "div.cpp"
-    src.write_text('static inline %s\nextern "C" void run(const float* a, const float* k, float* q, long n) {\n'
-                   '    for (long i = 0; i < n; ++i) q[i] = div_known(a[i], %s);\n}\n' % (line, use))
-    lib = tmp_path / "div.so"
-    subprocess.run(["g++", "-O2", "-ffp-contract=off", "-shared", "-fPIC", str(src), "-o", str(lib)], check=True)
-    run = ctypes.CDLL(str(lib)).run
+    run = host_build(tmp_path, "div", 'static inline %s\nextern "C" void run(const float* a, const float* k, float* q, long n) {\n'
+                     '    for (long i = 0; i < n; ++i) q[i] = div_known(a[i], %s);\n}\n' % (line, use)).run
     rng = np.random.default_rng(5)
     n = 2_000_000
     k = rng.uniform(1, 10, n).astype(np.float32)

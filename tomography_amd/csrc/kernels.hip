@@ -21,6 +21,7 @@
 // rows above and below: stage t is exact on lanes [t+1, 63-t) and the final
 // stage on [T, 64-T).  State is ping-ponged between two buffers per launch so
 // that overlapping ghost reads never see a neighbour's update.
+#include <algorithm>
 #include <type_traits>
 
 #include "device.h"
@@ -2077,6 +2078,10 @@ __global__ __launch_bounds__(256) void k_fold(const LaunchItem* __restrict__ ite
 // register r of lane l holds C[8(r/4) + 4(l/32) + r%4][l%32], so a lane ends
 // up holding all four rows of simulations 2q + l/32 (q = r/4) at angle l%32
 // and forms D and the phase without leaving its registers.
+// Split: the four waves share 8 simulations and take one 32-angle tile each,
+// so a workgroup's chain over the contour is a quarter as long.  Every output
+// element sees the same products in the same order in both layouts, so the
+// results are identical.
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kProjAngleTiles = 4;                 // 32-angle tiles per workgroup
 constexpr int kProjAngles = 32 * kProjAngleTiles;
@@ -2090,6 +2095,7 @@ __device__ __forceinline__ float2 far_field(float Nr, float Ni, float Lyr, float
     return make_float2(Lr + eta0 * Nr, Li + eta0 * Ni);
 }
 
+template <bool SPLIT>
 __global__ __launch_bounds__(64 * kProjWaves) void k_project_mfma(const int* __restrict__ sim_idx, int n_sims,
                                                                   const DevSim* __restrict__ sims,
                                                                   const float2* __restrict__ kinv, int A,
@@ -2098,8 +2104,9 @@ __global__ __launch_bounds__(64 * kProjWaves) void k_project_mfma(const int* __r
     __shared__ float2 wt[2][kProjChunk][kProjAngles];  // phase tiles {cos, sin}, double-buffered
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int a0 = blockIdx.x * kProjAngles, f = blockIdx.z;
-    constexpr int AT = kProjAngleTiles;                  // 32-angle tiles per wave
-    const int s0 = (blockIdx.y * kProjWaves + wv) * 8;   // this wave's first simulation
+    constexpr int AT = SPLIT ? 1 : kProjAngleTiles;      // 32-angle tiles per wave
+    const int s0 = SPLIT ? blockIdx.y * 8 : (blockIdx.y * kProjWaves + wv) * 8;  // this wave's first simulation
+    const int mt0 = SPLIT ? wv : 0;                      // this wave's first angle tile
     const DevSim* G = sims + sim_idx[0];                 // geometry shared by the group
     const int P = G->P, L1 = G->L1, L2 = G->L2, L3 = G->L3, F = G->nfreq;
     const bool fp64 = (G->flags & TOMO_FLAG_DFT_FP64) != 0;
@@ -2171,7 +2178,7 @@ __global__ __launch_bounds__(64 * kProjWaves) void k_project_mfma(const int* __r
         for (int j = 0; j < kProjChunk / 2; ++j) {
 #pragma unroll
             for (int m = 0; m < AT; ++m) {
-                const float2 w = wt[b][2 * j + kh][32 * m + (lane & 31)];
+                const float2 w = wt[b][2 * j + kh][32 * (mt0 + m) + (lane & 31)];
                 cre[m] = __builtin_amdgcn_mfma_f32_32x32x2f32(xr[j], w.x, cre[m], 0, 0, 0);
                 cre[m] = __builtin_amdgcn_mfma_f32_32x32x2f32(-xi[j], w.y, cre[m], 0, 0, 0);
                 cim[m] = __builtin_amdgcn_mfma_f32_32x32x2f32(xr[j], w.y, cim[m], 0, 0, 0);
@@ -2186,7 +2193,7 @@ __global__ __launch_bounds__(64 * kProjWaves) void k_project_mfma(const int* __r
     const float inv = ki.y;
 #pragma unroll
     for (int m = 0; m < AT; ++m) {
-        const int ab = a0 + 32 * m + (lane & 31);
+        const int ab = a0 + 32 * (mt0 + m) + (lane & 31);
         if (ab >= A) continue;
         float cph, sph;
         sincosf(6.283185307179586f * (float)ab / (float)A, &sph, &cph);
@@ -2613,21 +2620,43 @@ hipError_t launch_tres(int T, int rows_per_wave, int mode, const ResTile* tiles,
     return hipLaunchCooperativeKernel(f, dim3(ntiles), dim3(kResWaves * kWave), args, 0, st);
 }
 
+// Kernel of a projection: 0 the vector units, 1 the matrix cores split, 2 the
+// matrix cores with 8 simulations a wave.  All three times grow with the
+// contour, so the estimates are ns per contour point, from contours of 940 and
+// 4012 points (256^2, 1024^2): a vector workgroup costs the device 34 ps, 4 more
+// per simulation it holds and 3.5 more for each beyond the four SIMDs' first,
+// beside the chain's own 15 ns; a matrix-core
+// launch takes one chain while there is a workgroup per unit, and is bound by
+// the cores from four (split) or one (whole) on.  1024^2, us, vector / split:
+// 8 frequencies x 180 angles x 1 simulation 72 / 890, 32 x 720 x 8 1001 / 911,
+// 16 x 4096 x 1 1277 / 1192, 32 x 4096 x 8 4897 / 1942.  32 simulations fill the
+// waves of a whole workgroup; from there on the split is the faster one on some
+// contours only (32 x 720 x 64, 256^2 717 against 850, 96^2 239 against 204).
+static int project_route(int n_sims, int n_angles, int n_freq) {
+    auto per = [](int n, int d) { return (n + d - 1) / d; };
+    const int tiles = per(n_angles, kProjAngles) * n_freq, groups = per(n_sims, kChainSims);
+    const int second = n_sims / kChainSims * 4 + std::max(n_sims % kChainSims - 4, 0);
+    const double chain =
+        15 + 0.01 * per(n_angles, kChainAngles) * n_freq * (3.4 * groups + 0.4 * n_sims + 0.35 * second);
+    const int rs = per(tiles * groups, 256), rw = per(tiles * per(n_sims, 8 * kProjWaves), 256);
+    const double split = std::max(150.0 + 78 * rs, 118.0 * rs), whole = 415.0 * rw;
+    const bool halves = n_sims < 8 * kProjWaves && split < whole;
+    return chain < (halves ? split : whole) ? 0 : halves ? 1 : 2;
+}
+
 hipError_t launch_project(const int* sim_idx, int n_sims, int n_freq, const DevSim* sims, const float2* kinv,
                                int n_angles, float eta0, float* D, float* Pph, hipStream_t st) {
-    // Workgroups of either kernel.  Both times grow with the contour; on 512^2
-    // (8 frequencies of 180 angles) a round of up to 256 matrix-core
-    // workgroups takes 760 to 780 us and a vector workgroup 0.16 us of the
-    // device (128 simulations: 488 us against 778; 256: 923 against 783).
-    const int chain = (n_angles + kChainAngles - 1) / kChainAngles * n_freq * ((n_sims + kChainSims - 1) / kChainSims);
-    const int mfma = (n_angles + kProjAngles - 1) / kProjAngles * n_freq * ((n_sims + 8 * kProjWaves - 1) / (8 * kProjWaves));
-    if (chain < 5000 * ((mfma + 255) / 256)) {
-        dim3 g((n_angles + kChainAngles - 1) / kChainAngles, (n_sims + kChainSims - 1) / kChainSims, n_freq);
+    const int route = project_route(n_sims, n_angles, n_freq);
+    dim3 g((n_angles + kProjAngles - 1) / kProjAngles, (n_sims + 7) / 8, n_freq), b(64 * kProjWaves);
+    if (route == 0) {
+        g.x = (n_angles + kChainAngles - 1) / kChainAngles;
         TIMED_LAUNCH(k_project_chain, g, dim3(64 * kChainSims), 0, st, sim_idx, n_sims, sims, kinv, n_angles, eta0, D,
                      Pph);
+    } else if (route == 1) {
+        TIMED_LAUNCH(k_project_mfma<true>, g, b, 0, st, sim_idx, n_sims, sims, kinv, n_angles, eta0, D, Pph);
     } else {
-        dim3 g((n_angles + kProjAngles - 1) / kProjAngles, (n_sims + 8 * kProjWaves - 1) / (8 * kProjWaves), n_freq);
-        TIMED_LAUNCH(k_project_mfma, g, dim3(64 * kProjWaves), 0, st, sim_idx, n_sims, sims, kinv, n_angles, eta0, D, Pph);
+        g.y = (n_sims + 8 * kProjWaves - 1) / (8 * kProjWaves);
+        TIMED_LAUNCH(k_project_mfma<false>, g, b, 0, st, sim_idx, n_sims, sims, kinv, n_angles, eta0, D, Pph);
     }
     return hipGetLastError();
 }
